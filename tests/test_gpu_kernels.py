@@ -476,6 +476,21 @@ def test_attention_random_forests(seed):
             check_close(name, ref, got, TOL[dtype])
 
 
+@pytest.mark.parametrize("lens,par,n_past", [
+    ([1], [-1], 0), ([31], [-1], 0), ([33], [-1], 1), ([40, 24], [-1, 0], 31), ([63, 66], [-1, 0], 33),
+    ([97, 2, 30], [-1, 0, 0], 95), ([32, 32, 1], [-1, 0, 1], 64)])
+def test_attention_fp32_step_edges(lens, par, n_past):
+    """fp32 products as bf16 planes, in steps of 32 keys or queries: walks of
+    one step and of odd length, steps that straddle gateway and own keys,
+    ragged last rows, against the fp64 oracle at the fp32 bar."""
+    past_vis = [i % 5 != 2 for i in range(n_past)] if n_past else None
+    say(f"attention fp32 step edges lens={lens} n_past={n_past}")
+    res = _run(lens, par, torch.float32, seed=sum(lens) + n_past, past_vis=past_vis)
+    for name, (ref, got) in res.items():
+        if name != "lse":
+            check_close(name, ref, got, TOL[torch.float32])
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
 @pytest.mark.parametrize("shape", ["short", "split"])
 def test_attention_gateway(dtype, shape):
