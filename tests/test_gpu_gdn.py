@@ -194,6 +194,25 @@ def test_gdn_bwd_fp32_matches_autograd_oracle(case):
         assert _rel(a, b) < 1e-5, (case, name, _rel(a, b))
 
 
+@pytest.mark.parametrize("Hk,Hv", [(1, 2), (16, 32)], ids=["row_layout", "column_layout"])
+def test_gdn_scan_chunk_edges(Hk, Hv):
+    """Nodes of 1, 31, 32, 33, 64 and 65 tokens on one level (and a root of 33),
+    in the row layout of the level scans (12 pairs) and the column layout (192
+    pairs): fp32 outputs, states and gradients against the float64 oracle, at
+    the fp32 bar."""
+    lens, par = [33, 1, 31, 32, 33, 64, 65], [-1] + [0] * 6
+    T = sum(lens)
+    q, k, v, g, beta = _inputs(T, Hk, Hv, 41 + Hv, realistic_gates=True)
+    d_o = np.random.default_rng(12).standard_normal((T, Hv, D)).astype(np.float32)
+    print(f"gdn scan chunk edges: T={T} heads {Hk}/{Hv}", flush=True)
+    o, st = _run(q, k, v, g, beta, lens, par, torch.float32)
+    o_ref, st_ref = ogdn.gdn_tree(q, k, v, g, beta, lens, par, mode="exact")
+    assert _rel(o, o_ref) < 1e-5 and _rel(st, st_ref) < 1e-5
+    got = _run_bwd(q, k, v, g, beta, d_o, lens, par, torch.float32)
+    for name, a, b in zip(BWD_NAMES, got, _oracle_grads(q, k, v, g, beta, d_o, lens, par)):
+        assert _rel(a, b) < 1e-5, (name, _rel(a, b))
+
+
 @pytest.mark.parametrize("case", ["forest_multi_chunk", "c1_heads"])
 def test_gdn_bwd_bf16_matches_autograd_oracle(case):
     c = CASES[case]

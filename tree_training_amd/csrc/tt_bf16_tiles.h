@@ -59,8 +59,6 @@ constexpr int ROW_R = D + 8;
 template <int S>
 __device__ __forceinline__ int tile_off(int r, int d) { return r * S + d; }
 
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-
 // acc + v[i0] + v[i0+1] + v[i0+2] + v[i0+3] (fp32 accumulation, v_dot2c_f32_bf16).
 __device__ __forceinline__ float sum4_bf16(const bf16x8& v, int i0, float acc) {
     const bf16x2 one = {(bf16)1.0f, (bf16)1.0f};
@@ -72,28 +70,11 @@ __device__ __forceinline__ float sum4_bf16(const bf16x8& v, int i0, float acc) {
 // exceeds it by more than this many log2 units.
 #define TT_RESCALE_LOG2 8.0f
 
-template <int I>
-struct IntC {
-    static constexpr int value = I;
-};
-
 __device__ __forceinline__ bf16x8 zero8() {
     bf16x8 z;
 #pragma unroll
     for (int i = 0; i < 8; ++i) z[i] = (bf16)0.0f;
     return z;
-}
-
-typedef short v4i16 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
-typedef __attribute__((address_space(3))) void lds_void;
-typedef __attribute__((address_space(1))) const void glb_void;
-
-// ds_read_b64_tr_b16: within each 16-lane group, lane i receives element
-// (i & 3) of the 8-byte chunks read by lanes 4k + (i >> 2), k = 0..3.
-__device__ __forceinline__ bf16x4 ds_read_tr(const bf16* p) {
-    const v4i16 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(p));
-    return __builtin_bit_cast(bf16x4, r);
 }
 
 // MFMA operand "row = token, k = 16 head dims": X[r][d0 .. d0+7], d0 % 8 == 0.
@@ -188,19 +169,6 @@ __device__ __forceinline__ bf16x8 read_trg(const bf16* X, const TrOffsG& to, int
     const bf16* x = X + to.b[db] + (r0 >> 2) * GPITCH;
     return cat44(ds_read_tr(x), ds_read_tr(x + 2 * GPITCH));
 }
-
-template <int I>
-struct IntT {
-    static constexpr int value = I;
-};
-template <int N, int I = 0, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (I < N) {
-        f(IntT<I>{});
-        static_for<N, I + 1>(f);
-    }
-}
-
 
 // Direct global -> LDS staging (buffer_load ... lds): no staging registers and
 // no LDS store instructions. One wave instruction moves 64 x 16 bytes from

@@ -24,9 +24,10 @@
 //    independent per value column) and walks the node's chunks. Levels of
 //    one or two nodes use gdn_scan_rows_kernel instead (eight workgroups per
 //    pair, each wave a 32 x 16 slice), which gives the same bits.
-// fp32 end to end: the prep on fp32 MFMA (v_mfma_f32_32x32x2_f32) and the
-// vector ALUs, the scans on v_mfma_f32_16x16x4_f32.
+// fp32 accuracy end to end: the prep on fp32 MFMA (v_mfma_f32_32x32x2_f32) and
+// the vector ALUs, the scans (tt_gdn_scan.h) on bf16 planes of fp32 operands.
 #include "tt_gdn_common.h"
+#include "tt_gdn_scan.h"
 
 namespace {
 
@@ -215,485 +216,6 @@ __global__ __launch_bounds__(GT) void gdn_prep_kernel(GdnDev p, float* __restric
 }
 
 // ----------------------------------------------------------------------------
-// scan: per (node, v head), the node's chunks in order, on fp32 MFMA
-// ----------------------------------------------------------------------------
-
-struct ScanLds {
-    float W[GC * RS];     // W [token][state row]
-    float Q[GC * RS];     // q^ * scale
-    float K[GC * RS];     // k^ e^{G_L - G}
-    float A[GC * MS];
-    float G[GC];
-};
-
-// A chunk's scan inputs, held in registers one chunk ahead of their use (the
-// loads of the next chunk are in flight while a chunk computes): this
-// thread's share of the q and k rows (row t/8, dims 16 (t%8) .. +15, in the
-// problem dtype), of W's rows, four entries of A and the decays, and this
-// lane's 16 x 16 operand tiles of U (forward) or dO (reverse).
-template <typename TIn>
-struct ScanAhead {
-    using Vec = typename std::conditional<sizeof(TIn) == 2, bf16x8, f32x4>::type;
-    static constexpr int NV = 16 * (int)sizeof(TIn) / 16;   // vectors per 16 elements
-    Vec q[NV], k[NV];
-    f32x4 w[4];
-    float a[4];
-    float gi, gl, gt, gil, gll;   // G_i, G_L, G_t; low parts of G_i, G_L
-    f32x4 x[2];
-};
-
-// Loads the parts of chunk (start, len) that do not depend on the state: q/k
-// rows, W rows (with LOAD_W), A and the decays from its workspace slot cw.
-template <typename TIn, bool LOAD_W>
-__device__ __forceinline__ void scan_fetch_rows(const GdnDev& p, const float* cw, int start, int len, int h,
-                                                ScanAhead<TIn>& x) {
-    using Vec = typename ScanAhead<TIn>::Vec;
-    constexpr int NV = ScanAhead<TIn>::NV, EV = 16 / NV;
-    const int t = threadIdx.x, i = t >> 3, d0 = 16 * (t & 7), hk = h / p.rep;
-    if (i < len) {
-        const int64_t tok = start + i;
-        const TIn* qp = (const TIn*)p.q + tok * p.q_st + (int64_t)hk * p.q_sh + d0;
-        const TIn* kp = (const TIn*)p.k + tok * p.k_st + (int64_t)hk * p.k_sh + d0;
-#pragma unroll
-        for (int n = 0; n < NV; ++n) {
-            x.q[n] = *(const Vec*)(qp + EV * n);
-            x.k[n] = *(const Vec*)(kp + EV * n);
-        }
-    } else {
-#pragma unroll
-        for (int n = 0; n < NV; ++n) {
-#pragma unroll
-            for (int e = 0; e < EV; ++e) x.q[n][e] = x.k[n][e] = (TIn)0.0f;
-        }
-    }
-    if constexpr (LOAD_W) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) x.w[e] = *(const f32x4*)(cw + kWsW + i * GD + d0 + 4 * e);
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) x.a[e] = cw[kWsA + t + GT * e];
-    x.gi = cw[kWsG + i];
-    x.gl = cw[kWsG + GC - 1];
-    x.gt = cw[kWsG + (t & (GC - 1))];
-    x.gil = cw[kWsGlo + i];
-    x.gll = cw[kWsGlo + GC - 1];
-}
-
-// Writes a fetched chunk to LDS: Q = q^ * scale * qmul_i, K = k^ * kmul_i
-// (each rounded after the normalisation, then after the multiplier), W with
-// STORE_W, A and G. qmul / kmul: e^{G_i} / e^{G_L - G_i} where the scan needs
-// them (1 for none: the forward's Q).
-template <typename TIn, bool STORE_W, bool QMUL>
-__device__ __forceinline__ void scan_stage_rows(const GdnDev& p, const ScanAhead<TIn>& x, float* Q, float* K,
-                                                float* W, float* A, float* G) {
-    constexpr int NV = ScanAhead<TIn>::NV, EV = 16 / NV;
-    const int t = threadIdx.x, i = t >> 3, d0 = 16 * (t & 7);
-    float qv[16], kv[16];
-#pragma unroll
-    for (int n = 0; n < NV; ++n)
-#pragma unroll
-        for (int e = 0; e < EV; ++e) {
-            qv[EV * n + e] = (float)x.q[n][e];
-            kv[EV * n + e] = (float)x.k[n][e];
-        }
-    float sq = 0.0f, sk = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-        sq = fmaf(qv[e], qv[e], sq);
-        sk = fmaf(kv[e], kv[e], sk);
-    }
-    sq = row8_sum(sq);
-    sk = row8_sum(sk);
-    const float fq = (p.l2 ? 1.0f / sqrtf(sq + 1e-6f) : 1.0f) * p.scale;
-    const float fk = p.l2 ? 1.0f / sqrtf(sk + 1e-6f) : 1.0f;
-    const float eq = QMUL ? expf(x.gi) : 1.0f, ek = expf(gdiff(x.gl, x.gll, x.gi, x.gil));
-#pragma unroll
-    for (int e = 0; e < 16; e += 4) {
-        f32x4 qo, ko;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            qo[v] = qv[e + v] * fq;
-            ko[v] = kv[e + v] * fk;
-            if constexpr (QMUL) qo[v] *= eq;
-            ko[v] *= ek;
-        }
-        *(f32x4*)&Q[i * RS + d0 + e] = qo;
-        *(f32x4*)&K[i * RS + d0 + e] = ko;
-        if constexpr (STORE_W) *(f32x4*)&W[i * RS + d0 + e] = x.w[e / 4];
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int pi = t + GT * e;
-        A[(pi >> 5) * MS + (pi & 31)] = x.a[e];
-    }
-    if (t < GC) G[t] = x.gt;
-}
-
-// Column layout of the level scans. The value columns of the delta rule are
-// independent (column j of V', O and S depends only on column j of U, S and
-// V'); each wave owns 16 of them (16 x 16 fp32 MFMA tiles), and a (node,
-// v head) takes two workgroups of four waves (64 columns each) on different
-// CUs. A level with few nodes is a serial chain of chunks per node while most
-// CUs idle, and each chunk then runs on twice the MFMA pipes of one
-// workgroup. Workgroup x of a level launch takes a head and a column block;
-// with Hv a multiple of 8 the two blocks of a head are 8 apart (same XCD and
-// L2, dispatched together).
-constexpr int SCAN_COLS = 64;
-constexpr int kScanSplit = GD / SCAN_COLS;
-__device__ __forceinline__ void scan_block(const GdnDev& p, int& h, int& c0) {
-    const int bx = blockIdx.x;
-    int cs;
-    if ((p.hv & 7) == 0) {
-        h = ((bx >> 4) << 3) | (bx & 7);
-        cs = (bx >> 3) & 1;
-    } else {
-        h = bx >> 1;
-        cs = bx & 1;
-    }
-    c0 = SCAN_COLS * cs;
-}
-
-// Wave w owns value columns c0 + 16w .. +15 of one (node, v head): its
-// 128 x 16 state slice lives in eight 16 x 16 accumulator tiles (rows
-// 16 rb + 4 (l >> 4) + v) for the whole node. Per chunk (two 16-token tiles):
-//   V' = U - W S,  qS  (A = W / q^ rows from LDS, B = S from registers)
-//   O = e^G qS + A V'  (B = V' from registers)
-//   S <- e^{G_L} S + (k^ e^{G_L - G})^T V'  (A = k~ from LDS, B = V')
-// out may be null (the backward's recompute); chunk_sin / chunk_vp, when
-// given, receive each chunk's initial state and V' ([n_chunks, Hv, 128, 128]
-// and [n_chunks, Hv, 32, 128] floats).
-// TRUNC (the reference's per-node correction): V' = U - W S0 with S0 the
-// node's initial state for every chunk of the node. A first pass over the
-// node's chunks, while the state registers still hold S0, replaces each
-// chunk's U by its V' in the workspace; the scan proper then reads V' there.
-template <typename TIn, bool TRUNC>
-__global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn_scan_cols_kernel(GdnDev p, int lvl_begin, float* __restrict__ ws,
-                                                      TIn* __restrict__ out, float* __restrict__ states,
-                                                      float* __restrict__ chunk_sin, float* __restrict__ chunk_vp) {
-    __shared__ __attribute__((aligned(16))) ScanLds L;
-    const int node = p.level_nodes[lvl_begin + blockIdx.y];
-    if (node < 0 || node >= p.n_nodes) return;
-    int h, cb;
-    scan_block(p, h, cb);
-    const int t = threadIdx.x, wave = t >> 6, lane = t & 63, c16 = lane & 15, g4 = 4 * (lane >> 4);
-    const int j = cb + 16 * wave + c16;                                   // this lane's value column
-    const int jt = cb + 16 * wave;                                        // the wave's first column
-    const int start = p.node_start[node], len = p.node_len[node], chunk0 = p.node_chunk0[node];
-    int par = p.parent[node];
-    if (start < 0 || len < 0 || start > p.n_tokens - len) return;        // malformed node: skipped
-    if (chunk0 < 0 || chunk0 > p.n_chunks - tt_cdiv(len, GC)) return;
-    if (par >= node || par < -1) par = -1;                               // parents precede children
-
-    // S0: the parent's final state; a root's is the initial state (or zero).
-    const float* s0 = par >= 0 ? states + ((size_t)par * p.hv + h) * GD * GD
-                               : (p.init ? p.init + (size_t)h * GD * GD : nullptr);
-    f32x4 S[8];
-    if (s0) {
-#pragma unroll
-        for (int rb = 0; rb < 8; ++rb) S[rb] = load_t16(s0 + jt + 16 * rb * GD, lane);
-    } else {
-#pragma unroll
-        for (int rb = 0; rb < 8; ++rb) S[rb] = (f32x4){};
-    }
-
-    if constexpr (TRUNC) {
-        // V' = U - W S0 for every chunk (with S0 zero: V' = U as it is).
-        for (int c0 = 0; s0 && c0 < len; c0 += GC) {
-            float* cw = ws + ((size_t)(chunk0 + c0 / GC) * p.hv + h) * kWsChunk;
-            __syncthreads();   // readers of the previous chunk's W are done
-            {
-                const int i = t >> 3, d0 = 16 * (t & 7);
-#pragma unroll
-                for (int e = 0; e < 16; e += 4)
-                    *(f32x4*)&L.W[i * RS + d0 + e] = *(const f32x4*)(cw + kWsW + i * GD + d0 + e);
-            }
-            f32x4 vp[2];
-#pragma unroll
-            for (int tb = 0; tb < 2; ++tb) vp[tb] = load_t16(cw + kWsU + 16 * tb * GD + jt, lane);
-            __syncthreads();
-#pragma unroll
-            for (int rb = 0; rb < 8; ++rb)
-#pragma unroll
-                for (int tb = 0; tb < 2; ++tb) {
-                    const f32x4 wv = *(const f32x4*)&L.W[(16 * tb + c16) * RS + 16 * rb + g4];
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) vp[tb] = mfma16_f32(-wv[v], S[rb][v], vp[tb]);
-                }
-#pragma unroll
-            for (int tb = 0; tb < 2; ++tb) store_t16(cw + kWsU + 16 * tb * GD + jt, lane, vp[tb]);   // read back by this lane
-        }
-    }
-
-    // U (TRUNC: V', written by the first pass) and the state-independent
-    // chunk terms, one chunk ahead.
-    const int n_ch = tt_cdiv(len, GC);
-    ScanAhead<TIn> nx;
-    {
-        const float* cw = ws + ((size_t)chunk0 * p.hv + h) * kWsChunk;
-        scan_fetch_rows<TIn, !TRUNC>(p, cw, start, min(GC, len), h, nx);
-#pragma unroll
-        for (int tb = 0; tb < 2; ++tb) nx.x[tb] = load_t16(cw + kWsU + 16 * tb * GD + jt, lane);
-    }
-    for (int ci = 0; ci < n_ch; ++ci) {
-        const int c0 = GC * ci, Lc = min(GC, len - c0);
-        const size_t ch = (size_t)(chunk0 + ci) * p.hv + h;
-        if (chunk_sin) {
-            float* sp = chunk_sin + ch * GD * GD + jt;
-#pragma unroll
-            for (int rb = 0; rb < 8; ++rb) store_t16(sp + 16 * rb * GD, lane, S[rb]);
-        }
-        __syncthreads();   // readers of the previous chunk's tiles are done
-        scan_stage_rows<TIn, !TRUNC, false>(p, nx, L.Q, L.K, L.W, L.A, L.G);
-        f32x4 vp[2], qs[2];
-#pragma unroll
-        for (int tb = 0; tb < 2; ++tb) {
-            vp[tb] = nx.x[tb];
-            qs[tb] = (f32x4){};
-        }
-        if (ci + 1 < n_ch) {
-            const float* cw = ws + (ch + p.hv) * kWsChunk;
-            scan_fetch_rows<TIn, !TRUNC>(p, cw, start + c0 + GC, min(GC, len - c0 - GC), h, nx);
-#pragma unroll
-            for (int tb = 0; tb < 2; ++tb) nx.x[tb] = load_t16(cw + kWsU + 16 * tb * GD + jt, lane);
-        }
-        __syncthreads();
-
-        // V' = U - W S and q^ S over the 128 state rows as four partial sums of
-        // two row tiles each, added in order: the partition of the row layout's
-        // waves (gdn_scan_rows_kernel), so both layouts give the same bits.
-#pragma unroll
-        for (int w4 = 0; w4 < 4; ++w4) {
-            f32x4 pv[2] = {}, pq[2] = {};
-#pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                const int rb = 2 * w4 + r;
-#pragma unroll
-                for (int tb = 0; tb < 2; ++tb) {
-                    const int ro = (16 * tb + c16) * RS + 16 * rb + g4;
-                    const f32x4 qv = *(const f32x4*)&L.Q[ro];
-                    if constexpr (!TRUNC) {
-                        const f32x4 wv = *(const f32x4*)&L.W[ro];
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) pv[tb] = mfma16_f32(-wv[v], S[rb][v], pv[tb]);
-                    }
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) pq[tb] = mfma16_f32(qv[v], S[rb][v], pq[tb]);
-                    __builtin_amdgcn_sched_barrier(0);   // operand reads one step ahead at most (registers)
-                }
-            }
-#pragma unroll
-            for (int tb = 0; tb < 2; ++tb) {
-                if constexpr (!TRUNC) vp[tb] += pv[tb];
-                qs[tb] += pq[tb];
-            }
-        }
-        if (chunk_vp) {
-#pragma unroll
-            for (int tb = 0; tb < 2; ++tb) store_t16(chunk_vp + ch * GC * GD + 16 * tb * GD + jt, lane, vp[tb]);
-        }
-        // O = e^G (q^ S) + A V', token tile by token tile.
-#pragma unroll
-        for (int tb = 0; tb < 2; ++tb) {
-            f32x4 o;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) o[v] = qs[tb][v] * expf(L.G[16 * tb + g4 + v]);
-#pragma unroll
-            for (int tb2 = 0; tb2 < 2; ++tb2) {
-                const f32x4 av = *(const f32x4*)&L.A[(16 * tb + c16) * MS + 16 * tb2 + g4];
-#pragma unroll
-                for (int v = 0; v < 4; ++v) o = mfma16_f32(av[v], vp[tb2][v], o);
-            }
-            if (out) {
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int i = 16 * tb + g4 + v;
-                    if (i < Lc) out[((int64_t)(start + c0 + i) * p.hv + h) * GD + j] = (TIn)o[v];
-                }
-            }
-        }
-        // S <- e^{G_L} S + k~^T V': A[state row][token] = k~[token][state row].
-        {
-            const float el = expf(L.G[GC - 1]);
-#pragma unroll
-            for (int rb = 0; rb < 8; ++rb) {
-                S[rb] *= el;
-#pragma unroll
-                for (int tb = 0; tb < 2; ++tb) {
-#pragma unroll
-                    for (int v = 0; v < 4; ++v)
-                        S[rb] = mfma16_f32(L.K[(16 * tb + g4 + v) * RS + 16 * rb + c16], vp[tb][v], S[rb]);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
-        }
-    }
-
-    // Final state of the node (the initial state of its children).
-    float* sp = states + ((size_t)node * p.hv + h) * GD * GD + jt;
-#pragma unroll
-    for (int rb = 0; rb < 8; ++rb) store_t16(sp + 16 * rb * GD, lane, S[rb]);
-}
-
-// Row layout of the level scans, for levels of few nodes (the exact rule
-// only): a workgroup takes 16 value columns of one (node, v head), eight
-// workgroups per pair, and its wave w the state rows 32w .. 32w+31 of them.
-// The products over the state rows (W S and q^ S) are summed over the four
-// waves through LDS, in wave order; every wave then updates its own rows. A
-// chunk costs each wave about a quarter of the column layout's MFMAs, for
-// four times the workgroups: a level with few nodes runs a serial chain of
-// chunks on a mostly idle chip, and that chain gets shorter.
-constexpr int ROWS_COLS = 16;
-constexpr int kRowsSplit = GD / ROWS_COLS;
-__device__ __forceinline__ void rows_block(const GdnDev& p, int& h, int& c0) {
-    const int bx = blockIdx.x;
-    int cs;
-    if ((p.hv & 7) == 0) {   // the eight column blocks of a head on one XCD (same L2)
-        h = ((bx >> 6) << 3) | (bx & 7);
-        cs = (bx >> 3) & 7;
-    } else {
-        h = bx >> 3;
-        cs = bx & 7;
-    }
-    c0 = ROWS_COLS * cs;
-}
-
-struct ScanRowsLds {
-    ScanLds T;
-    f32x4 P[4][2][2][64];   // per wave: its partial W S and q^ S, both token tiles, lane-major
-};
-
-// As gdn_scan_cols_kernel (exact rule), in the row layout: wave w holds the
-// 32 x 16 slice S[32w .., c0 ..] in two 16 x 16 accumulator tiles.
-template <typename TIn>
-__global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn_scan_rows_kernel(GdnDev p, int lvl_begin, float* __restrict__ ws,
-                                                      TIn* __restrict__ out, float* __restrict__ states,
-                                                      float* __restrict__ chunk_sin, float* __restrict__ chunk_vp) {
-    __shared__ __attribute__((aligned(16))) ScanRowsLds L;
-    const int node = p.level_nodes[lvl_begin + blockIdx.y];
-    if (node < 0 || node >= p.n_nodes) return;
-    int h, cb;
-    rows_block(p, h, cb);
-    const int t = threadIdx.x, wave = t >> 6, lane = t & 63, c16 = lane & 15, g4 = 4 * (lane >> 4);
-    const int j = cb + c16;                                               // this lane's value column
-    const int rb0 = 2 * wave;                                             // the wave's first row tile
-    const int start = p.node_start[node], len = p.node_len[node], chunk0 = p.node_chunk0[node];
-    int par = p.parent[node];
-    if (start < 0 || len < 0 || start > p.n_tokens - len) return;        // malformed node: skipped
-    if (chunk0 < 0 || chunk0 > p.n_chunks - tt_cdiv(len, GC)) return;
-    if (par >= node || par < -1) par = -1;                               // parents precede children
-
-    const float* s0 = par >= 0 ? states + ((size_t)par * p.hv + h) * GD * GD
-                               : (p.init ? p.init + (size_t)h * GD * GD : nullptr);
-    f32x4 S[2];
-#pragma unroll
-    for (int r = 0; r < 2; ++r) S[r] = s0 ? load_t16(s0 + cb + 16 * (rb0 + r) * GD, lane) : (f32x4){};
-
-    const int n_ch = tt_cdiv(len, GC);
-    ScanAhead<TIn> nx;
-    {
-        const float* cw = ws + ((size_t)chunk0 * p.hv + h) * kWsChunk;
-        scan_fetch_rows<TIn, true>(p, cw, start, min(GC, len), h, nx);
-#pragma unroll
-        for (int tb = 0; tb < 2; ++tb) nx.x[tb] = load_t16(cw + kWsU + 16 * tb * GD + cb, lane);
-    }
-    for (int ci = 0; ci < n_ch; ++ci) {
-        const int c0 = GC * ci, Lc = min(GC, len - c0);
-        const size_t ch = (size_t)(chunk0 + ci) * p.hv + h;
-        if (chunk_sin) {
-            float* sp = chunk_sin + ch * GD * GD + cb;
-#pragma unroll
-            for (int r = 0; r < 2; ++r) store_t16(sp + 16 * (rb0 + r) * GD, lane, S[r]);
-        }
-        __syncthreads();   // readers of the previous chunk's tiles and partials are done
-        scan_stage_rows<TIn, true, false>(p, nx, L.T.Q, L.T.K, L.T.W, L.T.A, L.T.G);
-        f32x4 vp[2], qs[2], pv[2], pq[2];
-#pragma unroll
-        for (int tb = 0; tb < 2; ++tb) {
-            vp[tb] = nx.x[tb];
-            pv[tb] = pq[tb] = (f32x4){};
-        }
-        if (ci + 1 < n_ch) {
-            const float* cw = ws + (ch + p.hv) * kWsChunk;
-            scan_fetch_rows<TIn, true>(p, cw, start + c0 + GC, min(GC, len - c0 - GC), h, nx);
-#pragma unroll
-            for (int tb = 0; tb < 2; ++tb) nx.x[tb] = load_t16(cw + kWsU + 16 * tb * GD + cb, lane);
-        }
-        __syncthreads();
-
-        // this wave's rows of -W S and q^ S
-#pragma unroll
-        for (int r = 0; r < 2; ++r) {
-#pragma unroll
-            for (int tb = 0; tb < 2; ++tb) {
-                const int ro = (16 * tb + c16) * RS + 16 * (rb0 + r) + g4;
-                const f32x4 wv = *(const f32x4*)&L.T.W[ro];
-                const f32x4 qv = *(const f32x4*)&L.T.Q[ro];
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    pv[tb] = mfma16_f32(-wv[v], S[r][v], pv[tb]);
-                    pq[tb] = mfma16_f32(qv[v], S[r][v], pq[tb]);
-                }
-            }
-        }
-#pragma unroll
-        for (int tb = 0; tb < 2; ++tb) {
-            L.P[wave][0][tb][lane] = pv[tb];
-            L.P[wave][1][tb][lane] = pq[tb];
-        }
-        __syncthreads();
-        // V' = U - W S and q^ S, the partials summed in wave order
-#pragma unroll
-        for (int tb = 0; tb < 2; ++tb) {
-            qs[tb] = (f32x4){};
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-                vp[tb] += L.P[w][0][tb][lane];
-                qs[tb] += L.P[w][1][tb][lane];
-            }
-        }
-        if (chunk_vp && wave == 0) {
-#pragma unroll
-            for (int tb = 0; tb < 2; ++tb) store_t16(chunk_vp + ch * GC * GD + 16 * tb * GD + cb, lane, vp[tb]);
-        }
-        // O = e^G (q^ S) + A V': waves 0 and 1 take one token tile each
-        if (wave < 2) {
-            const int tb = wave;
-            f32x4 o;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) o[v] = qs[tb][v] * expf(L.T.G[16 * tb + g4 + v]);
-#pragma unroll
-            for (int tb2 = 0; tb2 < 2; ++tb2) {
-                const f32x4 av = *(const f32x4*)&L.T.A[(16 * tb + c16) * MS + 16 * tb2 + g4];
-#pragma unroll
-                for (int v = 0; v < 4; ++v) o = mfma16_f32(av[v], vp[tb2][v], o);
-            }
-            if (out) {
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int i = 16 * tb + g4 + v;
-                    if (i < Lc) out[((int64_t)(start + c0 + i) * p.hv + h) * GD + j] = (TIn)o[v];
-                }
-            }
-        }
-        // S <- e^{G_L} S + k~^T V' on this wave's rows
-        const float el = expf(L.T.G[GC - 1]);
-#pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            S[r] *= el;
-#pragma unroll
-            for (int tb = 0; tb < 2; ++tb)
-#pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    S[r] = mfma16_f32(L.T.K[(16 * tb + g4 + v) * RS + 16 * (rb0 + r) + c16], vp[tb][v], S[r]);
-        }
-    }
-
-    float* sp = states + ((size_t)node * p.hv + h) * GD * GD + cb;
-#pragma unroll
-    for (int r = 0; r < 2; ++r) store_t16(sp + 16 * (rb0 + r) * GD, lane, S[r]);
-}
-
-// ----------------------------------------------------------------------------
 // backward
 // ----------------------------------------------------------------------------
 // The backward recomputes the forward (prep + level scans, keeping each
@@ -713,296 +235,6 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 //    everything else: the chunk's 32 x 32 algebra (A, T = (I - N)^-1, N),
 //    dv, dbeta, dg (reverse cumulative sum of dG within the chunk), and
 //    dq, dk summed over the v heads of the group, then through the l2 norm.
-
-
-struct RscanLds {
-    float Q[GC * RS];     // e^G q^ * scale
-    float K[GC * RS];     // e^{G_L - G} k^
-    float W[GC * RS];
-    float A[GC * MS];
-    float G[GC];
-};
-
-// Column layout as gdn_scan_cols_kernel (scan_block). Wave w owns value
-// columns c0 + 16w .. +15: its 128 x 16 slice of dS lives in eight 16 x 16
-// accumulator tiles, dO of the chunk is loaded in accumulator layout (rows =
-// tokens, two 16-token tiles), and dV' is produced in it, so all three are
-// used straight from registers as MFMA B operands.
-// TRUNC (V' = U - W S0 with the node's initial state S0): the walk leaves out
-// the W term, and a second pass over the node's chunks subtracts
-// sum_c W_c^T dV'_c from the state gradient at the node's entry.
-template <typename TIn, bool TRUNC>
-__global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn_rscan_cols_kernel(
-        GdnDev p, int lvl_begin, const float* __restrict__ ws, const TIn* __restrict__ d_o, int64_t do_st,
-        int64_t do_sh, float* __restrict__ chunk_dso, float* __restrict__ chunk_dvp, float* __restrict__ node_dsin) {
-    __shared__ __attribute__((aligned(16))) RscanLds L;
-    const int node = p.level_nodes[lvl_begin + blockIdx.y];
-    if (node < 0 || node >= p.n_nodes) return;
-    int h, cb;
-    scan_block(p, h, cb);
-    const int t = threadIdx.x, wave = t >> 6, lane = t & 63, c16 = lane & 15, g4 = 4 * (lane >> 4);
-    const int j = cb + 16 * wave + c16;
-    const int jt = cb + 16 * wave;
-    const int start = p.node_start[node], len = p.node_len[node], chunk0 = p.node_chunk0[node];
-    if (start < 0 || len < 1 || start > p.n_tokens - len) return;        // malformed node: skipped
-    if (chunk0 < 0 || chunk0 > p.n_chunks - tt_cdiv(len, GC)) return;
-
-    // dS after the node: its state's incoming gradient, if any, plus the sum
-    // over its children of their dS at entry.
-    f32x4 dS[8];
-    if (p.d_states && (!p.d_states_last || node == p.n_nodes - 1)) {
-        const float* sp = p.d_states + ((size_t)(p.d_states_last ? 0 : node) * p.hv + h) * GD * GD + jt;
-#pragma unroll
-        for (int rb = 0; rb < 8; ++rb) dS[rb] = load_t16(sp + 16 * rb * GD, lane);
-    } else {
-#pragma unroll
-        for (int rb = 0; rb < 8; ++rb) dS[rb] = (f32x4){};
-    }
-    {
-        const int c_lo = max(p.child_off[node], 0), c_hi = min(p.child_off[node + 1], p.n_nodes);
-        for (int ci = c_lo; ci < c_hi; ++ci) {
-            const int child = p.child[ci];
-            if (child <= node || child >= p.n_nodes) continue;          // children follow their parent
-            const float* sp = node_dsin + ((size_t)child * p.hv + h) * GD * GD + jt;
-#pragma unroll
-            for (int rb = 0; rb < 8; ++rb) dS[rb] += load_t16(sp + 16 * rb * GD, lane);
-        }
-    }
-
-    // The chunk terms and dO rows of a chunk, one chunk ahead (the walk runs
-    // backwards).
-    const int n_ch = tt_cdiv(len, GC);
-    auto fetch = [&](int ci, ScanAhead<TIn>& x) {
-        const int c0 = GC * ci, Lc = min(GC, len - c0);
-        const float* cw = ws + ((size_t)(chunk0 + ci) * p.hv + h) * kWsChunk;
-        scan_fetch_rows<TIn, !TRUNC>(p, cw, start + c0, Lc, h, x);
-        const TIn* base = d_o + (int64_t)(start + c0) * do_st + (int64_t)h * do_sh + j;
-#pragma unroll
-        for (int tb = 0; tb < 2; ++tb)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {   // dO[token 16 tb + 4 (l >> 4) + v][j], zero past the chunk
-                const int i = 16 * tb + g4 + v;
-                x.x[tb][v] = i < Lc ? (float)base[(int64_t)i * do_st] : 0.0f;
-            }
-    };
-    ScanAhead<TIn> nx;
-    fetch(n_ch - 1, nx);
-    for (int ci = n_ch - 1; ci >= 0; --ci) {
-        const int c0 = GC * ci, Lc = min(GC, len - c0);
-        const size_t chn = (size_t)(chunk0 + ci) * p.hv + h;
-        {   // the gradient of this chunk's output state
-            float* sp = chunk_dso + chn * GD * GD + jt;
-#pragma unroll
-            for (int rb = 0; rb < 8; ++rb) store_t16(sp + 16 * rb * GD, lane, dS[rb]);
-        }
-        __syncthreads();   // readers of the previous chunk's tiles are done
-        scan_stage_rows<TIn, !TRUNC, true>(p, nx, L.Q, L.K, L.W, L.A, L.G);
-        const f32x4 dov[2] = {nx.x[0], nx.x[1]};
-        if (ci > 0) fetch(ci - 1, nx);
-        __syncthreads();
-
-        // dV' = A^T dO + k~ dS as four partial sums added in order, partial w4
-        // holding the A^T dO term of token tiles (w4 / 2, w4 % 2) and the
-        // state rows 32 w4 .. +31: the partition of the row layout's waves
-        // (gdn_rscan_rows_kernel), so both layouts give the same bits.
-        f32x4 dv[2];
-#pragma unroll
-        for (int tb = 0; tb < 2; ++tb) {
-            dv[tb] = (f32x4){};
-#pragma unroll
-            for (int w4 = 0; w4 < 4; ++w4) {
-                f32x4 pd = {};
-                if (tb == (w4 >> 1)) {
-#pragma unroll
-                    for (int v = 0; v < 4; ++v)
-                        pd = mfma16_f32(L.A[(16 * (w4 & 1) + g4 + v) * MS + 16 * tb + c16], dov[w4 & 1][v], pd);
-                }
-#pragma unroll
-                for (int r = 0; r < 2; ++r) {
-                    const int rb = 2 * w4 + r;
-                    const f32x4 kv = *(const f32x4*)&L.K[(16 * tb + c16) * RS + 16 * rb + g4];
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) pd = mfma16_f32(kv[v], dS[rb][v], pd);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                dv[tb] += pd;
-            }
-        }
-#pragma unroll
-        for (int tb = 0; tb < 2; ++tb) store_t16(chunk_dvp + chn * GC * GD + 16 * tb * GD + jt, lane, dv[tb]);
-
-        // dS <- e^{G_L} dS + (e^G q^)^T dO - W^T dV'
-        const float el = expf(L.G[GC - 1]);
-#pragma unroll
-        for (int rb = 0; rb < 8; ++rb) {
-            dS[rb] *= el;
-#pragma unroll
-            for (int tb = 0; tb < 2; ++tb) {
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int ro = (16 * tb + g4 + v) * RS + 16 * rb + c16;
-                    dS[rb] = mfma16_f32(L.Q[ro], dov[tb][v], dS[rb]);
-                    if constexpr (!TRUNC) dS[rb] = mfma16_f32(-L.W[ro], dv[tb][v], dS[rb]);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-    }
-    if constexpr (TRUNC) {
-        for (int ci = 0; ci < tt_cdiv(len, GC); ++ci) {
-            const size_t chn = (size_t)(chunk0 + ci) * p.hv + h;
-            const float* cw = ws + chn * kWsChunk;
-            __syncthreads();   // readers of the previous chunk's W are done
-            {
-                const int i = t >> 3, d0 = 16 * (t & 7);
-#pragma unroll
-                for (int e = 0; e < 16; e += 4)
-                    *(f32x4*)&L.W[i * RS + d0 + e] = *(const f32x4*)(cw + kWsW + i * GD + d0 + e);
-            }
-            f32x4 dv[2];   // this lane's own writes
-#pragma unroll
-            for (int tb = 0; tb < 2; ++tb) dv[tb] = load_t16(chunk_dvp + chn * GC * GD + 16 * tb * GD + jt, lane);
-            __syncthreads();
-#pragma unroll
-            for (int rb = 0; rb < 8; ++rb)
-#pragma unroll
-                for (int tb = 0; tb < 2; ++tb)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v)
-                        dS[rb] = mfma16_f32(-L.W[(16 * tb + g4 + v) * RS + 16 * rb + c16], dv[tb][v], dS[rb]);
-        }
-    }
-    // dS at the node's entry, summed into its parent by the next (shallower) level.
-    float* sp = node_dsin + ((size_t)node * p.hv + h) * GD * GD + jt;
-#pragma unroll
-    for (int rb = 0; rb < 8; ++rb) store_t16(sp + 16 * rb * GD, lane, dS[rb]);
-}
-
-struct RscanRowsLds {
-    RscanLds T;
-    f32x4 P[4][2][64];   // per wave: its partial dV', both token tiles, lane-major
-};
-
-// As gdn_rscan_cols_kernel (exact rule), in the row layout of
-// gdn_scan_rows_kernel: wave w holds dS[32w .., c0 ..]. dV' = A^T dO + k~ dS
-// is summed over the waves' rows through LDS, in wave order (wave w also adds
-// the A^T dO term of token tiles (w / 2, w % 2)); every wave then updates its
-// rows of dS.
-template <typename TIn>
-__global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn_rscan_rows_kernel(
-        GdnDev p, int lvl_begin, const float* __restrict__ ws, const TIn* __restrict__ d_o, int64_t do_st,
-        int64_t do_sh, float* __restrict__ chunk_dso, float* __restrict__ chunk_dvp, float* __restrict__ node_dsin) {
-    __shared__ __attribute__((aligned(16))) RscanRowsLds L;
-    const int node = p.level_nodes[lvl_begin + blockIdx.y];
-    if (node < 0 || node >= p.n_nodes) return;
-    int h, cb;
-    rows_block(p, h, cb);
-    const int t = threadIdx.x, wave = t >> 6, lane = t & 63, c16 = lane & 15, g4 = 4 * (lane >> 4);
-    const int j = cb + c16;
-    const int rb0 = 2 * wave;
-    const int start = p.node_start[node], len = p.node_len[node], chunk0 = p.node_chunk0[node];
-    if (start < 0 || len < 1 || start > p.n_tokens - len) return;        // malformed node: skipped
-    if (chunk0 < 0 || chunk0 > p.n_chunks - tt_cdiv(len, GC)) return;
-
-    f32x4 dS[2];
-    if (p.d_states && (!p.d_states_last || node == p.n_nodes - 1)) {
-        const float* sp = p.d_states + ((size_t)(p.d_states_last ? 0 : node) * p.hv + h) * GD * GD + cb;
-#pragma unroll
-        for (int r = 0; r < 2; ++r) dS[r] = load_t16(sp + 16 * (rb0 + r) * GD, lane);
-    } else {
-#pragma unroll
-        for (int r = 0; r < 2; ++r) dS[r] = (f32x4){};
-    }
-    {
-        const int c_lo = max(p.child_off[node], 0), c_hi = min(p.child_off[node + 1], p.n_nodes);
-        for (int ci = c_lo; ci < c_hi; ++ci) {
-            const int child = p.child[ci];
-            if (child <= node || child >= p.n_nodes) continue;          // children follow their parent
-            const float* sp = node_dsin + ((size_t)child * p.hv + h) * GD * GD + cb;
-#pragma unroll
-            for (int r = 0; r < 2; ++r) dS[r] += load_t16(sp + 16 * (rb0 + r) * GD, lane);
-        }
-    }
-
-    const int n_ch = tt_cdiv(len, GC);
-    auto fetch = [&](int ci, ScanAhead<TIn>& x) {
-        const int c0 = GC * ci, Lc = min(GC, len - c0);
-        const float* cw = ws + ((size_t)(chunk0 + ci) * p.hv + h) * kWsChunk;
-        scan_fetch_rows<TIn, true>(p, cw, start + c0, Lc, h, x);
-        const TIn* base = d_o + (int64_t)(start + c0) * do_st + (int64_t)h * do_sh + j;
-#pragma unroll
-        for (int tb = 0; tb < 2; ++tb)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {   // dO[token 16 tb + 4 (l >> 4) + v][j], zero past the chunk
-                const int i = 16 * tb + g4 + v;
-                x.x[tb][v] = i < Lc ? (float)base[(int64_t)i * do_st] : 0.0f;
-            }
-    };
-    ScanAhead<TIn> nx;
-    fetch(n_ch - 1, nx);
-    const int atb = wave >> 1, atb2 = wave & 1;   // this wave's A^T dO term
-    for (int ci = n_ch - 1; ci >= 0; --ci) {
-        const size_t chn = (size_t)(chunk0 + ci) * p.hv + h;
-        {
-            float* sp = chunk_dso + chn * GD * GD + cb;
-#pragma unroll
-            for (int r = 0; r < 2; ++r) store_t16(sp + 16 * (rb0 + r) * GD, lane, dS[r]);
-        }
-        __syncthreads();   // readers of the previous chunk's tiles and partials are done
-        scan_stage_rows<TIn, true, true>(p, nx, L.T.Q, L.T.K, L.T.W, L.T.A, L.T.G);
-        const f32x4 dov[2] = {nx.x[0], nx.x[1]};
-        if (ci > 0) fetch(ci - 1, nx);
-        __syncthreads();
-
-        f32x4 pd[2];
-#pragma unroll
-        for (int tb = 0; tb < 2; ++tb) {
-            pd[tb] = (f32x4){};
-            if (tb == atb) {
-#pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    pd[tb] = mfma16_f32(L.T.A[(16 * atb2 + g4 + v) * MS + 16 * tb + c16], dov[atb2][v], pd[tb]);
-            }
-#pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                const f32x4 kv = *(const f32x4*)&L.T.K[(16 * tb + c16) * RS + 16 * (rb0 + r) + g4];
-#pragma unroll
-                for (int v = 0; v < 4; ++v) pd[tb] = mfma16_f32(kv[v], dS[r][v], pd[tb]);
-            }
-            L.P[wave][tb][lane] = pd[tb];
-        }
-        __syncthreads();
-        f32x4 dv[2];
-#pragma unroll
-        for (int tb = 0; tb < 2; ++tb) {
-            dv[tb] = (f32x4){};
-#pragma unroll
-            for (int w = 0; w < 4; ++w) dv[tb] += L.P[w][tb][lane];
-        }
-        if (wave == 0) {
-#pragma unroll
-            for (int tb = 0; tb < 2; ++tb) store_t16(chunk_dvp + chn * GC * GD + 16 * tb * GD + cb, lane, dv[tb]);
-        }
-
-        // dS <- e^{G_L} dS + (e^G q^)^T dO - W^T dV' on this wave's rows
-        const float el = expf(L.T.G[GC - 1]);
-#pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            dS[r] *= el;
-#pragma unroll
-            for (int tb = 0; tb < 2; ++tb)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int ro = (16 * tb + g4 + v) * RS + 16 * (rb0 + r) + c16;
-                    dS[r] = mfma16_f32(L.T.Q[ro], dov[tb][v], dS[r]);
-                    dS[r] = mfma16_f32(-L.T.W[ro], dv[tb][v], dS[r]);
-                }
-        }
-    }
-    float* sp = node_dsin + ((size_t)node * p.hv + h) * GD * GD + cb;
-#pragma unroll
-    for (int r = 0; r < 2; ++r) store_t16(sp + 16 * (rb0 + r) * GD, lane, dS[r]);
-}
 
 // Gradient of the initial state: the sum over the roots, in node order (the
 // order in which a node's children's terms are summed), of their state

@@ -1,0 +1,762 @@
+// Level scans of the tree gated delta rule: the forward scan of the states and
+// the reverse scan of their gradients, per (node, v head), one launch per tree
+// level (tt_gdn.hip has the equations).
+//
+// The products run on the bf16 matrix cores (v_mfma_f32_16x16x32_bf16) on
+// operands split into bf16 planes (tt_planes.h): W, A, V', dV' and the states
+// into three, q, k and dO as they come (one plane for bf16 problems, exact;
+// three for fp32), with the l2 norms and decays as per-token factors on the
+// other operand or on the result. A 16-column slice of a chunk takes a wave
+// 108 MFMAs of 16 cycles forward and 102 reverse (bf16 problems) where
+// v_mfma_f32_16x16x4_f32 took 208 and 200 of 32. On the 16K agent tree (32 v
+// heads, bf16) the column-layout levels went 867 -> 600 us forward and 1098 ->
+// 830 reverse, the row-layout ones 164 -> 140 and 256 -> 228. What bounds them
+// now is what they move: the states and their gradients (2.2 GB written), W,
+// U, V' and dV'.
+#pragma once
+
+#include "tt_gdn_common.h"
+#include "tt_planes.h"
+
+namespace {
+
+// bf16 planes of a chunk's tiles in LDS, rows = tokens. A tile read by rows
+// (16 rows x 16 bytes a pass) has rows of 272 bytes (A: 80), one read by
+// columns through the transposing read (8 rows x 32 bytes) rows of 288 (96):
+// both reach every bank once a pass.
+constexpr int PR = GD + 8, PC = GD + 16;   // [token][state row] tiles
+constexpr int AR = GC + 8, AC = GC + 16;   // [token][token]
+template <typename TIn>
+constexpr int kInPlanes = sizeof(TIn) == 2 ? 1 : 3;
+
+__device__ __forceinline__ f32x4 mfma16b(const bf16x8& a, const bf16x8& b, const f32x4& c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+// An operand of N planes (h, m, l).
+template <int N>
+struct Op {
+    bf16x8 p[N];
+};
+// acc + A B, the smallest terms first.
+template <int NA, int NB>
+__device__ __forceinline__ f32x4 mul_planes(const Op<NA>& a, const Op<NB>& b, f32x4 acc) {
+    if constexpr (NA == 3) acc = mfma16b(a.p[2], b.p[0], acc);
+    if constexpr (NB == 3) acc = mfma16b(a.p[0], b.p[2], acc);
+    if constexpr (NA == 3 && NB == 3) acc = mfma16b(a.p[1], b.p[1], acc);
+    if constexpr (NA == 3) acc = mfma16b(a.p[1], b.p[0], acc);
+    if constexpr (NB == 3) acc = mfma16b(a.p[0], b.p[1], acc);
+    return mfma16b(a.p[0], b.p[0], acc);
+}
+// Two 16-row accumulator tiles (rows 4 (l >> 4) + v) as the operand of a
+// 32-deep contraction: element e of lane l is row 4 (l >> 4) + (e & 3) of tile
+// e / 4, the k order of every operand here.
+__device__ __forceinline__ Op<3> op_acc(const f32x4& t0, const f32x4& t1) {
+    Split8 w = split_begin(t0, t1);
+    w.all();
+    const Planes q = w.planes();
+    return {{q.h, q.m, q.l}};
+}
+// Row operand X[row][k0 + k] of a tile with rows of P elements (N planes, each
+// [GC][P]), g4 = 4 (l >> 4).
+template <int N, int P>
+__device__ __forceinline__ Op<N> op_rows(const __bf16* X, int row, int k0, int g4) {
+    Op<N> o;
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+        const __bf16* x = X + n * GC * P + row * P + k0 + g4;
+        o.p[n] = cat44(*(const bf16x4*)x, *(const bf16x4*)(x + 16));
+    }
+    return o;
+}
+// Column operand X[k][c0 + (l & 15)], k over the tile's 32 tokens.
+template <int N, int P>
+__device__ __forceinline__ Op<N> op_cols(const __bf16* X, int c0, int lane) {
+    const int j = lane & 15;
+    Op<N> o;
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+        const __bf16* x = X + n * GC * P + (4 * (lane >> 4) + (j >> 2)) * P + c0 + 4 * (j & 3);
+        o.p[n] = cat44(ds_read_tr(x), ds_read_tr(x + 16 * P));
+    }
+    return o;
+}
+
+// A chunk's scan inputs, held in registers one chunk ahead of their use (the
+// loads of the next chunk are in flight while a chunk computes): this
+// thread's share of the q and k rows (row t/8, dims 16 (t%8) .. +15, in the
+// problem dtype) and of W's rows, four entries of A (row t/8, columns
+// 4 (t%8) ..) and the decays, and this lane's 16 x 16 tiles of U (forward) or
+// dO (reverse).
+template <typename TIn>
+struct ScanAhead {
+    using Vec = typename std::conditional<sizeof(TIn) == 2, bf16x8, f32x4>::type;
+    static constexpr int NV = 16 * (int)sizeof(TIn) / 16;   // vectors per 16 elements
+    Vec q[NV], k[NV];
+    f32x4 w[4];
+    f32x4 a;
+    float gi, gl, gil, gll;   // G_i, G_L; their low parts
+    f32x4 x[2];
+};
+
+// Loads the parts of chunk (start, len) that do not depend on the state: q/k
+// rows, W rows (with LOAD_W), A and the decays from its workspace slot cw.
+template <typename TIn, bool LOAD_W>
+__device__ __forceinline__ void scan_fetch_rows(const GdnDev& p, const float* cw, int start, int len, int h,
+                                                ScanAhead<TIn>& x) {
+    using Vec = typename ScanAhead<TIn>::Vec;
+    constexpr int NV = ScanAhead<TIn>::NV, EV = 16 / NV;
+    const int t = threadIdx.x, i = t >> 3, d0 = 16 * (t & 7), hk = h / p.rep;
+    if (i < len) {
+        const int64_t tok = start + i;
+        const TIn* qp = (const TIn*)p.q + tok * p.q_st + (int64_t)hk * p.q_sh + d0;
+        const TIn* kp = (const TIn*)p.k + tok * p.k_st + (int64_t)hk * p.k_sh + d0;
+#pragma unroll
+        for (int n = 0; n < NV; ++n) {
+            x.q[n] = *(const Vec*)(qp + EV * n);
+            x.k[n] = *(const Vec*)(kp + EV * n);
+        }
+    } else {
+#pragma unroll
+        for (int n = 0; n < NV; ++n) {
+#pragma unroll
+            for (int e = 0; e < EV; ++e) x.q[n][e] = x.k[n][e] = (TIn)0.0f;
+        }
+    }
+    if constexpr (LOAD_W) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x.w[e] = *(const f32x4*)(cw + kWsW + i * GD + d0 + 4 * e);
+    }
+    x.a = *(const f32x4*)(cw + kWsA + i * GC + 4 * (t & 7));
+    x.gi = cw[kWsG + i];
+    x.gl = cw[kWsG + GC - 1];
+    x.gil = cw[kWsGlo + i];
+    x.gll = cw[kWsGlo + GC - 1];
+}
+
+// 16 consecutive elements of row i at column d0 as planes of a tile with rows of P elements.
+template <int P>
+__device__ __forceinline__ void put16(__bf16* X, int i, int d0, const bf16x8 (&x)[2]) {
+    *(bf16x8*)(X + i * P + d0) = x[0];
+    *(bf16x8*)(X + i * P + d0 + 8) = x[1];
+}
+template <int P>
+__device__ __forceinline__ void put16(__bf16* X, int i, int d0, const f32x4 (&x)[4]) {
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+        Split8 w = split_begin(x[2 * n], x[2 * n + 1]);
+        w.all();
+        const Planes q = w.planes();
+        __bf16* d = X + i * P + d0 + 8 * n;
+        *(bf16x8*)d = q.h;
+        *(bf16x8*)(d + GC * P) = q.m;
+        *(bf16x8*)(d + 2 * GC * P) = q.l;
+    }
+}
+// 1 / sqrt(|row|^2 + eps) (1 without the l2 norm) of the row whose 128
+// elements this thread and its seven neighbours hold.
+template <int NV, typename Vec>
+__device__ __forceinline__ float row_norm(const GdnDev& p, const Vec (&x)[NV]) {
+    constexpr int EV = 16 / NV;
+    float s = 0.0f;
+#pragma unroll
+    for (int n = 0; n < NV; ++n)
+#pragma unroll
+        for (int e = 0; e < EV; ++e) s = fmaf((float)x[n][e], (float)x[n][e], s);
+    s = row8_sum(s);
+    return p.l2 ? 1.0f / sqrtf(s + 1e-6f) : 1.0f;
+}
+
+// A fetched chunk in LDS: q, k, W (with STORE_W) and A as planes with rows of
+// PQ, PK, PW and PA elements, and the per-token factors fq = scale e^{G_i} /
+// |q_i| and fk = e^{G_L - G_i} / |k_i|.
+template <typename TIn, int PQ, int PK, int PW, int PA>
+struct ScanTiles {
+    static constexpr int NQ = kInPlanes<TIn>;
+    __bf16 Q[NQ * GC * PQ];
+    __bf16 K[NQ * GC * PK];
+    __bf16 W[3 * GC * PW];
+    __bf16 A[3 * GC * PA];
+    float fq[GC], fk[GC];
+    float el;   // e^{G_L}
+    template <bool STORE_W>
+    __device__ __forceinline__ void stage(const GdnDev& p, const ScanAhead<TIn>& x) {
+        const int t = threadIdx.x, i = t >> 3, d0 = 16 * (t & 7);
+        put16<PQ>(Q, i, d0, x.q);
+        put16<PK>(K, i, d0, x.k);
+        if constexpr (STORE_W) put16<PW>(W, i, d0, x.w);
+        {
+            float a0 = x.a[0], a1 = x.a[1], a2 = x.a[2], a3 = x.a[3];
+            __bf16* d = A + i * PA + 4 * (t & 7);
+#pragma unroll
+            for (int n = 0; n < 3; ++n) {
+                const uint32_t u0 = pack_bf16(a0, a1), u1 = pack_bf16(a2, a3);
+                *(u32x2*)(d + n * GC * PA) = (u32x2){u0, u1};
+                sub_bf16(u0, a0, a1);
+                sub_bf16(u1, a2, a3);
+            }
+        }
+        const float nq = row_norm(p, x.q), nk = row_norm(p, x.k);
+        if ((t & 7) == 0) {
+            fq[i] = nq * p.scale * expf(x.gi);
+            fk[i] = nk * expf(gdiff(x.gl, x.gll, x.gi, x.gil));
+            if (t == 0) el = expf(x.gl);
+        }
+    }
+};
+template <typename TIn>
+using FwdTiles = ScanTiles<TIn, PR, PC, PR, AR>;   // q, W and A by rows, k by columns
+template <typename TIn>
+using RevTiles = ScanTiles<TIn, PC, PR, PC, AC>;   // k by rows, q, W and A by columns
+
+// S e + x: the products of an update are summed apart and join the state with
+// one rounding.
+__device__ __forceinline__ f32x4 fma_tile(const f32x4& S, float e, const f32x4& x) {
+    f32x4 r;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) r[v] = fmaf(S[v], e, x[v]);
+    return r;
+}
+// x times the factors of tokens tok0 .. tok0 + 3, rounded (never fused into a
+// sum: both layouts must round alike).
+__device__ __forceinline__ f32x4 scale_tok(const f32x4& x, const float* f, int tok0) {
+#pragma clang fp contract(off)
+    const f32x4 s = *(const f32x4*)(f + tok0);
+    return x * s;
+}
+// O of the same tokens: fq (q S) + A V'.
+__device__ __forceinline__ f32x4 out_tok(const f32x4& qs, const float* fq, int tok0, const f32x4& av) {
+    const f32x4 s = *(const f32x4*)(fq + tok0);
+    f32x4 o;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) o[v] = fmaf(qs[v], s[v], av[v]);
+    return o;
+}
+
+// Column layout of the level scans. The value columns of the delta rule are
+// independent (column j of V', O and S depends only on column j of U, S and
+// V'); each wave owns 16 of them (16 x 16 fp32 MFMA tiles), and a (node,
+// v head) takes two workgroups of four waves (64 columns each) on different
+// CUs. A level with few nodes is a serial chain of chunks per node while most
+// CUs idle, and each chunk then runs on twice the MFMA pipes of one
+// workgroup. Workgroup x of a level launch takes a head and a column block;
+// with Hv a multiple of 8 the two blocks of a head are 8 apart (same XCD and
+// L2, dispatched together).
+constexpr int SCAN_COLS = 64;
+constexpr int kScanSplit = GD / SCAN_COLS;
+__device__ __forceinline__ void scan_block(const GdnDev& p, int& h, int& c0) {
+    const int bx = blockIdx.x;
+    int cs;
+    if ((p.hv & 7) == 0) {
+        h = ((bx >> 4) << 3) | (bx & 7);
+        cs = (bx >> 3) & 1;
+    } else {
+        h = bx >> 1;
+        cs = bx & 1;
+    }
+    c0 = SCAN_COLS * cs;
+}
+
+// Start of a node's forward scan: its parent's final state (a root's: the
+// initial state, or none).
+struct ScanNode {
+    int node, start, len, chunk0, n_ch;
+    const float* s0;
+    __device__ __forceinline__ bool init(const GdnDev& p, int lvl_begin) {
+        node = p.level_nodes[lvl_begin + blockIdx.y];
+        if (node < 0 || node >= p.n_nodes) return false;
+        start = p.node_start[node];
+        len = p.node_len[node];
+        chunk0 = p.node_chunk0[node];
+        if (start < 0 || len < 0 || start > p.n_tokens - len) return false;        // malformed node: skipped
+        n_ch = tt_cdiv(len, GC);
+        return chunk0 >= 0 && chunk0 <= p.n_chunks - n_ch;
+    }
+    __device__ __forceinline__ const float* state0(const GdnDev& p, const float* states, int h) const {
+        int par = p.parent[node];
+        if (par >= node || par < -1) par = -1;                                     // parents precede children
+        return par >= 0 ? states + ((size_t)par * p.hv + h) * GD * GD
+                        : (p.init ? p.init + (size_t)h * GD * GD : nullptr);
+    }
+};
+
+// Wave w owns value columns c0 + 16w .. +15 of one (node, v head): its
+// 128 x 16 state slice lives in eight 16 x 16 accumulator tiles (rows
+// 16 rb + 4 (l >> 4) + v) for the whole node, split into planes once a chunk.
+// Per chunk (two 16-token tiles):
+//   V' = U - W S,  qS  (A = W / q rows from LDS, B = S from registers)
+//   O = fq qS + A V'  (B = V' from registers)
+//   S <- e^{G_L} S + k^T (fk V')  (A = k from LDS, B = fk V')
+// out may be null (the backward's recompute); chunk_sin / chunk_vp, when
+// given, receive each chunk's initial state and V' ([n_chunks, Hv, 128, 128]
+// and [n_chunks, Hv, 32, 128] floats).
+// TRUNC (the reference's per-node correction): V' = U - W S0 with S0 the
+// node's initial state for every chunk of the node. A first pass over the
+// node's chunks, while the state registers still hold S0, replaces each
+// chunk's U by its V' in the workspace; the scan proper then reads V' there.
+template <typename TIn, bool TRUNC>
+__global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn_scan_cols_kernel(GdnDev p, int lvl_begin, float* __restrict__ ws,
+                                                      TIn* __restrict__ out, float* __restrict__ states,
+                                                      float* __restrict__ chunk_sin, float* __restrict__ chunk_vp) {
+    constexpr int NQ = kInPlanes<TIn>;
+    __shared__ __attribute__((aligned(16))) FwdTiles<TIn> L;
+    ScanNode nd;
+    if (!nd.init(p, lvl_begin)) return;
+    int h, cb;
+    scan_block(p, h, cb);
+    const int t = threadIdx.x, wave = t >> 6, lane = t & 63, c16 = lane & 15, g4 = 4 * (lane >> 4);
+    const int jt = cb + 16 * wave, j = jt + c16;                          // the wave's first and this lane's column
+    const int start = nd.start, len = nd.len, chunk0 = nd.chunk0, n_ch = nd.n_ch;
+    const float* s0 = nd.state0(p, states, h);
+    f32x4 S[8];
+    if (s0) {
+#pragma unroll
+        for (int rb = 0; rb < 8; ++rb) S[rb] = load_t16(s0 + jt + 16 * rb * GD, lane);
+    } else {
+#pragma unroll
+        for (int rb = 0; rb < 8; ++rb) S[rb] = (f32x4){};
+    }
+
+    if constexpr (TRUNC) {
+        // V' = U - W S0 for every chunk (with S0 zero: V' = U as it is).
+        Op<3> s0p[4];
+#pragma unroll
+        for (int w4 = 0; w4 < 4; ++w4) s0p[w4] = op_acc(S[2 * w4], S[2 * w4 + 1]);
+        for (int c0 = 0; s0 && c0 < len; c0 += GC) {
+            float* cw = ws + ((size_t)(chunk0 + c0 / GC) * p.hv + h) * kWsChunk;
+            f32x4 w[4], vp[2];
+            const int i = t >> 3, d0 = 16 * (t & 7);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[e] = *(const f32x4*)(cw + kWsW + i * GD + d0 + 4 * e);
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb) vp[tb] = load_t16(cw + kWsU + 16 * tb * GD + jt, lane);
+            lds_barrier();   // readers of the previous chunk's W are done
+            put16<PR>(L.W, i, d0, w);
+            lds_barrier();
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb) {
+                f32x4 pv = {};
+#pragma unroll
+                for (int w4 = 0; w4 < 4; ++w4)
+                    pv = mul_planes(op_rows<3, PR>(L.W, 16 * tb + c16, 32 * w4, g4), s0p[w4], pv);
+                store_t16(cw + kWsU + 16 * tb * GD + jt, lane, vp[tb] - pv);   // read back by this lane
+            }
+        }
+    }
+
+    // U (TRUNC: V', written by the first pass) and the state-independent
+    // chunk terms, one chunk ahead.
+    ScanAhead<TIn> nx;
+    auto fetch = [&](int ci) {
+        const float* cw = ws + ((size_t)(chunk0 + ci) * p.hv + h) * kWsChunk;
+        scan_fetch_rows<TIn, !TRUNC>(p, cw, start + GC * ci, min(GC, len - GC * ci), h, nx);
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb) nx.x[tb] = load_t16(cw + kWsU + 16 * tb * GD + jt, lane);
+    };
+    if (n_ch > 0) fetch(0);
+    for (int ci = 0; ci < n_ch; ++ci) {
+        const int c0 = GC * ci, Lc = min(GC, len - c0);
+        const size_t ch = (size_t)(chunk0 + ci) * p.hv + h;
+        if (chunk_sin) {
+            float* sp = chunk_sin + ch * GD * GD + jt;
+#pragma unroll
+            for (int rb = 0; rb < 8; ++rb) store_t16(sp + 16 * rb * GD, lane, S[rb]);
+        }
+        lds_barrier();   // readers of the previous chunk's tiles are done
+        L.template stage<!TRUNC>(p, nx);
+        f32x4 vp[2] = {nx.x[0], nx.x[1]}, qs[2] = {};
+        if (ci + 1 < n_ch) fetch(ci + 1);
+        lds_barrier();
+
+        // V' = U - W S and q S over the 128 state rows as four partial sums
+        // added in order: the partition of the row layout's waves
+        // (gdn_scan_rows_kernel), so both layouts give the same bits.
+#pragma unroll
+        for (int w4 = 0; w4 < 4; ++w4) {
+            const Op<3> sp = op_acc(S[2 * w4], S[2 * w4 + 1]);
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb) {
+                if constexpr (!TRUNC)
+                    vp[tb] -= mul_planes(op_rows<3, PR>(L.W, 16 * tb + c16, 32 * w4, g4), sp, (f32x4){});
+                qs[tb] += mul_planes(op_rows<NQ, PR>(L.Q, 16 * tb + c16, 32 * w4, g4), sp, (f32x4){});
+            }
+        }
+        if (chunk_vp) {
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb) store_t16(chunk_vp + ch * GC * GD + 16 * tb * GD + jt, lane, vp[tb]);
+        }
+        // O = fq (q S) + A V', token tile by token tile.
+        if (out) {
+            const Op<3> vpl = op_acc(vp[0], vp[1]);
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb) {
+                const f32x4 av = mul_planes(op_rows<3, AR>(L.A, 16 * tb + c16, 0, g4), vpl, (f32x4){});
+                const f32x4 o = out_tok(qs[tb], L.fq, 16 * tb + g4, av);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int i = 16 * tb + g4 + v;
+                    if (i < Lc) out[((int64_t)(start + c0 + i) * p.hv + h) * GD + j] = (TIn)o[v];
+                }
+            }
+        }
+        // S <- e^{G_L} S + k^T (fk V')
+        {
+            const Op<3> vs = op_acc(scale_tok(vp[0], L.fk, g4), scale_tok(vp[1], L.fk, 16 + g4));
+            const float el = L.el;
+#pragma unroll
+            for (int rb = 0; rb < 8; ++rb)
+                S[rb] = fma_tile(S[rb], el, mul_planes(op_cols<NQ, PC>(L.K, 16 * rb, lane), vs, (f32x4){}));
+        }
+    }
+
+    // Final state of the node (the initial state of its children).
+    float* sp = states + ((size_t)nd.node * p.hv + h) * GD * GD + jt;
+#pragma unroll
+    for (int rb = 0; rb < 8; ++rb) store_t16(sp + 16 * rb * GD, lane, S[rb]);
+}
+
+// Row layout of the level scans, for levels of few nodes (the exact rule
+// only): a workgroup takes 16 value columns of one (node, v head), eight
+// workgroups per pair, and its wave w the state rows 32w .. 32w+31 of them.
+// The products over the state rows (W S and q^ S) are summed over the four
+// waves through LDS, in wave order; every wave then updates its own rows. A
+// chunk costs each wave about a quarter of the column layout's MFMAs, for
+// four times the workgroups: a level with few nodes runs a serial chain of
+// chunks on a mostly idle chip, and that chain gets shorter.
+constexpr int ROWS_COLS = 16;
+constexpr int kRowsSplit = GD / ROWS_COLS;
+__device__ __forceinline__ void rows_block(const GdnDev& p, int& h, int& c0) {
+    const int bx = blockIdx.x;
+    int cs;
+    if ((p.hv & 7) == 0) {   // the eight column blocks of a head on one XCD (same L2)
+        h = ((bx >> 6) << 3) | (bx & 7);
+        cs = (bx >> 3) & 7;
+    } else {
+        h = bx >> 3;
+        cs = bx & 7;
+    }
+    c0 = ROWS_COLS * cs;
+}
+
+template <typename TIn>
+struct ScanRowsLds {
+    FwdTiles<TIn> T;
+    f32x4 P[4][2][2][64];   // per wave: its partial W S and q S, both token tiles, lane-major
+};
+
+// As gdn_scan_cols_kernel (exact rule), in the row layout: wave w holds the
+// 32 x 16 slice S[32w .., c0 ..] in two 16 x 16 accumulator tiles.
+template <typename TIn>
+__global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn_scan_rows_kernel(GdnDev p, int lvl_begin, float* __restrict__ ws,
+                                                      TIn* __restrict__ out, float* __restrict__ states,
+                                                      float* __restrict__ chunk_sin, float* __restrict__ chunk_vp) {
+    constexpr int NQ = kInPlanes<TIn>;
+    __shared__ __attribute__((aligned(16))) ScanRowsLds<TIn> L;
+    ScanNode nd;
+    if (!nd.init(p, lvl_begin)) return;
+    int h, cb;
+    rows_block(p, h, cb);
+    const int t = threadIdx.x, wave = t >> 6, lane = t & 63, c16 = lane & 15, g4 = 4 * (lane >> 4);
+    const int j = cb + c16;                                               // this lane's value column
+    const int rb0 = 2 * wave;                                             // the wave's first row tile
+    const int start = nd.start, len = nd.len, chunk0 = nd.chunk0, n_ch = nd.n_ch;
+    const float* s0 = nd.state0(p, states, h);
+    f32x4 S[2];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) S[r] = s0 ? load_t16(s0 + cb + 16 * (rb0 + r) * GD, lane) : (f32x4){};
+
+    ScanAhead<TIn> nx;
+    auto fetch = [&](int ci) {
+        const float* cw = ws + ((size_t)(chunk0 + ci) * p.hv + h) * kWsChunk;
+        scan_fetch_rows<TIn, true>(p, cw, start + GC * ci, min(GC, len - GC * ci), h, nx);
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb) nx.x[tb] = load_t16(cw + kWsU + 16 * tb * GD + cb, lane);
+    };
+    if (n_ch > 0) fetch(0);
+    for (int ci = 0; ci < n_ch; ++ci) {
+        const int c0 = GC * ci, Lc = min(GC, len - c0);
+        const size_t ch = (size_t)(chunk0 + ci) * p.hv + h;
+        if (chunk_sin) {
+            float* sp = chunk_sin + ch * GD * GD + cb;
+#pragma unroll
+            for (int r = 0; r < 2; ++r) store_t16(sp + 16 * (rb0 + r) * GD, lane, S[r]);
+        }
+        lds_barrier();   // readers of the previous chunk's tiles and partials are done
+        L.T.template stage<true>(p, nx);
+        f32x4 vp[2] = {nx.x[0], nx.x[1]}, qs[2] = {};
+        if (ci + 1 < n_ch) fetch(ci + 1);
+        const Op<3> sp = op_acc(S[0], S[1]);
+        lds_barrier();
+
+        // this wave's rows of W S and q S
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb) {
+            L.P[wave][0][tb][lane] =
+                mul_planes(op_rows<3, PR>(L.T.W, 16 * tb + c16, 32 * wave, g4), sp, (f32x4){});
+            L.P[wave][1][tb][lane] =
+                mul_planes(op_rows<NQ, PR>(L.T.Q, 16 * tb + c16, 32 * wave, g4), sp, (f32x4){});
+        }
+        lds_barrier();
+        // V' = U - W S and q S, the partials summed in wave order
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb) {
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                vp[tb] -= L.P[w][0][tb][lane];
+                qs[tb] += L.P[w][1][tb][lane];
+            }
+        }
+        if (chunk_vp && wave == 0) {
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb) store_t16(chunk_vp + ch * GC * GD + 16 * tb * GD + cb, lane, vp[tb]);
+        }
+        // S <- e^{G_L} S + k^T (fk V') on this wave's rows
+        const Op<3> vs = op_acc(scale_tok(vp[0], L.T.fk, g4), scale_tok(vp[1], L.T.fk, 16 + g4));
+        const float el = L.T.el;
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+            S[r] = fma_tile(S[r], el, mul_planes(op_cols<NQ, PC>(L.T.K, 16 * (rb0 + r), lane), vs, (f32x4){}));
+        // O = fq (q S) + A V': waves 0 and 1 take one token tile each
+        if (out && wave < 2) {
+            const int tb = wave;
+            const Op<3> vpl = op_acc(vp[0], vp[1]);
+            const f32x4 av = mul_planes(op_rows<3, AR>(L.T.A, 16 * tb + c16, 0, g4), vpl, (f32x4){});
+            const f32x4 o = out_tok(tb ? qs[1] : qs[0], L.T.fq, 16 * tb + g4, av);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int i = 16 * tb + g4 + v;
+                if (i < Lc) out[((int64_t)(start + c0 + i) * p.hv + h) * GD + j] = (TIn)o[v];
+            }
+        }
+    }
+
+    float* sp = states + ((size_t)nd.node * p.hv + h) * GD * GD + cb;
+#pragma unroll
+    for (int r = 0; r < 2; ++r) store_t16(sp + 16 * (rb0 + r) * GD, lane, S[r]);
+}
+
+// ----------------------------------------------------------------------------
+// reverse scan
+// ----------------------------------------------------------------------------
+// dS after a node, NT 16-row tiles from row tile rb0 at the columns of
+// `col0`: its state's incoming gradient, if any, plus the sum over its
+// children of their dS at entry.
+template <int NT>
+__device__ __forceinline__ void rscan_start(const GdnDev& p, int node, int h, int rb0, int col0, int lane,
+                                            const float* node_dsin, f32x4 (&dS)[NT]) {
+    if (p.d_states && (!p.d_states_last || node == p.n_nodes - 1)) {
+        const float* sp = p.d_states + ((size_t)(p.d_states_last ? 0 : node) * p.hv + h) * GD * GD + col0;
+#pragma unroll
+        for (int r = 0; r < NT; ++r) dS[r] = load_t16(sp + 16 * (rb0 + r) * GD, lane);
+    } else {
+#pragma unroll
+        for (int r = 0; r < NT; ++r) dS[r] = (f32x4){};
+    }
+    const int c_lo = max(p.child_off[node], 0), c_hi = min(p.child_off[node + 1], p.n_nodes);
+    for (int ci = c_lo; ci < c_hi; ++ci) {
+        const int child = p.child[ci];
+        if (child <= node || child >= p.n_nodes) continue;              // children follow their parent
+        const float* sp = node_dsin + ((size_t)child * p.hv + h) * GD * GD + col0;
+#pragma unroll
+        for (int r = 0; r < NT; ++r) dS[r] += load_t16(sp + 16 * (rb0 + r) * GD, lane);
+    }
+}
+// The chunk terms and this lane's dO tiles (column j, zero past the chunk).
+template <typename TIn, bool LOAD_W>
+__device__ __forceinline__ void rscan_fetch(const GdnDev& p, const ScanNode& nd, int ci, int h, int j, int g4,
+                                            const float* ws, const TIn* d_o, int64_t do_st, int64_t do_sh,
+                                            ScanAhead<TIn>& x) {
+    const int c0 = GC * ci, Lc = min(GC, nd.len - c0);
+    const float* cw = ws + ((size_t)(nd.chunk0 + ci) * p.hv + h) * kWsChunk;
+    scan_fetch_rows<TIn, LOAD_W>(p, cw, nd.start + c0, Lc, h, x);
+    const TIn* base = d_o + (int64_t)(nd.start + c0) * do_st + (int64_t)h * do_sh + j;
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int i = 16 * tb + g4 + v;
+            x.x[tb][v] = i < Lc ? (float)base[(int64_t)i * do_st] : 0.0f;
+        }
+}
+// dO as an operand: its bf16 values as they are, or three planes.
+template <typename TIn>
+__device__ __forceinline__ Op<kInPlanes<TIn>> op_in(const f32x4& t0, const f32x4& t1) {
+    if constexpr (kInPlanes<TIn> == 1)
+        return {{pack8(t0[0], t0[1], t0[2], t0[3], t1[0], t1[1], t1[2], t1[3])}};
+    else
+        return op_acc(t0, t1);
+}
+
+// Column layout as gdn_scan_cols_kernel (scan_block). Wave w owns value
+// columns c0 + 16w .. +15: its 128 x 16 slice of dS lives in eight 16 x 16
+// accumulator tiles, dO of the chunk is loaded in accumulator layout (rows =
+// tokens, two 16-token tiles), and dV' is produced in it, so all three are
+// MFMA B operands straight from registers:
+//   dV' = A^T dO + fk (k dS),  dS <- e^{G_L} dS + q^T (fq dO) - W^T dV'.
+// TRUNC (V' = U - W S0 with the node's initial state S0): the walk leaves out
+// the W term, and a second pass over the node's chunks subtracts
+// sum_c W_c^T dV'_c from the state gradient at the node's entry.
+template <typename TIn, bool TRUNC>
+__global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn_rscan_cols_kernel(
+        GdnDev p, int lvl_begin, const float* __restrict__ ws, const TIn* __restrict__ d_o, int64_t do_st,
+        int64_t do_sh, float* __restrict__ chunk_dso, float* __restrict__ chunk_dvp, float* __restrict__ node_dsin) {
+    constexpr int NQ = kInPlanes<TIn>;
+    __shared__ __attribute__((aligned(16))) RevTiles<TIn> L;
+    ScanNode nd;
+    if (!nd.init(p, lvl_begin) || nd.len < 1) return;
+    int h, cb;
+    scan_block(p, h, cb);
+    const int t = threadIdx.x, wave = t >> 6, lane = t & 63, c16 = lane & 15, g4 = 4 * (lane >> 4);
+    const int jt = cb + 16 * wave, j = jt + c16;
+    f32x4 dS[8];
+    rscan_start<8>(p, nd.node, h, 0, jt, lane, node_dsin, dS);
+
+    // one chunk ahead (the walk runs backwards)
+    ScanAhead<TIn> nx;
+    rscan_fetch<TIn, !TRUNC>(p, nd, nd.n_ch - 1, h, j, g4, ws, d_o, do_st, do_sh, nx);
+    for (int ci = nd.n_ch - 1; ci >= 0; --ci) {
+        const size_t chn = (size_t)(nd.chunk0 + ci) * p.hv + h;
+        {   // the gradient of this chunk's output state
+            float* sp = chunk_dso + chn * GD * GD + jt;
+#pragma unroll
+            for (int rb = 0; rb < 8; ++rb) store_t16(sp + 16 * rb * GD, lane, dS[rb]);
+        }
+        lds_barrier();   // readers of the previous chunk's tiles are done
+        L.template stage<!TRUNC>(p, nx);
+        const f32x4 dov[2] = {nx.x[0], nx.x[1]};
+        if (ci > 0) rscan_fetch<TIn, !TRUNC>(p, nd, ci - 1, h, j, g4, ws, d_o, do_st, do_sh, nx);
+        lds_barrier();
+
+        // dV' as four partial sums added in order, partial w4 holding the
+        // state rows 32 w4 .. +31 and (w4 < 2) the A^T dO term of token tile
+        // w4: the partition of the row layout's waves (gdn_rscan_rows_kernel),
+        // so both layouts give the same bits.
+        const Op<NQ> dop = op_in<TIn>(dov[0], dov[1]);
+        f32x4 dv[2] = {};
+#pragma unroll
+        for (int w4 = 0; w4 < 4; ++w4) {
+            const Op<3> sp = op_acc(dS[2 * w4], dS[2 * w4 + 1]);
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb) {
+                f32x4 pd = scale_tok(
+                    mul_planes(op_rows<NQ, PR>(L.K, 16 * tb + c16, 32 * w4, g4), sp, (f32x4){}), L.fk, 16 * tb + g4);
+                if (tb == w4) pd = mul_planes(op_cols<3, AC>(L.A, 16 * tb, lane), dop, pd);
+                dv[tb] += pd;
+            }
+        }
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb) store_t16(chunk_dvp + chn * GC * GD + 16 * tb * GD + jt, lane, dv[tb]);
+
+        // dS <- e^{G_L} dS + q^T (fq dO) - W^T dV'
+        const Op<3> dos = op_acc(scale_tok(dov[0], L.fq, g4), scale_tok(dov[1], L.fq, 16 + g4));
+        const Op<3> dvs = op_acc(-dv[0], -dv[1]);
+        const float el = L.el;
+#pragma unroll
+        for (int rb = 0; rb < 8; ++rb) {
+            f32x4 x = mul_planes(op_cols<NQ, PC>(L.Q, 16 * rb, lane), dos, (f32x4){});
+            if constexpr (!TRUNC) x = mul_planes(op_cols<3, PC>(L.W, 16 * rb, lane), dvs, x);
+            dS[rb] = fma_tile(dS[rb], el, x);
+        }
+    }
+    if constexpr (TRUNC) {
+        for (int ci = 0; ci < nd.n_ch; ++ci) {
+            const size_t chn = (size_t)(nd.chunk0 + ci) * p.hv + h;
+            const float* cw = ws + chn * kWsChunk;
+            const int i = t >> 3, d0 = 16 * (t & 7);
+            f32x4 w[4], dv[2];   // dV': this lane's own writes
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[e] = *(const f32x4*)(cw + kWsW + i * GD + d0 + 4 * e);
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb) dv[tb] = load_t16(chunk_dvp + chn * GC * GD + 16 * tb * GD + jt, lane);
+            lds_barrier();   // readers of the previous chunk's W are done
+            put16<PC>(L.W, i, d0, w);
+            lds_barrier();
+            const Op<3> dvs = op_acc(-dv[0], -dv[1]);
+#pragma unroll
+            for (int rb = 0; rb < 8; ++rb) dS[rb] += mul_planes(op_cols<3, PC>(L.W, 16 * rb, lane), dvs, (f32x4){});
+        }
+    }
+    // dS at the node's entry, summed into its parent by the next (shallower) level.
+    float* sp = node_dsin + ((size_t)nd.node * p.hv + h) * GD * GD + jt;
+#pragma unroll
+    for (int rb = 0; rb < 8; ++rb) store_t16(sp + 16 * rb * GD, lane, dS[rb]);
+}
+
+template <typename TIn>
+struct RscanRowsLds {
+    RevTiles<TIn> T;
+    f32x4 P[4][2][64];   // per wave: its partial dV', both token tiles, lane-major
+};
+
+// As gdn_rscan_cols_kernel (exact rule), in the row layout of
+// gdn_scan_rows_kernel: wave w holds dS[32w .., c0 ..]. dV' is summed over the
+// waves' rows through LDS, in wave order (waves 0 and 1 also add the A^T dO
+// term of token tiles 0 and 1); every wave then updates its rows of dS.
+template <typename TIn>
+__global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn_rscan_rows_kernel(
+        GdnDev p, int lvl_begin, const float* __restrict__ ws, const TIn* __restrict__ d_o, int64_t do_st,
+        int64_t do_sh, float* __restrict__ chunk_dso, float* __restrict__ chunk_dvp, float* __restrict__ node_dsin) {
+    constexpr int NQ = kInPlanes<TIn>;
+    __shared__ __attribute__((aligned(16))) RscanRowsLds<TIn> L;
+    ScanNode nd;
+    if (!nd.init(p, lvl_begin) || nd.len < 1) return;
+    int h, cb;
+    rows_block(p, h, cb);
+    const int t = threadIdx.x, wave = t >> 6, lane = t & 63, c16 = lane & 15, g4 = 4 * (lane >> 4);
+    const int j = cb + c16;
+    const int rb0 = 2 * wave;
+    f32x4 dS[2];
+    rscan_start<2>(p, nd.node, h, rb0, cb, lane, node_dsin, dS);
+
+    ScanAhead<TIn> nx;
+    rscan_fetch<TIn, true>(p, nd, nd.n_ch - 1, h, j, g4, ws, d_o, do_st, do_sh, nx);
+    for (int ci = nd.n_ch - 1; ci >= 0; --ci) {
+        const size_t chn = (size_t)(nd.chunk0 + ci) * p.hv + h;
+        {
+            float* sp = chunk_dso + chn * GD * GD + cb;
+#pragma unroll
+            for (int r = 0; r < 2; ++r) store_t16(sp + 16 * (rb0 + r) * GD, lane, dS[r]);
+        }
+        lds_barrier();   // readers of the previous chunk's tiles and partials are done
+        L.T.template stage<true>(p, nx);
+        const f32x4 dov[2] = {nx.x[0], nx.x[1]};
+        if (ci > 0) rscan_fetch<TIn, true>(p, nd, ci - 1, h, j, g4, ws, d_o, do_st, do_sh, nx);
+        const Op<3> sp = op_acc(dS[0], dS[1]);
+        lds_barrier();
+
+        const Op<NQ> dop = op_in<TIn>(dov[0], dov[1]);
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb) {
+            f32x4 pd = scale_tok(mul_planes(op_rows<NQ, PR>(L.T.K, 16 * tb + c16, 32 * wave, g4), sp, (f32x4){}),
+                                 L.T.fk, 16 * tb + g4);
+            if (tb == wave) pd = mul_planes(op_cols<3, AC>(L.T.A, 16 * tb, lane), dop, pd);
+            L.P[wave][tb][lane] = pd;
+        }
+        lds_barrier();
+        f32x4 dv[2] = {};
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb) {
+#pragma unroll
+            for (int w = 0; w < 4; ++w) dv[tb] += L.P[w][tb][lane];
+        }
+        if (wave == 0) {
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb) store_t16(chunk_dvp + chn * GC * GD + 16 * tb * GD + cb, lane, dv[tb]);
+        }
+
+        // dS <- e^{G_L} dS + q^T (fq dO) - W^T dV' on this wave's rows
+        const Op<3> dos = op_acc(scale_tok(dov[0], L.T.fq, g4), scale_tok(dov[1], L.T.fq, 16 + g4));
+        const Op<3> dvs = op_acc(-dv[0], -dv[1]);
+        const float el = L.T.el;
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            f32x4 x = mul_planes(op_cols<NQ, PC>(L.T.Q, 16 * (rb0 + r), lane), dos, (f32x4){});
+            x = mul_planes(op_cols<3, PC>(L.T.W, 16 * (rb0 + r), lane), dvs, x);
+            dS[r] = fma_tile(dS[r], el, x);
+        }
+    }
+    float* sp = node_dsin + ((size_t)nd.node * p.hv + h) * GD * GD + cb;
+#pragma unroll
+    for (int r = 0; r < 2; ++r) store_t16(sp + 16 * (rb0 + r) * GD, lane, dS[r]);
+}
+
+}  // namespace
