@@ -441,239 +441,263 @@ __global__ __launch_bounds__(GT) void gdn_dw_s0_kernel(GdnDev p, const float* __
     store_acc<0>(acc_mat(dwo + chn * GC * GD, GC, half, 32 * wave + col), -w);
 }
 
+// One 16 x 16 quadrant a wave of a 32 x 32 product: rows 16 qi + g4 + v,
+// column 16 qj + c16, in accumulator layout.
+template <typename TIn>
 struct ChunkGradLds {
-    float Qs[GC * RS];    // q^ * scale
-    float Ks[GC * RS];    // k^
-    float P1[GC * RS];
-    float P2[GC * RS];
-    float P3[GC * RS];    // v; later Y = T^T dT (stride MS)
-    float KK[GC * MS];    // k^ k^T
-    float M1[GC * MS];    // A -> dP -> dT -> E
-    float M2[GC * MS];    // T
-    float M3[GC * MS];    // dA * A + dN * N (the pair terms of dG)
-    float R[4][GC * RR];  // per-wave partial 32 x 32 products (contraction split over the waves)
-    float G[GC];
-    float Glo[GC];
-    float B[GC];
-    float Grow[GC];
-    float Crow[GC];
+    static constexpr int NQ = kInPlanes<TIn>;
+    __bf16 Q[NQ * GC * PC];   // q and k as they come
+    __bf16 K[NQ * GC * PC];
+    union {
+        __bf16 X[3 * GC * PR];   // V', then dV', then dW
+        float J[GC * RS];        // the last join of product and element-wise terms
+    };
+    union {
+        __bf16 P[2 * 3 * GC * AC];   // dP fk_j and dP fq_i
+        float Y[GC * MS];            // Y = T^T dT
+    };
+    float T[GC * MS];
+    float M[GC * MS];     // dT, then E
+    float S[GC * MS];     // dA * A + dN * N (the pair terms of dG), then its row prefix sums
+    float G[GC], Glo[GC], B[GC], Bg[GC], fq[GC], fk[GC];   // Bg: beta e^G
+    float Grow[GC], Crow[GC];
+    float bv[2][GC], bk[2][GC];   // column sums over the row tiles of T * (dV' v^T), T * (dW k^^T)
+    float db[2][GC];              // row sums over the column tiles of the pair terms of dbeta
 };
 
-// Thread t owns row i = t/8 of the element-wise work: in [GC x GD] results
-// the columns 32m + 4s + e (s = t%8, m, e < 4), in [GC x GC] results s + 8e.
-// The products run on fp32 MFMA: a [GC x GD] result is split by columns
-// (wave w: columns 32w .. 32w+31, in accumulator layout), a [GC x GC] one by
-// contraction (wave w: k in [32w, 32w+32), partials summed through LDS).
+// Four fp32 values at columns c0 .. c0 + 3 of row i of a tile of planes.
+template <int N, int P>
+__device__ __forceinline__ f32x4 row4(const __bf16* X, int i, int c0) {
+    f32x4 r = load4(X + i * P + c0);
+    if constexpr (N == 3) {
+        r += load4(X + GC * P + i * P + c0);
+        r += load4(X + 2 * GC * P + i * P + c0);
+    }
+    return r;
+}
+// A row of the problem dtype as an operand: columns k0 + g4 .. +3 and
+// k0 + 16 + g4 .. +3 (zeros when the row does not exist).
+template <typename TIn>
+__device__ __forceinline__ Op<kInPlanes<TIn>> op_global(const TIn* row, bool in, int k0, int g4) {
+    if constexpr (kInPlanes<TIn> == 1) {
+        const bf16x4 z = {};
+        return {{cat44(in ? *(const bf16x4*)(row + k0 + g4) : z, in ? *(const bf16x4*)(row + k0 + 16 + g4) : z)}};
+    } else {
+        const f32x4 z = {};
+        return op_acc(in ? load4(row + k0 + g4) : z, in ? load4(row + k0 + 16 + g4) : z);
+    }
+}
+// Column operand f X[k][c0 + c16] of a [GC][MS] fp32 matrix, k over its 32 rows.
+__device__ __forceinline__ Op<3> op_fcols(const float* X, int c0, int c16, int g4, float f) {
+    f32x4 a, b;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        a[v] = f * X[(g4 + v) * MS + c0 + c16];
+        b[v] = f * X[(16 + g4 + v) * MS + c0 + c16];
+    }
+    return op_acc(a, b);
+}
+// A [32 x 32] accumulator quadrant into planes with rows of AC elements.
+__device__ __forceinline__ void put_quadrant(__bf16* X, int row, int colj, const f32x4& x) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        float r = x[v];
+#pragma unroll
+        for (int n = 0; n < 3; ++n) {
+            const __bf16 b = (__bf16)r;
+            X[n * GC * AC + (row + v) * AC + colj] = b;
+            r -= (float)b;
+        }
+    }
+}
+// The compiler moves no work across: overlapped, the phases of a head do not
+// fit the registers.
+__device__ __forceinline__ void phase() { __builtin_amdgcn_sched_barrier(0); }
+__device__ __forceinline__ float sum16(float x) {   // over the 16 lanes of a row of accumulators
+    x += __shfl_xor(x, 1);
+    x += __shfl_xor(x, 2);
+    x += __shfl_xor(x, 4);
+    return x + __shfl_xor(x, 8);
+}
+
+// Products by tiles of v_mfma_f32_16x16x32_bf16 on planes: a [32 x 32] result
+// is a quadrant a wave (the upper one holds nothing that is read and is left
+// out), a [32 x 128] one 32 columns a wave. The three [32 x 128] inputs that
+// need splitting (V', dV', dW) pass through one LDS tile in turn, each loaded a
+// phase ahead; q, k, v and dO of bf16 problems are used as they come. A head
+// is a chain of nine barriers, so latency bounds the kernel: 78 KB of LDS and
+// 256 registers (bf16) let two workgroups share a CU, one working behind the
+// other's barriers and loads. 16K agent tree, 16/32 heads, bf16: 1553 -> 1032
+// us against one workgroup a CU on fp32 MFMAs (120 KB, sums of four partial
+// products through LDS); fp32, 2,081 tokens, 4/8 heads: 84 -> 70 us.
+// Element-wise work: thread t owns row i = t/8 and columns 32m + 4s + e
+// (s = t%8; m, e < 4) of [32 x 128] rows; [32 x 32] results stay in the
+// quadrant layout.
 // TRUNC (the reference's per-node correction): U and W do not come from the
 // chunk's T, so the T part is left out; dv and dbeta are complete already
 // (tt_gdn_trunc.hip), and trk (dk^ of the correction, [chunk, Hv, 32, 128])
 // and trg (the node-level suffix sums of its dG, [chunk, Hv, 32]) are added.
 template <typename TIn, bool TRUNC>
-__global__ __launch_bounds__(GT) void gdn_bwd_chunk_kernel(GdnDev p, const TIn* __restrict__ d_o, int64_t do_st,
-                                                           int64_t do_sh, const float* __restrict__ ws,
-                                                           const float* __restrict__ chunk_vp,
-                                                           const float* __restrict__ chunk_dvp,
-                                                           const float* __restrict__ xo, const float* __restrict__ dwo,
-                                                           const float* __restrict__ dkto,
-                                                           const float* __restrict__ sdot, TIn* __restrict__ dq,
-                                                           TIn* __restrict__ dk, TIn* __restrict__ dv,
-                                                           float* __restrict__ dg, float* __restrict__ dbeta,
-                                                           const float* __restrict__ trk, const float* __restrict__ trg) {
-    __shared__ __attribute__((aligned(16))) ChunkGradLds L;
+__global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(sizeof(TIn) == 2 ? 2 : 1, 2))) void gdn_bwd_chunk_kernel(
+        GdnDev p, const TIn* __restrict__ d_o, int64_t do_st, int64_t do_sh, const float* __restrict__ ws,
+        const float* __restrict__ chunk_vp, const float* __restrict__ chunk_dvp, const float* __restrict__ xo,
+        const float* __restrict__ dwo, const float* __restrict__ dkto, const float* __restrict__ sdot,
+        TIn* __restrict__ dq, TIn* __restrict__ dk, TIn* __restrict__ dv, float* __restrict__ dg,
+        float* __restrict__ dbeta, const float* __restrict__ trk, const float* __restrict__ trg) {
+    constexpr int NQ = kInPlanes<TIn>;
+    __shared__ __attribute__((aligned(16))) ChunkGradLds<TIn> L;
     const int c = blockIdx.x, hk = blockIdx.y, t = threadIdx.x;
     int start, len;
     if (!chunk_span(p, c, start, len)) return;
     const int i = t >> 3, s = t & 7;
-    const int wave = t >> 6, lane = t & 63, col = lane & 31, half = lane >> 5, cw0 = 32 * wave;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, c16 = lane & 15, g4 = 4 * (lane >> 4);
+    const int qi = wave >> 1, qj = wave & 1;            // this wave's quadrant ...
+    const bool lower = qi >= qj;                        // ... and whether it holds pairs j <= i
+    const int qr = 16 * qi + g4, qc = 16 * qj + c16;    // this lane's first row and its column there
+    const int w0 = 32 * wave;                           // this wave's columns of [32 x 128] results
     const bool valid = i < len;
     const int64_t tok = start + i;
 
-    load_chunk_rows<TIn>(p, start, len, hk * p.rep, L.Qs, L.Ks, nullptr);
-    __syncthreads();
-    put_partial(L.R[wave], quarter_nt(L.Ks, L.Ks, 1.0f, col, half, wave, (f32x16){}), col, half);   // k^ k^T
-    __syncthreads();
+    {   // q and k rows as they come, and their norms
+        using Vec = typename std::conditional<sizeof(TIn) == 2, bf16x8, f32x4>::type;
+        constexpr int NV = (int)sizeof(TIn), EV = 16 / NV;
+        Vec qv[NV], kv[NV];
+        const TIn* qp = (const TIn*)p.q + tok * p.q_st + (int64_t)hk * p.q_sh + 16 * s;
+        const TIn* kp = (const TIn*)p.k + tok * p.k_st + (int64_t)hk * p.k_sh + 16 * s;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int j = s + 8 * e;
-        L.KK[i * MS + j] = L.R[0][i * RR + j] + L.R[1][i * RR + j] + L.R[2][i * RR + j] + L.R[3][i * RR + j];
+        for (int n = 0; n < NV; ++n) {
+            if (valid) {
+                qv[n] = *(const Vec*)(qp + EV * n);
+                kv[n] = *(const Vec*)(kp + EV * n);
+            } else {
+#pragma unroll
+                for (int e = 0; e < EV; ++e) qv[n][e] = kv[n][e] = (TIn)0.0f;
+            }
+        }
+        put16<PC>(L.Q, i, 16 * s, qv);
+        put16<PC>(L.K, i, 16 * s, kv);
+        const float nq = row_norm(p, qv), nk = row_norm(p, kv);
+        if (s == 0) {
+            L.fq[i] = nq * p.scale;
+            L.fk[i] = nk;
+        }
+    }
+    // One of the [32 x 128] fp32 inputs of a head on its way to L.X: row i,
+    // columns 16 s .. +15.
+    f32x4 xr[4];
+    auto fetch_x = [&](const float* src, size_t chn) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) xr[e] = *(const f32x4*)(src + (chn * GC + i) * GD + 16 * s + 4 * e);
+    };
+    const size_t chn0 = (size_t)c * p.hv + hk * p.rep;
+    fetch_x(chunk_vp, chn0);
+    lds_barrier();
+    f32x4 kk = {};   // k^ k^T
+    if (!TRUNC && lower) {
+        Sum2 x;
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+            x.add(op_rows<NQ, PC>(L.K, 16 * qi + c16, 32 * m, g4), op_rows<NQ, PC>(L.K, 16 * qj + c16, 32 * m, g4));
+        kk = x.sum();
+#pragma unroll
+        for (int v = 0; v < 4; ++v) kk[v] *= L.fk[qr + v] * L.fk[qc];
     }
     float dqa[16], dka[16];   // element-wise terms (row layout)
 #pragma unroll
     for (int e = 0; e < 16; ++e) dqa[e] = dka[e] = 0.0f;
-    f32x16 dqm = {}, dkm = {};   // product terms (accumulator layout, columns cw0 + col)
+    f32x4 dqm[2][2] = {}, dkm[2][2] = {};   // product terms: row tile, column tile w0 + 16 cb
 
 #pragma unroll 1
     for (int hh = 0; hh < p.rep; ++hh) {
         const int h = hk * p.rep + hh;
-        const size_t chn = (size_t)c * p.hv + h;
+        const size_t chn = chn0 + hh;
+        // The thread's coordinates, made opaque to the compiler once a head and
+        // again halfway: hoisted out of the loop, the LDS and global addresses
+        // made of them spill 150 registers.
+#define TT_CHUNK_COORDS()                                                                                \
+    int to = threadIdx.x;                                                                                \
+    asm volatile("" : "+v"(to));                                                                         \
+    const int i = to >> 3, s = to & 7, lane = to & 63, c16 = lane & 15, g4 = 4 * (lane >> 4);            \
+    const int qr = 16 * qi + g4, qc = 16 * qj + c16;                                                     \
+    (void)i, (void)s, (void)lane, (void)c16, (void)g4, (void)qr, (void)qc
+        TT_CHUNK_COORDS();
+        const bool valid = i < len;
+        const int64_t tok = start + i;
         const float* cw = ws + chn * kWsChunk;
         // e^{G_L} <S, dS> for dg, loaded here so its latency hides behind the head's work
-        const float gsd = t < GC ? sdot[chn] : 0.0f;
-        __syncthreads();   // the previous head's readers are done
-        if (t < GC) {
-            L.G[t] = cw[kWsG + t];
-            L.Glo[t] = cw[kWsGlo + t];
-            L.B[t] = t < len ? p.beta[(int64_t)(start + t) * p.b_st + h] : 0.0f;
-        }
-        tile_in(d_o + (int64_t)start * do_st + (int64_t)h * do_sh, do_st, len, L.P1);
-        tile_in(chunk_vp + chn * GC * GD, GD, GC, L.P2);
+        const float gsd = sdot[chn];
+        f32x4 aq;   // this lane's entries of A
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int j = s + 8 * e;
-            L.M1[i * MS + j] = cw[kWsA + i * GC + j];
-            if constexpr (!TRUNC) L.M2[i * MS + j] = cw[kWsT + i * GC + j];
-        }
-        __syncthreads();
-        // dA = dO V'^T (partials per wave)
-        put_partial(L.R[wave], quarter_nt(L.P1, L.P2, 1.0f, col, half, wave, (f32x16){}), col, half);
-        __syncthreads();
-        const float gi = L.G[i], gl = L.G[GC - 1], egi = expf(gi), bi = L.B[i];
-        const float gil = L.Glo[i], gll = L.Glo[GC - 1];
-        // this thread's share of row i's own dG terms (those of e^{G_i} alone), dbeta, c
-        float dgp = 0.0f, dbp = 0.0f, cp = 0.0f;
-
-        // dG from A = (q^ k^T) * D, then dP = dA * D (j <= i).
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int j = s + 8 * e;
-            const float da = L.R[0][i * RR + j] + L.R[1][i * RR + j] + L.R[2][i * RR + j] + L.R[3][i * RR + j];
-            const float dae = j <= i ? da : 0.0f;
-            const float pa = dae * L.M1[i * MS + j];
-            L.M3[i * MS + j] = pa;
-            L.M1[i * MS + j] = j <= i ? dae * expf(gdiff(gi, gil, L.G[j], L.Glo[j])) : 0.0f;
-        }
-        // O's state term e^G q^ S: dq^ += e^G X, dG += e^G q^ . X.
+        for (int v = 0; v < 4; ++v) aq[v] = cw[kWsA + (qr + v) * GC + qc];
+        Op<NQ> dop[4];   // dO rows of the quadrant's row tile
         {
-            const float* xr = xo + chn * GC * GD + i * GD;
-            float xq = 0.0f;
+            const TIn* row = d_o + (int64_t)(start + 16 * qi + c16) * do_st + (int64_t)h * do_sh;
 #pragma unroll
-            for (int m = 0; m < 4; ++m) {
-                const f32x4 x = *(const f32x4*)(xr + 32 * m + 4 * s);
-                const f32x4 q = *(const f32x4*)&L.Qs[i * RS + 32 * m + 4 * s];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) dqa[4 * m + e] = fmaf(egi, x[e], dqa[4 * m + e]);
-                xq += dot4(q, x);
-            }
-            dgp = fmaf(egi, xq, dgp);
+            for (int m = 0; m < 4; ++m) dop[m] = op_global<TIn>(row, 16 * qi + c16 < len, 32 * m, g4);
         }
-        __syncthreads();   // dP complete
-        // dq^ += dP k^, dk^ += dP^T q^ (contraction over the chunk's 32 tokens).
-#pragma unroll
-        for (int m = 0; m < 4; ++m) {
-            const f32x4 a = op_row4(L.M1, MS, col, half, 0, m);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int r = 4 * m + e;
-                dqm = mfma_f32(a[e], op_col(L.Ks, RS, half, 0, r, cw0, col), dqm);
-                dkm = mfma_f32(op_col(L.M1, MS, half, 0, r, 0, col), op_col(L.Qs, RS, half, 0, r, cw0, col), dkm);
-            }
+        // the previous head's last readers of X, T, G and B are two barriers back
+        put16<PR>(L.X, i, 16 * s, xr);
+        if constexpr (!TRUNC) *(f32x4*)&L.T[i * MS + 4 * s] = *(const f32x4*)(cw + kWsT + i * GC + 4 * s);
+        if (t < GC) {
+            const float gt = cw[kWsG + t], bt = t < len ? p.beta[(int64_t)(start + t) * p.b_st + h] : 0.0f;
+            L.G[t] = gt;
+            L.Glo[t] = cw[kWsGlo + t];
+            L.B[t] = bt;
+            L.Bg[t] = bt * expf(gt);
         }
-        if constexpr (!TRUNC) {
-            __syncthreads();   // P1, P2 and R readers are done
-            tile_in(chunk_dvp + chn * GC * GD, GD, GC, L.P1);
-            tile_in(dwo + chn * GC * GD, GD, GC, L.P2);
-            tile_in((const TIn*)p.v + (int64_t)start * p.v_st + (int64_t)h * p.v_sh, p.v_st, len, L.P3);
-            __syncthreads();
+        if constexpr (!TRUNC) fetch_x(chunk_dvp, chn);
+        lds_barrier();
+        const float gi = L.G[i], gl = L.G[GC - 1], egi = expf(gi);
+        const float ed = expf(gdiff(gl, L.Glo[GC - 1], gi, L.Glo[i])), egl = expf(gl);
+        const float bj = L.B[qc], ej = expf(L.G[qc] + L.Glo[qc]), fkj = L.fk[qc];
 
-            // dT = dV' (beta v)^T + dW (beta e^G k^)^T (partials per wave); dBv =
-            // T^T dV', dBk = T^T dW (columns of this wave).
-            {
-                const float bj = L.B[col], bgj = bj * expf(L.G[col] + L.Glo[col]);
-                f32x16 tp = quarter_nt(L.P1, L.P3, bj, col, half, wave, (f32x16){});
-                tp = quarter_nt(L.P2, L.Ks, bgj, col, half, wave, tp);
-                put_partial(L.R[wave], tp, col, half);
+        // dA = dO V'^T; the pair terms dA * A of dG; dP = dA * D (j <= i), once
+        // times fk_j (for dq^) and once times fq_i (for dk^).
+        f32x4 pair = {};
+        {
+            f32x4 da = {};
+            if (lower) {
+                Sum2 x;
+#pragma unroll
+                for (int m = 0; m < 4; ++m) x.add(dop[m], op_rows<3, PR>(L.X, 16 * qj + c16, 32 * m, g4));
+                da = x.sum();
             }
-            f32x16 dbvm = {}, dbkm = {};
+            f32x4 pk, pq;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float a = op_col(L.M2, MS, half, 0, r, 0, col);
-                dbvm = mfma_f32(a, op_col(L.P1, RS, half, 0, r, cw0, col), dbvm);
-                dbkm = mfma_f32(a, op_col(L.P2, RS, half, 0, r, cw0, col), dbkm);
+            for (int v = 0; v < 4; ++v) {
+                const int r = qr + v;
+                const bool in = qc <= r;
+                const float x = in ? da[v] : 0.0f;
+                pair[v] = x * aq[v];
+                const float dpv = in ? x * expf(gdiff(L.G[r], L.Glo[r], L.G[qc], L.Glo[qc])) : 0.0f;
+                pk[v] = v & 1 ? -(dpv * fkj) : dpv * fkj;   // rows i of dP: alt(i)
+                pq[v] = dpv * (L.fq[r] * alt(c16));         // rows j of dP^T: alt(j)
             }
-            __syncthreads();   // R complete; P1, P2 readers are done
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                L.P1[acc_row(r, half) * RS + cw0 + col] = dbvm[r];
-                L.P2[acc_row(r, half) * RS + cw0 + col] = dbkm[r];
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int j = s + 8 * e;
-                L.M1[i * MS + j] = L.R[0][i * RR + j] + L.R[1][i * RR + j] + L.R[2][i * RR + j] + L.R[3][i * RR + j];
-            }
-            __syncthreads();   // dBv, dBk and dT complete
-            // dv = beta dBv; dbeta, dk^, dG from U = T (beta v) and W = T (beta e^G k^).
-            {
-                float vb = 0.0f, kb = 0.0f;
-                const float bge = bi * egi;
-#pragma unroll
-                for (int m = 0; m < 4; ++m) {
-                    const f32x4 vv = *(const f32x4*)&L.P3[i * RS + 32 * m + 4 * s];
-                    const f32x4 kv = *(const f32x4*)&L.Ks[i * RS + 32 * m + 4 * s];
-                    const f32x4 dbv = *(const f32x4*)&L.P1[i * RS + 32 * m + 4 * s];
-                    const f32x4 dbk = *(const f32x4*)&L.P2[i * RS + 32 * m + 4 * s];
-                    f32x4 o;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        vb = fmaf(vv[e], dbv[e], vb);
-                        kb = fmaf(kv[e], dbk[e], kb);
-                        dka[4 * m + e] = fmaf(bge, dbk[e], dka[4 * m + e]);
-                        o[e] = bi * dbv[e];
-                    }
-                    if (valid) store4(dv + tok * p.dv_st + h * GD + 32 * m + 4 * s, o);
-                }
-                dbp += vb + egi * kb;
-                dgp = fmaf(bge, kb, dgp);
-            }
-            __syncthreads();   // P3 (v) readers are done
-            // Y = T^T dT into P3 (stride MS)
-            {
-                float y[4] = {};
-#pragma unroll 4
-                for (int m = 0; m < GC; ++m) {
-                    const float tmi = L.M2[m * MS + i];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) y[e] = fmaf(tmi, L.M1[m * MS + s + 8 * e], y[e]);
-                }
-#pragma unroll
-                for (int e = 0; e < 4; ++e) L.P3[i * MS + s + 8 * e] = y[e];
-            }
-            __syncthreads();
-            // dN = Y T^T (strictly lower): dbeta, dG and E = dL/d(k^ k^T) from
-            // N = -beta (k^ k^T) * D.
-            {
-                float ev[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int j = s + 8 * e;
-                    float dn = 0.0f;
-#pragma unroll 4
-                    for (int m = 0; m < GC; ++m) dn = fmaf(L.P3[i * MS + m], L.M2[j * MS + m], dn);
-                    ev[e] = 0.0f;
-                    if (j < i) {
-                        const float dd = expf(gdiff(gi, gil, L.G[j], L.Glo[j])), kk = L.KK[i * MS + j];
-                        const float pa = dn * (-bi * kk * dd);
-                        dbp = fmaf(dn, -kk * dd, dbp);
-                        ev[e] = -dn * bi * dd;
-                        L.M3[i * MS + j] += pa;
-                    }
-                }
-#pragma unroll
-                for (int e = 0; e < 4; ++e) L.M1[i * MS + s + 8 * e] = ev[e];   // dT's readers passed the last barrier
-            }
-            __syncthreads();
-            // dk^ += (E + E^T) k^
+            put_quadrant(L.P, qr, qc, pk);
+            put_quadrant(L.P + 3 * GC * AC, qr, qc, pq);
+        }
+        phase();
+        // O's state term e^G q^ S: dq^ += e^G X, dG += e^G q^ . X; the output
+        // state's (e^{G_L - G} k^)^T V': dk^, and c_i = e^{G_L - G_i} k^_i . dK~_i.
+        float dgp = 0.0f, cp = 0.0f;
+        {
+            const float* xp = xo + (chn * GC + i) * GD;
+            const float* kp = dkto + (chn * GC + i) * GD;
 #pragma unroll
             for (int m = 0; m < 4; ++m) {
-                const f32x4 a = op_row4(L.M1, MS, col, half, 0, m);
+                const f32x4 x = *(const f32x4*)(xp + 32 * m + 4 * s), y = *(const f32x4*)(kp + 32 * m + 4 * s);
+                dgp += dot4(row4<NQ, PC>(L.Q, i, 32 * m + 4 * s), x);
+                cp += dot4(row4<NQ, PC>(L.K, i, 32 * m + 4 * s), y);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const int r = 4 * m + e;
-                    const float ae = a[e] + op_col(L.M1, MS, half, 0, r, 0, col);
-                    dkm = mfma_f32(ae, op_col(L.Ks, RS, half, 0, r, cw0, col), dkm);
+                    dqa[4 * m + e] = fmaf(egi, x[e], dqa[4 * m + e]);
+                    dka[4 * m + e] = fmaf(ed, y[e], dka[4 * m + e]);
                 }
             }
-        } else {   // the correction's dk^ (its dv, dbeta are complete)
+            dgp = row8_sum(dgp) * (egi * L.fq[i]);
+            cp = row8_sum(cp) * (ed * L.fk[i]);
+        }
+        if constexpr (TRUNC) {   // the correction's dk^ (its dv, dbeta are complete)
             const float* kr = trk + (chn * GC + i) * GD;
 #pragma unroll
             for (int m = 0; m < 4; ++m) {
@@ -682,12 +706,193 @@ __global__ __launch_bounds__(GT) void gdn_bwd_chunk_kernel(GdnDev p, const TIn* 
                 for (int e = 0; e < 4; ++e) dka[4 * m + e] += x[e];
             }
         }
-        // M3 holds every pair term of dG (its last writers passed a barrier):
-        // its rows become exclusive prefix sums, M3[i][c] = sum_{j < c} p_ij
-        // (thread (i, s): four columns, a scan over the row's eight threads),
-        // for the dg sums below.
+        phase();
+        lds_barrier();   // dP complete, X's readers are done
+        if constexpr (!TRUNC) {
+            put16<PR>(L.X, i, 16 * s, xr);
+            fetch_x(dwo, chn);
+        } else if (hh + 1 < p.rep) {
+            fetch_x(chunk_vp, chn + 1);
+        }
+        phase();
+        // dq^ += dP k^, dk^ += dP^T q^ (contraction over the chunk's 32 tokens).
+#pragma unroll
+        for (int cb = 0; cb < 2; ++cb) {
+            phase();
+            const Op<NQ> kc = op_cols<NQ, PC>(L.K, w0 + 16 * cb, lane), qcv = op_cols<NQ, PC>(L.Q, w0 + 16 * cb, lane);
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb) {
+                add_alt(dqm[tb][cb], mul_planes(op_rows<3, AC>(L.P, 16 * tb + c16, 0, g4), kc, (f32x4){}));
+                add_alt(dkm[tb][cb], mul_planes(op_cols<3, AC>(L.P + 3 * GC * AC, 16 * tb, lane), qcv, (f32x4){}));
+            }
+        }
+        float dbp = 0.0f;
+        if constexpr (!TRUNC) {
+            TT_CHUNK_COORDS();
+            const Op<3> tt[2] = {op_fcols(L.T, 0, c16, g4, alt(c16)), op_fcols(L.T, 16, c16, g4, alt(c16))};   // T^T by rows
+            Op<NQ> vop[4];   // v rows of the quadrant's column tile
+            {
+                const TIn* row = (const TIn*)p.v + (int64_t)(start + 16 * qj + c16) * p.v_st + (int64_t)h * p.v_sh;
+#pragma unroll
+                for (int m = 0; m < 4; ++m) vop[m] = op_global<TIn>(row, 16 * qj + c16 < len, 32 * m, g4);
+            }
+            phase();
+            lds_barrier();   // dV' in X; dP's readers are done
+            // dT's part dV' v^T, and dBv = T^T dV': dv = beta dBv.
+            TIn* const dvh = dv + (int64_t)start * p.dv_st + h * GD + w0;   // uniform; 32-bit offsets of its rows
+            f32x4 tv = {};
+            if (lower) {
+                Sum2 x;
+#pragma unroll
+                for (int m = 0; m < 4; ++m) x.add(op_rows<3, PR>(L.X, 16 * qi + c16, 32 * m, g4), vop[m]);
+                tv = x.sum();
+            }
+#pragma unroll
+            for (int cb = 0; cb < 2; ++cb) {
+                phase();
+                const Op<3> x = op_cols<3, PR>(L.X, w0 + 16 * cb, lane);
+#pragma unroll
+                for (int tb = 0; tb < 2; ++tb) {
+                    const f32x4 o = mul_planes(tt[tb], x, (f32x4){});
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const int r = 16 * tb + g4 + v;
+                        const float x = v & 1 ? -o[v] : o[v];
+                        if (r < len) dvh[(unsigned)(r * p.dv_st + 16 * cb + c16)] = (TIn)(L.B[r] * x);
+                    }
+                }
+            }
+            phase();
+            lds_barrier();   // X's readers are done
+            put16<PR>(L.X, i, 16 * s, xr);
+            if (hh + 1 < p.rep) fetch_x(chunk_vp, chn + 1);
+            lds_barrier();
+            // dT's part dW k^^T, and dBk = T^T dW: dk^ += beta e^G dBk.
+            f32x4 tk = {};
+            if (lower) {
+                Sum2 x;
+#pragma unroll
+                for (int m = 0; m < 4; ++m)
+                    x.add(op_rows<3, PR>(L.X, 16 * qi + c16, 32 * m, g4),
+                          op_rows<NQ, PC>(L.K, 16 * qj + c16, 32 * m, g4));
+                tk = x.sum();
+            }
+#pragma unroll
+            for (int cb = 0; cb < 2; ++cb) {
+                phase();
+                const Op<3> x = op_cols<3, PR>(L.X, w0 + 16 * cb, lane);
+#pragma unroll
+                for (int tb = 0; tb < 2; ++tb) {
+                    const f32x4 o = mul_planes(tt[tb], x, (f32x4){});
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const int r = 16 * tb + g4 + v;
+                        dkm[tb][cb][v] = fmaf(L.Bg[r], v & 1 ? -o[v] : o[v], dkm[tb][cb][v]);
+                    }
+                }
+            }
+            phase();
+            // dbeta and dG take sum_c v_ic dBv_ic = sum_m T_mi (dV' v^T)_mi and
+            // the same of k^ and dW: column sums over the rows of T * (...).
+            {
+                float sv = 0.0f, sk = 0.0f;
+                f32x4 dt;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const float tm = L.T[(qr + v) * MS + qc], k1 = tk[v] * fkj;
+                    sv = fmaf(tm, tv[v], sv);
+                    sk = fmaf(tm, k1, sk);
+                    dt[v] = bj * fmaf(ej, k1, tv[v]);   // dT = dV' (beta v)^T + dW (beta e^G k^)^T
+                }
+                sv += __shfl_xor(sv, 16);
+                sk += __shfl_xor(sk, 16);
+                sv += __shfl_xor(sv, 32);
+                sk += __shfl_xor(sk, 32);
+                if (g4 == 0) {
+                    L.bv[qi][qc] = sv;
+                    L.bk[qi][qc] = sk;
+                }
+#pragma unroll
+                for (int v = 0; v < 4; ++v) L.M[(qr + v) * MS + qc] = dt[v];
+            }
+            lds_barrier();   // dT complete
+            phase();
+            // Y = T^T dT (only m' <= i is read)
+            if (lower) {
+                const f32x4 y = mul_planes(qi ? tt[1] : tt[0], op_fcols(L.M, 16 * qj, c16, g4, 1.0f), (f32x4){});
+#pragma unroll
+                for (int v = 0; v < 4; ++v) L.Y[(qr + v) * MS + qc] = v & 1 ? -y[v] : y[v];
+            }
+            {
+                const float vb = L.bv[0][i] + L.bv[1][i], kb = L.bk[0][i] + L.bk[1][i];
+                dbp = fmaf(egi, kb, vb);
+                dgp = fmaf(L.Bg[i], kb, dgp);
+            }
+            lds_barrier();   // Y complete, dT's readers are done
+            // dN = Y T^T (strictly lower): dbeta, dG and E = dL/d(k^ k^T) from
+            // N = -beta (k^ k^T) * D.
+            {
+                f32x4 dn = {};
+                if (lower) {
+                    const int yr = (16 * qi + c16) * MS + g4, tr = (16 * qj + c16) * MS + g4;
+                    // m' <= j: the second half of Y's and T's rows is not read for the upper column tile
+                    const f32x4 z = {};
+                    dn = mul_planes(op_acc(*(const f32x4*)&L.Y[yr], qi && qj ? *(const f32x4*)&L.Y[yr + 16] : z),
+                                    op_acc(*(const f32x4*)&L.T[tr], qj ? *(const f32x4*)&L.T[tr + 16] : z), (f32x4){});
+                }
+                f32x4 db;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int r = qr + v;
+                    const bool in = qc < r;
+                    const float dd = in ? expf(gdiff(L.G[r], L.Glo[r], L.G[qc], L.Glo[qc])) : 0.0f;
+                    const float x = in ? -dn[v] * dd : 0.0f;   // dN D
+                    db[v] = x * kk[v];
+                    pair[v] = fmaf(L.B[r], db[v], pair[v]);
+                    L.M[r * MS + qc] = x * L.B[r];
+                }
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const float r = sum16(db[v]);
+                    if (c16 == 0) L.db[qj][qr + v] = r;
+                }
+            }
+        }
+        phase();
         {
-            f32x4 v = *(const f32x4*)&L.M3[i * MS + 4 * s];
+            TT_CHUNK_COORDS();
+#pragma unroll
+            for (int v = 0; v < 4; ++v) L.S[(qr + v) * MS + qc] = pair[v];
+        }
+        if (s == 0) {
+            L.Grow[i] = dgp;
+            L.Crow[i] = cp;
+        }
+        lds_barrier();
+        if constexpr (!TRUNC) {
+            // dk^ += (E + E^T) k^
+            const f32x4 f0 = *(const f32x4*)(L.fk + g4) * alt(c16), f1 = *(const f32x4*)(L.fk + 16 + g4) * alt(c16);
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb) {
+                const int r = 16 * tb + c16;
+                f32x4 a = *(const f32x4*)&L.M[r * MS + g4], b = *(const f32x4*)&L.M[r * MS + 16 + g4];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    a[v] = (a[v] + L.M[(g4 + v) * MS + r]) * f0[v];
+                    b[v] = (b[v] + L.M[(16 + g4 + v) * MS + r]) * f1[v];
+                }
+                const Op<3> e = op_acc(a, b);
+#pragma unroll
+                for (int cb = 0; cb < 2; ++cb)
+                    add_alt(dkm[tb][cb], mul_planes(e, op_cols<NQ, PC>(L.K, w0 + 16 * cb, lane), (f32x4){}));
+            }
+            if (s == 0 && valid) dbeta[tok * p.hv + h] = dbp + (L.db[0][i] + L.db[1][i]);
+        }
+        // S holds every pair term of dG: its rows become exclusive prefix sums,
+        // S[i][c] = sum_{j < c} p_ij (thread (i, s): four columns, a scan over
+        // the row's eight threads), for the dg sums below.
+        {
+            f32x4 v = *(const f32x4*)&L.S[i * MS + 4 * s];
             const float tot = v[0] + v[1] + v[2] + v[3];
             float pre = __shfl_up(tot, 1, 8);
             if (s == 0) pre = 0.0f;
@@ -701,79 +906,52 @@ __global__ __launch_bounds__(GT) void gdn_bwd_chunk_kernel(GdnDev p, const TIn* 
             x[1] = pre + v[0];
             x[2] = x[1] + v[1];
             x[3] = x[2] + v[2];
-            *(f32x4*)&L.M3[i * MS + 4 * s] = x;
-        }
-        // The output state S_out = e^{G_L} S + (e^{G_L - G} k^)^T V': dk^ and dG.
-        {
-            const float* kr = dkto + chn * GC * GD + i * GD;
-            const float ed = expf(gdiff(gl, gll, gi, gil));
-            float kt = 0.0f;
-#pragma unroll
-            for (int m = 0; m < 4; ++m) {
-                const f32x4 x = *(const f32x4*)(kr + 32 * m + 4 * s);
-                const f32x4 kv = *(const f32x4*)&L.Ks[i * RS + 32 * m + 4 * s];
-                kt += dot4(kv, x);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) dka[4 * m + e] = fmaf(ed, x[e], dka[4 * m + e]);
-            }
-            cp = ed * kt;
-        }
-        dgp = row8_sum(dgp);
-        dbp = row8_sum(dbp);
-        cp = row8_sum(cp);
-        if (s == 0) {
-            L.Grow[i] = dgp;
-            L.Crow[i] = cp;
-            if (!TRUNC && valid) dbeta[tok * p.hv + h] = dbp;
+            *(f32x4*)&L.S[i * MS + 4 * s] = x;
         }
         // dg_t = sum of dG_u over u >= t within the chunk (G is its cumulative
-        // sum). A pair term p_ij (M3, i > j: the factors e^{G_i - G_j} of A and
+        // sum). A pair term p_ij (S, i > j: the factors e^{G_i - G_j} of A and
         // N) adds to dG_i and subtracts from dG_j, so it reaches dg_t exactly
         // when i >= t > j; a term c_i of the output state's e^{G_L - G_i}
         // (Crow) reaches it when i < t; e^{G_L} S's reaches every t. Summing
         // just those sets, rather than suffix sums of row minus column sums
         // in which the pairs inside [t, L] cancel only up to rounding, keeps
-        // dg accurate relative to its own size: dg_t = sum_{i >= t} M3[i][t]
-        // + sum_{i < t} c_i + the e^{G_L} term + the suffix sum of the terms
-        // of e^{G_i} alone.
-        __syncthreads();
-        if (t < GC) {
-            float cross = 0.0f, cpre = 0.0f;
-#pragma unroll 4
-            for (int r = 0; r < GC; ++r) {
-                cross += r >= t ? L.M3[r * MS + t] : 0.0f;
-                cpre += r < t ? L.Crow[r] : 0.0f;
-            }
-            float dG = L.Grow[t];
+        // dg accurate relative to its own size: dg_t = sum_{i >= t} (S[i][t] +
+        // the terms of e^{G_i} alone) + sum_{i < t} c_i + the e^{G_L} term.
+        // Token t's eight threads take rows s, s + 8, s + 16 and s + 24.
+        lds_barrier();
+        {
+            float x = 0.0f;
 #pragma unroll
-            for (int o = 1; o < GC; o <<= 1) {
-                const float up = __shfl_down(dG, o, GC);
-                if (t + o < GC) dG += up;
+            for (int e = 0; e < 4; ++e) {
+                const int r = s + 8 * e;
+                x += r >= i ? L.S[r * MS + i] + L.Grow[r] : L.Crow[r];
             }
-            dG += cross + cpre + expf(gl) * gsd;
-            if constexpr (TRUNC) dG += trg[chn * GC + t];
-            if (t < len) dg[(int64_t)(start + t) * p.hv + h] = dG;
+            x = row8_sum(x) + egl * gsd;
+            if constexpr (TRUNC) x += trg[chn * GC + i];
+            if (s == 0 && valid) dg[tok * p.hv + h] = x;
         }
     }
 
-    // The product terms join the element-wise ones (through P1, P2).
-    __syncthreads();
+#undef TT_CHUNK_COORDS
+    // The product terms join the element-wise ones through J, dq^ then dk^.
+    auto join = [&](const f32x4 (&m)[2][2], float (&a)[16]) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        L.P1[acc_row(r, half) * RS + cw0 + col] = dqm[r];
-        L.P2[acc_row(r, half) * RS + cw0 + col] = dkm[r];
-    }
-    __syncthreads();
+        for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        const f32x4 a = *(const f32x4*)&L.P1[i * RS + 32 * m + 4 * s];
-        const f32x4 b = *(const f32x4*)&L.P2[i * RS + 32 * m + 4 * s];
+            for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            dqa[4 * m + e] += a[e];
-            dka[4 * m + e] += b[e];
+                for (int v = 0; v < 4; ++v) L.J[(16 * tb + g4 + v) * RS + w0 + 16 * cb + c16] = m[tb][cb][v];
+        lds_barrier();
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            const f32x4 x = *(const f32x4*)&L.J[i * RS + 32 * n + 4 * s];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a[4 * n + e] += x[e];
         }
-    }
+        lds_barrier();
+    };
+    join(dqm, dqa);
+    join(dkm, dka);
 
     // Through q^ = scale q / sqrt(|q|^2 + eps) and k^ = k / sqrt(|k|^2 + eps).
     if (valid) {

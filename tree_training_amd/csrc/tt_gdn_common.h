@@ -32,11 +32,6 @@ __device__ __forceinline__ float gdiff(float hi_i, float lo_i, float hi_j, float
     return (hi_i - hi_j) + (lo_i - lo_j);
 }
 
-template <int I>
-struct IntC4 {
-    static constexpr int value = I;
-};
-
 template <typename T>
 __device__ __forceinline__ void load16(const T* p, float (&x)[16]) {
     if constexpr (sizeof(T) == 2) {
@@ -132,17 +127,8 @@ __device__ __forceinline__ f32x16 mfma_f32(float a, float b, const f32x16& c) {
     return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
 
-// v_mfma_f32_16x16x4_f32: D[16x16] += A[16x4] B[4x16]; lane l supplies
-// A[l & 15][l >> 4] and B[l >> 4][l & 15], and accumulator element v of lane
-// l is D[4 (l >> 4) + v][l & 15]. Step v of a 16-deep contraction pairs
-// k = 4 (l >> 4) + v across the four lane groups, so a 16-row block held as
-// accumulators is directly the B operand, element v of each lane.
-__device__ __forceinline__ f32x4 mfma16_f32(float a, float b, const f32x4& c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
 // A 16 x 16 tile of a row-major fp32 matrix of GD-float rows in the layout
-// of mfma16_f32's accumulators: element v of lane l is row 4 (l >> 4) + v,
+// of a 16 x 16 MFMA's accumulators: element v of lane l is row 4 (l >> 4) + v,
 // column l & 15, of the tile at `base`.
 __device__ __forceinline__ f32x4 load_t16(const float* base, int lane) {
     const float* p = base + 4 * (lane >> 4) * GD + (lane & 15);
@@ -172,27 +158,11 @@ __device__ __forceinline__ AccMat acc_mat(const float* base, int rows, int half,
     return m;
 }
 template <int ROW0>
-__device__ __forceinline__ f32x16 load_acc(const AccMat& m) {
-    f32x16 v;
-#pragma unroll
-    for (int r = 0; r < 16; ++r)
-        v[r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(m.rs, m.vo[r & 3], (ROW0 + 8 * (r >> 2)) * GD * 4, 0));
-    return v;
-}
-template <int ROW0>
 __device__ __forceinline__ void store_acc(const AccMat& m, const f32x16& v) {
 #pragma unroll
     for (int r = 0; r < 16; ++r)
         __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[r]), m.rs, m.vo[r & 3], (ROW0 + 8 * (r >> 2)) * GD * 4, 0);
 }
-template <typename F>
-__device__ __forceinline__ void for_tiles(F&& f) {
-    f(IntC4<0>{});
-    f(IntC4<1>{});
-    f(IntC4<2>{});
-    f(IntC4<3>{});
-}
-
 template <typename T>
 __device__ __forceinline__ f32x4 load4(const T* p) {
     if constexpr (sizeof(T) == 2) {
@@ -228,10 +198,6 @@ __device__ __forceinline__ void tile_in(const T* base, int64_t row_stride, int l
 // Row operand X[col][kb + k]: four steps per 16-byte read.
 __device__ __forceinline__ f32x4 op_row4(const float* X, int stride, int col, int half, int kb, int m) {
     return *(const f32x4*)&X[col * stride + kb + 8 * m + 4 * half];
-}
-// Column operand X[kb + k][c0 + col], one step.
-__device__ __forceinline__ float op_col(const float* X, int stride, int half, int kb, int r, int c0, int col) {
-    return X[(kb + acc_row(r, half)) * stride + c0 + col];
 }
 // 32 x 32 partial product over this wave's quarter of a 128-deep contraction:
 // D[i][j] = sum_k A[i][k] B[j][k] (both read as rows), B scaled by bs (a

@@ -15,71 +15,9 @@
 // U, V' and dV'.
 #pragma once
 
-#include "tt_gdn_common.h"
-#include "tt_planes.h"
+#include "tt_gdn_planes.h"
 
 namespace {
-
-// bf16 planes of a chunk's tiles in LDS, rows = tokens. A tile read by rows
-// (16 rows x 16 bytes a pass) has rows of 272 bytes (A: 80), one read by
-// columns through the transposing read (8 rows x 32 bytes) rows of 288 (96):
-// both reach every bank once a pass.
-constexpr int PR = GD + 8, PC = GD + 16;   // [token][state row] tiles
-constexpr int AR = GC + 8, AC = GC + 16;   // [token][token]
-template <typename TIn>
-constexpr int kInPlanes = sizeof(TIn) == 2 ? 1 : 3;
-
-__device__ __forceinline__ f32x4 mfma16b(const bf16x8& a, const bf16x8& b, const f32x4& c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-// An operand of N planes (h, m, l).
-template <int N>
-struct Op {
-    bf16x8 p[N];
-};
-// acc + A B, the smallest terms first.
-template <int NA, int NB>
-__device__ __forceinline__ f32x4 mul_planes(const Op<NA>& a, const Op<NB>& b, f32x4 acc) {
-    if constexpr (NA == 3) acc = mfma16b(a.p[2], b.p[0], acc);
-    if constexpr (NB == 3) acc = mfma16b(a.p[0], b.p[2], acc);
-    if constexpr (NA == 3 && NB == 3) acc = mfma16b(a.p[1], b.p[1], acc);
-    if constexpr (NA == 3) acc = mfma16b(a.p[1], b.p[0], acc);
-    if constexpr (NB == 3) acc = mfma16b(a.p[0], b.p[1], acc);
-    return mfma16b(a.p[0], b.p[0], acc);
-}
-// Two 16-row accumulator tiles (rows 4 (l >> 4) + v) as the operand of a
-// 32-deep contraction: element e of lane l is row 4 (l >> 4) + (e & 3) of tile
-// e / 4, the k order of every operand here.
-__device__ __forceinline__ Op<3> op_acc(const f32x4& t0, const f32x4& t1) {
-    Split8 w = split_begin(t0, t1);
-    w.all();
-    const Planes q = w.planes();
-    return {{q.h, q.m, q.l}};
-}
-// Row operand X[row][k0 + k] of a tile with rows of P elements (N planes, each
-// [GC][P]), g4 = 4 (l >> 4).
-template <int N, int P>
-__device__ __forceinline__ Op<N> op_rows(const __bf16* X, int row, int k0, int g4) {
-    Op<N> o;
-#pragma unroll
-    for (int n = 0; n < N; ++n) {
-        const __bf16* x = X + n * GC * P + row * P + k0 + g4;
-        o.p[n] = cat44(*(const bf16x4*)x, *(const bf16x4*)(x + 16));
-    }
-    return o;
-}
-// Column operand X[k][c0 + (l & 15)], k over the tile's 32 tokens.
-template <int N, int P>
-__device__ __forceinline__ Op<N> op_cols(const __bf16* X, int c0, int lane) {
-    const int j = lane & 15;
-    Op<N> o;
-#pragma unroll
-    for (int n = 0; n < N; ++n) {
-        const __bf16* x = X + n * GC * P + (4 * (lane >> 4) + (j >> 2)) * P + c0 + 4 * (j & 3);
-        o.p[n] = cat44(ds_read_tr(x), ds_read_tr(x + 16 * P));
-    }
-    return o;
-}
 
 // A chunk's scan inputs, held in registers one chunk ahead of their use (the
 // loads of the next chunk are in flight while a chunk computes): this
@@ -133,43 +71,22 @@ __device__ __forceinline__ void scan_fetch_rows(const GdnDev& p, const float* cw
     x.gll = cw[kWsGlo + GC - 1];
 }
 
-// 16 consecutive elements of row i at column d0 as planes of a tile with rows of P elements.
-template <int P>
-__device__ __forceinline__ void put16(__bf16* X, int i, int d0, const bf16x8 (&x)[2]) {
-    *(bf16x8*)(X + i * P + d0) = x[0];
-    *(bf16x8*)(X + i * P + d0 + 8) = x[1];
+// x times alt(i) (bf16 values: the sign bits).
+__device__ __forceinline__ void alt_row(bf16x8 (&x)[2], int i) {
+    const unsigned m = i & 1 ? 0x80008000u : 0u;
+#pragma unroll
+    for (int n = 0; n < 2; ++n) x[n] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, x[n]) ^ (u32x4){m, m, m, m});
 }
-template <int P>
-__device__ __forceinline__ void put16(__bf16* X, int i, int d0, const f32x4 (&x)[4]) {
+__device__ __forceinline__ void alt_row(f32x4 (&x)[4], int i) {
 #pragma unroll
-    for (int n = 0; n < 2; ++n) {
-        Split8 w = split_begin(x[2 * n], x[2 * n + 1]);
-        w.all();
-        const Planes q = w.planes();
-        __bf16* d = X + i * P + d0 + 8 * n;
-        *(bf16x8*)d = q.h;
-        *(bf16x8*)(d + GC * P) = q.m;
-        *(bf16x8*)(d + 2 * GC * P) = q.l;
-    }
-}
-// 1 / sqrt(|row|^2 + eps) (1 without the l2 norm) of the row whose 128
-// elements this thread and its seven neighbours hold.
-template <int NV, typename Vec>
-__device__ __forceinline__ float row_norm(const GdnDev& p, const Vec (&x)[NV]) {
-    constexpr int EV = 16 / NV;
-    float s = 0.0f;
-#pragma unroll
-    for (int n = 0; n < NV; ++n)
-#pragma unroll
-        for (int e = 0; e < EV; ++e) s = fmaf((float)x[n][e], (float)x[n][e], s);
-    s = row8_sum(s);
-    return p.l2 ? 1.0f / sqrtf(s + 1e-6f) : 1.0f;
+    for (int n = 0; n < 4; ++n) x[n] *= alt(i);
 }
 
 // A fetched chunk in LDS: q, k, W (with STORE_W) and A as planes with rows of
 // PQ, PK, PW and PA elements, and the per-token factors fq = scale e^{G_i} /
-// |q_i| and fk = e^{G_L - G_i} / |k_i|.
-template <typename TIn, int PQ, int PK, int PW, int PA>
+// |q_i| and fk = e^{G_L - G_i} / |k_i|. ALT (the reverse scan): rows i of k and
+// columns i of A times alt(i), so that dV' comes out times alt of its token.
+template <typename TIn, int PQ, int PK, int PW, int PA, bool ALT>
 struct ScanTiles {
     static constexpr int NQ = kInPlanes<TIn>;
     __bf16 Q[NQ * GC * PQ];
@@ -182,10 +99,18 @@ struct ScanTiles {
     __device__ __forceinline__ void stage(const GdnDev& p, const ScanAhead<TIn>& x) {
         const int t = threadIdx.x, i = t >> 3, d0 = 16 * (t & 7);
         put16<PQ>(Q, i, d0, x.q);
-        put16<PK>(K, i, d0, x.k);
+        if constexpr (ALT) {
+            typename ScanAhead<TIn>::Vec k[ScanAhead<TIn>::NV];
+#pragma unroll
+            for (int n = 0; n < ScanAhead<TIn>::NV; ++n) k[n] = x.k[n];
+            alt_row(k, i);
+            put16<PK>(K, i, d0, k);
+        } else {
+            put16<PK>(K, i, d0, x.k);
+        }
         if constexpr (STORE_W) put16<PW>(W, i, d0, x.w);
         {
-            float a0 = x.a[0], a1 = x.a[1], a2 = x.a[2], a3 = x.a[3];
+            float a0 = x.a[0], a1 = ALT ? -x.a[1] : x.a[1], a2 = x.a[2], a3 = ALT ? -x.a[3] : x.a[3];
             __bf16* d = A + i * PA + 4 * (t & 7);
 #pragma unroll
             for (int n = 0; n < 3; ++n) {
@@ -204,9 +129,9 @@ struct ScanTiles {
     }
 };
 template <typename TIn>
-using FwdTiles = ScanTiles<TIn, PR, PC, PR, AR>;   // q, W and A by rows, k by columns
+using FwdTiles = ScanTiles<TIn, PR, PC, PR, AR, false>;   // q, W and A by rows, k by columns
 template <typename TIn>
-using RevTiles = ScanTiles<TIn, PC, PR, PC, AC>;   // k by rows, q, W and A by columns
+using RevTiles = ScanTiles<TIn, PC, PR, PC, AC, true>;   // k by rows, q, W and A by columns
 
 // S e + x: the products of an update are summed apart and join the state with
 // one rounding.
@@ -577,15 +502,6 @@ __device__ __forceinline__ void rscan_fetch(const GdnDev& p, const ScanNode& nd,
             x.x[tb][v] = i < Lc ? (float)base[(int64_t)i * do_st] : 0.0f;
         }
 }
-// dO as an operand: its bf16 values as they are, or three planes.
-template <typename TIn>
-__device__ __forceinline__ Op<kInPlanes<TIn>> op_in(const f32x4& t0, const f32x4& t1) {
-    if constexpr (kInPlanes<TIn> == 1)
-        return {{pack8(t0[0], t0[1], t0[2], t0[3], t1[0], t1[1], t1[2], t1[3])}};
-    else
-        return op_acc(t0, t1);
-}
-
 // Column layout as gdn_scan_cols_kernel (scan_block). Wave w owns value
 // columns c0 + 16w .. +15: its 128 x 16 slice of dS lives in eight 16 x 16
 // accumulator tiles, dO of the chunk is loaded in accumulator layout (rows =
@@ -640,7 +556,7 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
                 f32x4 pd = scale_tok(
                     mul_planes(op_rows<NQ, PR>(L.K, 16 * tb + c16, 32 * w4, g4), sp, (f32x4){}), L.fk, 16 * tb + g4);
                 if (tb == w4) pd = mul_planes(op_cols<3, AC>(L.A, 16 * tb, lane), dop, pd);
-                dv[tb] += pd;
+                add_alt(dv[tb], pd);
             }
         }
 #pragma unroll
@@ -736,7 +652,7 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 #pragma unroll
         for (int tb = 0; tb < 2; ++tb) {
 #pragma unroll
-            for (int w = 0; w < 4; ++w) dv[tb] += L.P[w][tb][lane];
+            for (int w = 0; w < 4; ++w) add_alt(dv[tb], L.P[w][tb][lane]);
         }
         if (wave == 0) {
 #pragma unroll
