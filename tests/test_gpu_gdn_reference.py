@@ -165,6 +165,25 @@ def test_reference_mode_saved_forward_equals_recompute(dtype):
         assert torch.equal(a, b), name
 
 
+@pytest.mark.parametrize("Hk,Hv", [(1, 2), (16, 32)])
+def test_reference_mode_block_edges(Hk, Hv):
+    """Nodes of 1, 31, 32, 33, 64, 65 and 97 tokens on one level (and a root of
+    33): whole, ragged and single-token correction blocks, in the row layout of
+    the level scans (14 pairs) and the column layout (224 pairs): fp32 outputs,
+    states and gradients against the float64 oracle, at the fp32 bar."""
+    lens, par = [33, 1, 31, 32, 33, 64, 65, 97], [-1] + [0] * 7
+    T = sum(lens)
+    q, k, v, g, beta = _inputs(T, Hk, Hv, 43 + Hv, realistic_gates=True)
+    d_o = np.random.default_rng(14).standard_normal((T, Hv, D)).astype(np.float32)
+    print(f"gdn reference block edges: T={T} heads {Hk}/{Hv}", flush=True)
+    o, st = _run(q, k, v, g, beta, lens, par, torch.float32)
+    o_ref, st_ref = ogdn.gdn_tree(q, k, v, g, beta, lens, par, mode="reference")
+    assert _rel(o, o_ref) < 1e-5 and _rel(st, st_ref) < 1e-5
+    got = _run_bwd(q, k, v, g, beta, d_o, lens, par, torch.float32)
+    for name, a, b in zip(BWD_NAMES, got, _oracle_grads(q, k, v, g, beta, d_o, lens, par)):
+        assert _rel(a, b) < 1e-5, (name, _rel(a, b))
+
+
 def test_reference_mode_agent16k_two_heads_matches_oracle():
     """Full c5 topology (agent tree, 16,318 tokens, 54 nodes of 64-512 tokens,
     realistic gates), fp32, one q/k head shared by two v heads, against the

@@ -475,18 +475,6 @@ __device__ __forceinline__ f32x4 row4(const __bf16* X, int i, int c0) {
     }
     return r;
 }
-// A row of the problem dtype as an operand: columns k0 + g4 .. +3 and
-// k0 + 16 + g4 .. +3 (zeros when the row does not exist).
-template <typename TIn>
-__device__ __forceinline__ Op<kInPlanes<TIn>> op_global(const TIn* row, bool in, int k0, int g4) {
-    if constexpr (kInPlanes<TIn> == 1) {
-        const bf16x4 z = {};
-        return {{cat44(in ? *(const bf16x4*)(row + k0 + g4) : z, in ? *(const bf16x4*)(row + k0 + 16 + g4) : z)}};
-    } else {
-        const f32x4 z = {};
-        return op_acc(in ? load4(row + k0 + g4) : z, in ? load4(row + k0 + 16 + g4) : z);
-    }
-}
 // Column operand f X[k][c0 + c16] of a [GC][MS] fp32 matrix, k over its 32 rows.
 __device__ __forceinline__ Op<3> op_fcols(const float* X, int c0, int c16, int g4, float f) {
     f32x4 a, b;
@@ -497,28 +485,9 @@ __device__ __forceinline__ Op<3> op_fcols(const float* X, int c0, int c16, int g
     }
     return op_acc(a, b);
 }
-// A [32 x 32] accumulator quadrant into planes with rows of AC elements.
-__device__ __forceinline__ void put_quadrant(__bf16* X, int row, int colj, const f32x4& x) {
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        float r = x[v];
-#pragma unroll
-        for (int n = 0; n < 3; ++n) {
-            const __bf16 b = (__bf16)r;
-            X[n * GC * AC + (row + v) * AC + colj] = b;
-            r -= (float)b;
-        }
-    }
-}
 // The compiler moves no work across: overlapped, the phases of a head do not
 // fit the registers.
 __device__ __forceinline__ void phase() { __builtin_amdgcn_sched_barrier(0); }
-__device__ __forceinline__ float sum16(float x) {   // over the 16 lanes of a row of accumulators
-    x += __shfl_xor(x, 1);
-    x += __shfl_xor(x, 2);
-    x += __shfl_xor(x, 4);
-    return x + __shfl_xor(x, 8);
-}
 
 // Products by tiles of v_mfma_f32_16x16x32_bf16 on planes: a [32 x 32] result
 // is a quadrant a wave (the upper one holds nothing that is read and is left
@@ -673,8 +642,8 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(sizeof(TIn) 
                 pk[v] = v & 1 ? -(dpv * fkj) : dpv * fkj;   // rows i of dP: alt(i)
                 pq[v] = dpv * (L.fq[r] * alt(c16));         // rows j of dP^T: alt(j)
             }
-            put_quadrant(L.P, qr, qc, pk);
-            put_quadrant(L.P + 3 * GC * AC, qr, qc, pq);
+            put_quadrant<AC>(L.P, qr, qc, pk);
+            put_quadrant<AC>(L.P + 3 * GC * AC, qr, qc, pq);
         }
         phase();
         // O's state term e^G q^ S: dq^ += e^G X, dG += e^G q^ . X; the output
@@ -1000,8 +969,8 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(sizeof(TIn) 
 }  // namespace
 
 // Float counts per (chunk, v head) of the truncated mode's node-level terms:
-// the node-level decay [32] and R (beta [v | e^G k]) rows [32 x 256].
-constexpr size_t kTrGn = GC, kTrY1 = (size_t)GC * 2 * GD;
+// the node-level decay and 1 / |k| [32] each, and R (beta [v | e^G k]) rows [32 x 256].
+constexpr size_t kTrGn = 2 * GC, kTrY1 = (size_t)GC * 2 * GD;
 
 size_t tt_gdn_ws_bytes_impl(int n_chunks, int n_heads_v, bool trunc) {
     return (size_t)n_chunks * (size_t)n_heads_v * (kWsChunk + (trunc ? kTrGn + kTrY1 : 0)) * sizeof(float);
@@ -1015,18 +984,16 @@ template <typename TIn, bool TRUNC>
 void launch_prep(const GdnDev& d, float* prep, hipStream_t s) {
     hipLaunchKernelGGL((gdn_prep_kernel<TIn, TRUNC>), dim3(d.n_chunks, d.hv), dim3(GT), 0, s, d, prep);
 }
-// A level of n nodes runs in the row layout (exact rule) when the column
+// A level of n nodes runs in the row layout when the column
 // layout would leave most of the chip idle: at most TT_GDN_ROWS_MAX_PAIRS
 // (node, v head) pairs, two column workgroups each. On the 16K agent tree (32
 // v heads) 64 pairs (levels of one or two nodes) timed best: 5.60 -> 5.40 ms
-// per step, against 5.43 ms for 128 and for 256.
+// per step, against 5.43 ms for 128 and for 256. The truncated rule on a
+// 4,096-token tree (16 v heads): scans of both directions 863 -> 710 us with it.
 #ifndef TT_GDN_ROWS_MAX_PAIRS
 #define TT_GDN_ROWS_MAX_PAIRS 64
 #endif
-template <bool TRUNC>
-bool use_rows(const GdnDev& d, int n) {
-    return !TRUNC && (int64_t)n * d.hv <= TT_GDN_ROWS_MAX_PAIRS;
-}
+bool use_rows(const GdnDev& d, int n) { return (int64_t)n * d.hv <= TT_GDN_ROWS_MAX_PAIRS; }
 
 template <typename TIn, bool TRUNC>
 void launch_scan(const GdnDev& d, int b, int n, float* prep, TIn* out, float* states, float* sin, float* vp,
@@ -1034,8 +1001,8 @@ void launch_scan(const GdnDev& d, int b, int n, float* prep, TIn* out, float* st
     // grid (v head x column block, node): all heads of a level's first
     // (longest) nodes are dispatched first
     for (int b0 = 0; b0 < n; b0 += kMaxGridY) {
-        if (use_rows<TRUNC>(d, n))
-            hipLaunchKernelGGL((gdn_scan_rows_kernel<TIn>), dim3(d.hv * kRowsSplit, min(kMaxGridY, n - b0)),
+        if (use_rows(d, n))
+            hipLaunchKernelGGL((gdn_scan_rows_kernel<TIn, TRUNC>), dim3(d.hv * kRowsSplit, min(kMaxGridY, n - b0)),
                                dim3(GT), 0, s, d, b + b0, prep, out, states, sin, vp);
         else
             hipLaunchKernelGGL((gdn_scan_cols_kernel<TIn, TRUNC>), dim3(d.hv * kScanSplit, min(kMaxGridY, n - b0)),
@@ -1084,7 +1051,7 @@ int tt_gdn_fwd_launch(const GdnDev& d, const int32_t* level_offsets, int n_level
 
 // The backward's float buffers. "Saved" (what the forward can keep for it):
 // per (chunk, v head) the prep terms [kWsChunk], the chunk's initial state S
-// [128 x 128] and V' [32 x 128]; TRUNC: also the node-level decay [32] and
+// [128 x 128] and V' [32 x 128]; TRUNC: also the node-level decay and 1 / |k| [32] each and
 // R-rows y1 [32 x 256]. Scratch: per (chunk, v head) dS [128 x 128], dV', X,
 // dW, dK~ [32 x 128]; TRUNC: dF1, dY0 [32 x 256], the correction's dk^
 // [32 x 128] and dG [32]; per (node, v head) dS at entry [128 x 128]; when the
@@ -1172,8 +1139,8 @@ static int gdn_bwd_run(const GdnDev& d, const int32_t* level_offsets, int n_leve
         const int b = level_offsets[l], n = level_offsets[l + 1] - b;
         if (n <= 0) continue;
         for (int b0 = 0; b0 < n; b0 += kMaxGridY) {
-            if (use_rows<TRUNC>(d, n))
-                hipLaunchKernelGGL((gdn_rscan_rows_kernel<TIn>), dim3(d.hv * kRowsSplit, min(kMaxGridY, n - b0)),
+            if (use_rows(d, n))
+                hipLaunchKernelGGL((gdn_rscan_rows_kernel<TIn, TRUNC>), dim3(d.hv * kRowsSplit, min(kMaxGridY, n - b0)),
                                    dim3(GT), 0, s, d, b + b0, w.prep, d_o, do_st, do_sh, w.dso, w.dvp, w.dsn);
             else
                 hipLaunchKernelGGL((gdn_rscan_cols_kernel<TIn, TRUNC>),

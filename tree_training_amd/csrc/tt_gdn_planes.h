@@ -140,4 +140,37 @@ __device__ __forceinline__ Op<kInPlanes<TIn>> op_in(const f32x4& t0, const f32x4
         return op_acc(t0, t1);
 }
 
+// A row of the problem dtype as an operand: columns k0 + g4 .. +3 and
+// k0 + 16 + g4 .. +3 (zeros when the row does not exist).
+template <typename TIn>
+__device__ __forceinline__ Op<kInPlanes<TIn>> op_global(const TIn* row, bool in, int k0, int g4) {
+    if constexpr (kInPlanes<TIn> == 1) {
+        const bf16x4 z = {};
+        return {{cat44(in ? *(const bf16x4*)(row + k0 + g4) : z, in ? *(const bf16x4*)(row + k0 + 16 + g4) : z)}};
+    } else {
+        const f32x4 z = {};
+        return op_acc(in ? load4(row + k0 + g4) : z, in ? load4(row + k0 + 16 + g4) : z);
+    }
+}
+// A [32 x 32] accumulator quadrant into planes with rows of P elements.
+template <int P>
+__device__ __forceinline__ void put_quadrant(__bf16* X, int row, int colj, const f32x4& x) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        float r = x[v];
+#pragma unroll
+        for (int n = 0; n < 3; ++n) {
+            const __bf16 b = (__bf16)r;
+            X[n * GC * P + (row + v) * P + colj] = b;
+            r -= (float)b;
+        }
+    }
+}
+__device__ __forceinline__ float sum16(float x) {   // over the 16 lanes of a row of accumulators
+    x += __shfl_xor(x, 1);
+    x += __shfl_xor(x, 2);
+    x += __shfl_xor(x, 4);
+    return x + __shfl_xor(x, 8);
+}
+
 }  // namespace

@@ -37,8 +37,8 @@ struct ScanAhead {
 };
 
 // Loads the parts of chunk (start, len) that do not depend on the state: q/k
-// rows, W rows (with LOAD_W), A and the decays from its workspace slot cw.
-template <typename TIn, bool LOAD_W>
+// rows, W rows, A and the decays from its workspace slot cw.
+template <typename TIn>
 __device__ __forceinline__ void scan_fetch_rows(const GdnDev& p, const float* cw, int start, int len, int h,
                                                 ScanAhead<TIn>& x) {
     using Vec = typename ScanAhead<TIn>::Vec;
@@ -60,10 +60,8 @@ __device__ __forceinline__ void scan_fetch_rows(const GdnDev& p, const float* cw
             for (int e = 0; e < EV; ++e) x.q[n][e] = x.k[n][e] = (TIn)0.0f;
         }
     }
-    if constexpr (LOAD_W) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) x.w[e] = *(const f32x4*)(cw + kWsW + i * GD + d0 + 4 * e);
-    }
+    for (int e = 0; e < 4; ++e) x.w[e] = *(const f32x4*)(cw + kWsW + i * GD + d0 + 4 * e);
     x.a = *(const f32x4*)(cw + kWsA + i * GC + 4 * (t & 7));
     x.gi = cw[kWsG + i];
     x.gl = cw[kWsG + GC - 1];
@@ -82,7 +80,7 @@ __device__ __forceinline__ void alt_row(f32x4 (&x)[4], int i) {
     for (int n = 0; n < 4; ++n) x[n] *= alt(i);
 }
 
-// A fetched chunk in LDS: q, k, W (with STORE_W) and A as planes with rows of
+// A fetched chunk in LDS: q, k, W and A as planes with rows of
 // PQ, PK, PW and PA elements, and the per-token factors fq = scale e^{G_i} /
 // |q_i| and fk = e^{G_L - G_i} / |k_i|. ALT (the reverse scan): rows i of k and
 // columns i of A times alt(i), so that dV' comes out times alt of its token.
@@ -95,7 +93,6 @@ struct ScanTiles {
     __bf16 A[3 * GC * PA];
     float fq[GC], fk[GC];
     float el;   // e^{G_L}
-    template <bool STORE_W>
     __device__ __forceinline__ void stage(const GdnDev& p, const ScanAhead<TIn>& x) {
         const int t = threadIdx.x, i = t >> 3, d0 = 16 * (t & 7);
         put16<PQ>(Q, i, d0, x.q);
@@ -108,7 +105,7 @@ struct ScanTiles {
         } else {
             put16<PK>(K, i, d0, x.k);
         }
-        if constexpr (STORE_W) put16<PW>(W, i, d0, x.w);
+        put16<PW>(W, i, d0, x.w);
         {
             float a0 = x.a[0], a1 = ALT ? -x.a[1] : x.a[1], a2 = x.a[2], a3 = ALT ? -x.a[3] : x.a[3];
             __bf16* d = A + i * PA + 4 * (t & 7);
@@ -215,9 +212,7 @@ struct ScanNode {
 // given, receive each chunk's initial state and V' ([n_chunks, Hv, 128, 128]
 // and [n_chunks, Hv, 32, 128] floats).
 // TRUNC (the reference's per-node correction): V' = U - W S0 with S0 the
-// node's initial state for every chunk of the node. A first pass over the
-// node's chunks, while the state registers still hold S0, replaces each
-// chunk's U by its V' in the workspace; the scan proper then reads V' there.
+// node's initial state, whose planes stay in registers, for every chunk.
 template <typename TIn, bool TRUNC>
 __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn_scan_cols_kernel(GdnDev p, int lvl_begin, float* __restrict__ ws,
                                                       TIn* __restrict__ out, float* __restrict__ states,
@@ -241,39 +236,17 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
         for (int rb = 0; rb < 8; ++rb) S[rb] = (f32x4){};
     }
 
+    Op<3> s0p[4];   // TRUNC
     if constexpr (TRUNC) {
-        // V' = U - W S0 for every chunk (with S0 zero: V' = U as it is).
-        Op<3> s0p[4];
 #pragma unroll
         for (int w4 = 0; w4 < 4; ++w4) s0p[w4] = op_acc(S[2 * w4], S[2 * w4 + 1]);
-        for (int c0 = 0; s0 && c0 < len; c0 += GC) {
-            float* cw = ws + ((size_t)(chunk0 + c0 / GC) * p.hv + h) * kWsChunk;
-            f32x4 w[4], vp[2];
-            const int i = t >> 3, d0 = 16 * (t & 7);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) w[e] = *(const f32x4*)(cw + kWsW + i * GD + d0 + 4 * e);
-#pragma unroll
-            for (int tb = 0; tb < 2; ++tb) vp[tb] = load_t16(cw + kWsU + 16 * tb * GD + jt, lane);
-            lds_barrier();   // readers of the previous chunk's W are done
-            put16<PR>(L.W, i, d0, w);
-            lds_barrier();
-#pragma unroll
-            for (int tb = 0; tb < 2; ++tb) {
-                f32x4 pv = {};
-#pragma unroll
-                for (int w4 = 0; w4 < 4; ++w4)
-                    pv = mul_planes(op_rows<3, PR>(L.W, 16 * tb + c16, 32 * w4, g4), s0p[w4], pv);
-                store_t16(cw + kWsU + 16 * tb * GD + jt, lane, vp[tb] - pv);   // read back by this lane
-            }
-        }
     }
 
-    // U (TRUNC: V', written by the first pass) and the state-independent
-    // chunk terms, one chunk ahead.
+    // U and the state-independent chunk terms, one chunk ahead.
     ScanAhead<TIn> nx;
     auto fetch = [&](int ci) {
         const float* cw = ws + ((size_t)(chunk0 + ci) * p.hv + h) * kWsChunk;
-        scan_fetch_rows<TIn, !TRUNC>(p, cw, start + GC * ci, min(GC, len - GC * ci), h, nx);
+        scan_fetch_rows<TIn>(p, cw, start + GC * ci, min(GC, len - GC * ci), h, nx);
 #pragma unroll
         for (int tb = 0; tb < 2; ++tb) nx.x[tb] = load_t16(cw + kWsU + 16 * tb * GD + jt, lane);
     };
@@ -287,7 +260,7 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
             for (int rb = 0; rb < 8; ++rb) store_t16(sp + 16 * rb * GD, lane, S[rb]);
         }
         lds_barrier();   // readers of the previous chunk's tiles are done
-        L.template stage<!TRUNC>(p, nx);
+        L.stage(p, nx);
         f32x4 vp[2] = {nx.x[0], nx.x[1]}, qs[2] = {};
         if (ci + 1 < n_ch) fetch(ci + 1);
         lds_barrier();
@@ -300,8 +273,7 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
             const Op<3> sp = op_acc(S[2 * w4], S[2 * w4 + 1]);
 #pragma unroll
             for (int tb = 0; tb < 2; ++tb) {
-                if constexpr (!TRUNC)
-                    vp[tb] -= mul_planes(op_rows<3, PR>(L.W, 16 * tb + c16, 32 * w4, g4), sp, (f32x4){});
+                vp[tb] -= mul_planes(op_rows<3, PR>(L.W, 16 * tb + c16, 32 * w4, g4), TRUNC ? s0p[w4] : sp, (f32x4){});
                 qs[tb] += mul_planes(op_rows<NQ, PR>(L.Q, 16 * tb + c16, 32 * w4, g4), sp, (f32x4){});
             }
         }
@@ -339,8 +311,7 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     for (int rb = 0; rb < 8; ++rb) store_t16(sp + 16 * rb * GD, lane, S[rb]);
 }
 
-// Row layout of the level scans, for levels of few nodes (the exact rule
-// only): a workgroup takes 16 value columns of one (node, v head), eight
+// Row layout of the level scans, for levels of few nodes: a workgroup takes 16 value columns of one (node, v head), eight
 // workgroups per pair, and its wave w the state rows 32w .. 32w+31 of them.
 // The products over the state rows (W S and q^ S) are summed over the four
 // waves through LDS, in wave order; every wave then updates its own rows. A
@@ -368,9 +339,9 @@ struct ScanRowsLds {
     f32x4 P[4][2][2][64];   // per wave: its partial W S and q S, both token tiles, lane-major
 };
 
-// As gdn_scan_cols_kernel (exact rule), in the row layout: wave w holds the
-// 32 x 16 slice S[32w .., c0 ..] in two 16 x 16 accumulator tiles.
-template <typename TIn>
+// As gdn_scan_cols_kernel, in the row layout: wave w holds the 32 x 16 slice
+// S[32w .., c0 ..] in two 16 x 16 accumulator tiles.
+template <typename TIn, bool TRUNC>
 __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn_scan_rows_kernel(GdnDev p, int lvl_begin, float* __restrict__ ws,
                                                       TIn* __restrict__ out, float* __restrict__ states,
                                                       float* __restrict__ chunk_sin, float* __restrict__ chunk_vp) {
@@ -388,11 +359,12 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     f32x4 S[2];
 #pragma unroll
     for (int r = 0; r < 2; ++r) S[r] = s0 ? load_t16(s0 + cb + 16 * (rb0 + r) * GD, lane) : (f32x4){};
+    const Op<3> s0p = op_acc(S[0], S[1]);   // TRUNC
 
     ScanAhead<TIn> nx;
     auto fetch = [&](int ci) {
         const float* cw = ws + ((size_t)(chunk0 + ci) * p.hv + h) * kWsChunk;
-        scan_fetch_rows<TIn, true>(p, cw, start + GC * ci, min(GC, len - GC * ci), h, nx);
+        scan_fetch_rows<TIn>(p, cw, start + GC * ci, min(GC, len - GC * ci), h, nx);
 #pragma unroll
         for (int tb = 0; tb < 2; ++tb) nx.x[tb] = load_t16(cw + kWsU + 16 * tb * GD + cb, lane);
     };
@@ -406,7 +378,7 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
             for (int r = 0; r < 2; ++r) store_t16(sp + 16 * (rb0 + r) * GD, lane, S[r]);
         }
         lds_barrier();   // readers of the previous chunk's tiles and partials are done
-        L.T.template stage<true>(p, nx);
+        L.T.stage(p, nx);
         f32x4 vp[2] = {nx.x[0], nx.x[1]}, qs[2] = {};
         if (ci + 1 < n_ch) fetch(ci + 1);
         const Op<3> sp = op_acc(S[0], S[1]);
@@ -416,7 +388,7 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 #pragma unroll
         for (int tb = 0; tb < 2; ++tb) {
             L.P[wave][0][tb][lane] =
-                mul_planes(op_rows<3, PR>(L.T.W, 16 * tb + c16, 32 * wave, g4), sp, (f32x4){});
+                mul_planes(op_rows<3, PR>(L.T.W, 16 * tb + c16, 32 * wave, g4), TRUNC ? s0p : sp, (f32x4){});
             L.P[wave][1][tb][lane] =
                 mul_planes(op_rows<NQ, PR>(L.T.Q, 16 * tb + c16, 32 * wave, g4), sp, (f32x4){});
         }
@@ -486,13 +458,13 @@ __device__ __forceinline__ void rscan_start(const GdnDev& p, int node, int h, in
     }
 }
 // The chunk terms and this lane's dO tiles (column j, zero past the chunk).
-template <typename TIn, bool LOAD_W>
+template <typename TIn>
 __device__ __forceinline__ void rscan_fetch(const GdnDev& p, const ScanNode& nd, int ci, int h, int j, int g4,
                                             const float* ws, const TIn* d_o, int64_t do_st, int64_t do_sh,
                                             ScanAhead<TIn>& x) {
     const int c0 = GC * ci, Lc = min(GC, nd.len - c0);
     const float* cw = ws + ((size_t)(nd.chunk0 + ci) * p.hv + h) * kWsChunk;
-    scan_fetch_rows<TIn, LOAD_W>(p, cw, nd.start + c0, Lc, h, x);
+    scan_fetch_rows<TIn>(p, cw, nd.start + c0, Lc, h, x);
     const TIn* base = d_o + (int64_t)(nd.start + c0) * do_st + (int64_t)h * do_sh + j;
 #pragma unroll
     for (int tb = 0; tb < 2; ++tb)
@@ -508,9 +480,9 @@ __device__ __forceinline__ void rscan_fetch(const GdnDev& p, const ScanNode& nd,
 // tokens, two 16-token tiles), and dV' is produced in it, so all three are
 // MFMA B operands straight from registers:
 //   dV' = A^T dO + fk (k dS),  dS <- e^{G_L} dS + q^T (fq dO) - W^T dV'.
-// TRUNC (V' = U - W S0 with the node's initial state S0): the walk leaves out
-// the W term, and a second pass over the node's chunks subtracts
-// sum_c W_c^T dV'_c from the state gradient at the node's entry.
+// TRUNC (V' = U - W S0 with the node's initial state S0): the W terms of all
+// chunks belong to the gradient at the node's entry; they are summed apart
+// and join it there.
 template <typename TIn, bool TRUNC>
 __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn_rscan_cols_kernel(
         GdnDev p, int lvl_begin, const float* __restrict__ ws, const TIn* __restrict__ d_o, int64_t do_st,
@@ -526,9 +498,10 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     f32x4 dS[8];
     rscan_start<8>(p, nd.node, h, 0, jt, lane, node_dsin, dS);
 
+    f32x4 wsum[8] = {};   // TRUNC: - sum_c W_c^T dV'_c
     // one chunk ahead (the walk runs backwards)
     ScanAhead<TIn> nx;
-    rscan_fetch<TIn, !TRUNC>(p, nd, nd.n_ch - 1, h, j, g4, ws, d_o, do_st, do_sh, nx);
+    rscan_fetch<TIn>(p, nd, nd.n_ch - 1, h, j, g4, ws, d_o, do_st, do_sh, nx);
     for (int ci = nd.n_ch - 1; ci >= 0; --ci) {
         const size_t chn = (size_t)(nd.chunk0 + ci) * p.hv + h;
         {   // the gradient of this chunk's output state
@@ -537,9 +510,9 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
             for (int rb = 0; rb < 8; ++rb) store_t16(sp + 16 * rb * GD, lane, dS[rb]);
         }
         lds_barrier();   // readers of the previous chunk's tiles are done
-        L.template stage<!TRUNC>(p, nx);
+        L.stage(p, nx);
         const f32x4 dov[2] = {nx.x[0], nx.x[1]};
-        if (ci > 0) rscan_fetch<TIn, !TRUNC>(p, nd, ci - 1, h, j, g4, ws, d_o, do_st, do_sh, nx);
+        if (ci > 0) rscan_fetch<TIn>(p, nd, ci - 1, h, j, g4, ws, d_o, do_st, do_sh, nx);
         lds_barrier();
 
         // dV' as four partial sums added in order, partial w4 holding the
@@ -569,27 +542,14 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 #pragma unroll
         for (int rb = 0; rb < 8; ++rb) {
             f32x4 x = mul_planes(op_cols<NQ, PC>(L.Q, 16 * rb, lane), dos, (f32x4){});
-            if constexpr (!TRUNC) x = mul_planes(op_cols<3, PC>(L.W, 16 * rb, lane), dvs, x);
+            if constexpr (TRUNC) wsum[rb] += mul_planes(op_cols<3, PC>(L.W, 16 * rb, lane), dvs, (f32x4){});
+            else x = mul_planes(op_cols<3, PC>(L.W, 16 * rb, lane), dvs, x);
             dS[rb] = fma_tile(dS[rb], el, x);
         }
     }
     if constexpr (TRUNC) {
-        for (int ci = 0; ci < nd.n_ch; ++ci) {
-            const size_t chn = (size_t)(nd.chunk0 + ci) * p.hv + h;
-            const float* cw = ws + chn * kWsChunk;
-            const int i = t >> 3, d0 = 16 * (t & 7);
-            f32x4 w[4], dv[2];   // dV': this lane's own writes
 #pragma unroll
-            for (int e = 0; e < 4; ++e) w[e] = *(const f32x4*)(cw + kWsW + i * GD + d0 + 4 * e);
-#pragma unroll
-            for (int tb = 0; tb < 2; ++tb) dv[tb] = load_t16(chunk_dvp + chn * GC * GD + 16 * tb * GD + jt, lane);
-            lds_barrier();   // readers of the previous chunk's W are done
-            put16<PC>(L.W, i, d0, w);
-            lds_barrier();
-            const Op<3> dvs = op_acc(-dv[0], -dv[1]);
-#pragma unroll
-            for (int rb = 0; rb < 8; ++rb) dS[rb] += mul_planes(op_cols<3, PC>(L.W, 16 * rb, lane), dvs, (f32x4){});
-        }
+        for (int rb = 0; rb < 8; ++rb) dS[rb] += wsum[rb];
     }
     // dS at the node's entry, summed into its parent by the next (shallower) level.
     float* sp = node_dsin + ((size_t)nd.node * p.hv + h) * GD * GD + jt;
@@ -603,11 +563,10 @@ struct RscanRowsLds {
     f32x4 P[4][2][64];   // per wave: its partial dV', both token tiles, lane-major
 };
 
-// As gdn_rscan_cols_kernel (exact rule), in the row layout of
-// gdn_scan_rows_kernel: wave w holds dS[32w .., c0 ..]. dV' is summed over the
+// As gdn_rscan_cols_kernel, in the row layout of gdn_scan_rows_kernel: wave w holds dS[32w .., c0 ..]. dV' is summed over the
 // waves' rows through LDS, in wave order (waves 0 and 1 also add the A^T dO
 // term of token tiles 0 and 1); every wave then updates its rows of dS.
-template <typename TIn>
+template <typename TIn, bool TRUNC>
 __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn_rscan_rows_kernel(
         GdnDev p, int lvl_begin, const float* __restrict__ ws, const TIn* __restrict__ d_o, int64_t do_st,
         int64_t do_sh, float* __restrict__ chunk_dso, float* __restrict__ chunk_dvp, float* __restrict__ node_dsin) {
@@ -622,9 +581,10 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     const int rb0 = 2 * wave;
     f32x4 dS[2];
     rscan_start<2>(p, nd.node, h, rb0, cb, lane, node_dsin, dS);
+    f32x4 wsum[2] = {};   // TRUNC: - sum_c W_c^T dV'_c
 
     ScanAhead<TIn> nx;
-    rscan_fetch<TIn, true>(p, nd, nd.n_ch - 1, h, j, g4, ws, d_o, do_st, do_sh, nx);
+    rscan_fetch<TIn>(p, nd, nd.n_ch - 1, h, j, g4, ws, d_o, do_st, do_sh, nx);
     for (int ci = nd.n_ch - 1; ci >= 0; --ci) {
         const size_t chn = (size_t)(nd.chunk0 + ci) * p.hv + h;
         {
@@ -633,9 +593,9 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
             for (int r = 0; r < 2; ++r) store_t16(sp + 16 * (rb0 + r) * GD, lane, dS[r]);
         }
         lds_barrier();   // readers of the previous chunk's tiles and partials are done
-        L.T.template stage<true>(p, nx);
+        L.T.stage(p, nx);
         const f32x4 dov[2] = {nx.x[0], nx.x[1]};
-        if (ci > 0) rscan_fetch<TIn, true>(p, nd, ci - 1, h, j, g4, ws, d_o, do_st, do_sh, nx);
+        if (ci > 0) rscan_fetch<TIn>(p, nd, ci - 1, h, j, g4, ws, d_o, do_st, do_sh, nx);
         const Op<3> sp = op_acc(dS[0], dS[1]);
         lds_barrier();
 
@@ -666,9 +626,14 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
             f32x4 x = mul_planes(op_cols<NQ, PC>(L.T.Q, 16 * (rb0 + r), lane), dos, (f32x4){});
-            x = mul_planes(op_cols<3, PC>(L.T.W, 16 * (rb0 + r), lane), dvs, x);
+            if constexpr (TRUNC) wsum[r] += mul_planes(op_cols<3, PC>(L.T.W, 16 * (rb0 + r), lane), dvs, (f32x4){});
+            else x = mul_planes(op_cols<3, PC>(L.T.W, 16 * (rb0 + r), lane), dvs, x);
             dS[r] = fma_tile(dS[r], el, x);
         }
+    }
+    if constexpr (TRUNC) {
+#pragma unroll
+        for (int r = 0; r < 2; ++r) dS[r] += wsum[r];
     }
     float* sp = node_dsin + ((size_t)nd.node * p.hv + h) * GD * GD + cb;
 #pragma unroll

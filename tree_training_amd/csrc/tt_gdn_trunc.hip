@@ -9,7 +9,7 @@
 // R is never stored: a node is cut into the same 32-row blocks the scans walk
 // (one block = one chunk), and R applied to a block-row is a sum over the
 // node's other blocks (earlier ones for R, later ones for R^T), each R block
-// formed on the fly from k^ k^T (fp32 MFMA) and the decays. The work is
+// formed on the fly from k^ k^T and the decays (bf16 planes, tt_planes.h). The work is
 // quadratic in the node length, like the reference's L x L matrices.
 //
 // Backward, given dF = [dV' | dW] of every chunk (level scans):
@@ -22,12 +22,11 @@
 // plus the Y0 terms (dv = beta dY0_v, dbeta, dk^ and dG from beta e^G k^). The
 // node-level dG becomes dg by a suffix sum over the node; the chunk backward
 // (tt_gdn.hip) adds dk^ and that suffix sum to its own terms.
-#include "tt_gdn_common.h"
+#include "tt_gdn_planes.h"
 
 namespace {
 
 constexpr int GW = 2 * GD;        // width of [v | k] rows
-constexpr int RX = GW + 8;        // LDS row stride of [GC x GW] tiles: rows 4 apart land 32 banks apart
 
 // Node of chunk c and the chunk's block index within it; false for a malformed list.
 __device__ __forceinline__ bool chunk_block(const GdnDev& p, int c, int& node, int& b, int& nb) {
@@ -39,74 +38,19 @@ __device__ __forceinline__ bool chunk_block(const GdnDev& p, int c, int& node, i
     return len >= 1 && b >= 0 && b < nb && c0 >= 0 && c0 <= p.n_chunks - nb;
 }
 
-// l2-normalised k rows of one chunk into K (stride RS), zeros past len; with
-// X, also that chunk's Y0 rows [beta v | beta e^G k^] (stride RX). gn: the
-// chunk's 32 node-level decays. Thread t handles row t/8, dims 16*(t%8)..+15.
-template <typename TIn>
-__device__ __forceinline__ void load_k_rows(const GdnDev& p, int start, int len, int h, float* K, float* X,
-                                            const float* gn) {
-    const int t = threadIdx.x, i = t >> 3, d0 = 16 * (t & 7), hk = h / p.rep;
-    const bool valid = i < len;
-    const int64_t tok = start + i;
-    float kv[16], vv[16];
-    if (valid) {
-        load16((const TIn*)p.k + tok * p.k_st + hk * p.k_sh + d0, kv);
-        if (X) load16((const TIn*)p.v + tok * p.v_st + h * p.v_sh + d0, vv);
-    } else {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) kv[e] = vv[e] = 0.0f;
-    }
-    float sk = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) sk = fmaf(kv[e], kv[e], sk);
-    sk = row8_sum(sk);
-    const float fk = p.l2 ? 1.0f / sqrtf(sk + 1e-6f) : 1.0f;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) kv[e] *= fk;
-#pragma unroll
-    for (int e = 0; e < 16; e += 4)
-        *(f32x4*)&K[i * RS + d0 + e] = (f32x4){kv[e], kv[e + 1], kv[e + 2], kv[e + 3]};
-    if (X) {
-        const float bt = valid ? p.beta[tok * p.b_st + h] : 0.0f;
-        const float bg = bt * expf(gn[i]);
-#pragma unroll
-        for (int e = 0; e < 16; e += 4) {
-            *(f32x4*)&X[i * RX + d0 + e] = (f32x4){bt * vv[e], bt * vv[e + 1], bt * vv[e + 2], bt * vv[e + 3]};
-            *(f32x4*)&X[i * RX + GD + d0 + e] =
-                (f32x4){bg * kv[e], bg * kv[e + 1], bg * kv[e + 2], bg * kv[e + 3]};
-        }
-    }
-}
+// Values of the chunk rows held per (chunk, head) beside the chunk terms: the
+// node-level decay and 1 / |k| (1 without the l2 norm).
+struct NodeRows {
+    const float* gn;   // [chunk, hv, 32]
+    const float* fk;   // [chunk, hv, 32]
+};
 
-// Decays and betas of one chunk's 32 rows (beta zero past len), threads < 32.
-__device__ __forceinline__ void load_gb(const GdnDev& p, int start, int len, int h, const float* gn, float* G,
-                                        float* B) {
-    const int t = threadIdx.x;
-    if (t < GC) {
-        G[t] = gn[t];
-        B[t] = t < len ? p.beta[(int64_t)(start + t) * p.b_st + h] : 0.0f;
-    }
-}
-
-// k^_t k^_p^T partial over head dims 32w .. 32w+31 (wave w), into KP[w] as
-// rows of the target block, columns of the partner block.
-__device__ __forceinline__ void kk_partial(const float* Kt, const float* Kp, float* KP) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, col = lane & 31, half = lane >> 5;
-    f32x16 kk = {};
-#pragma unroll
-    for (int q4 = 0; q4 < 4; ++q4) {
-        const int k0 = 32 * wave + 8 * q4 + 4 * half;
-        const f32x4 a = *(const f32x4*)&Kt[col * RS + k0];
-        const f32x4 b = *(const f32x4*)&Kp[col * RS + k0];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) kk = mfma_f32(a[e], b[e], kk);
-    }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) KP[wave * GC * MS + acc_row(r, half) * MS + col] = kk[r];
-}
-
-__device__ __forceinline__ float sum4(const float* P, int idx) {
-    return P[idx] + P[GC * MS + idx] + P[2 * GC * MS + idx] + P[3 * GC * MS + idx];
+// Workgroup -> (chunk, v head), heads fastest: with Hv a multiple of 8 a head
+// stays on one XCD, whose L2 then holds the blocks that a node's workgroups
+// share.
+__device__ __forceinline__ void chunk_head(const GdnDev& p, int& c, int& h) {
+    c = __builtin_amdgcn_readfirstlane(blockIdx.x / p.hv);
+    h = __builtin_amdgcn_readfirstlane(blockIdx.x % p.hv);
 }
 
 // ----------------------------------------------------------------------------
@@ -127,6 +71,104 @@ __global__ __launch_bounds__(64) void gdn_gnode_kernel(GdnDev p, const float* __
         carry += last;
     }
 }
+// fk = 1 / |k| and Y0 = [beta v | beta e^G k^] of every row, Y0 into the
+// chunk terms' U and W slots.
+template <typename TIn>
+__global__ __launch_bounds__(GT) void gdn_y0_kernel(GdnDev p, float* __restrict__ prep, const float* __restrict__ gn,
+                                                    float* __restrict__ fk) {
+    int c, h, start, len;
+    chunk_head(p, c, h);
+    if (!chunk_span(p, c, start, len)) return;
+    const int t = threadIdx.x, i = t >> 3, d0 = 16 * (t & 7);
+    const size_t chn = (size_t)c * p.hv + h;
+    const int64_t tok = start + i;
+    float kv[16], vv[16], bt = 0.0f;
+    if (i < len) {
+        load16((const TIn*)p.k + tok * p.k_st + (int64_t)(h / p.rep) * p.k_sh + d0, kv);
+        load16((const TIn*)p.v + tok * p.v_st + (int64_t)h * p.v_sh + d0, vv);
+        bt = p.beta[tok * p.b_st + h];
+    } else {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) kv[e] = vv[e] = 0.0f;
+    }
+    float sk = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) sk = fmaf(kv[e], kv[e], sk);
+    sk = row8_sum(sk);
+    const float f = p.l2 ? 1.0f / sqrtf(sk + 1e-6f) : 1.0f, bg = bt * expf(gn[chn * GC + i]);
+    if ((t & 7) == 0) fk[chn * GC + i] = f;
+    float* u = prep + chn * kWsChunk + kWsU + i * GD + d0;
+    float* w = prep + chn * kWsChunk + kWsW + i * GD + d0;
+#pragma unroll
+    for (int e = 0; e < 16; e += 4) {
+        *(f32x4*)(u + e) = (f32x4){bt * vv[e], bt * vv[e + 1], bt * vv[e + 2], bt * vv[e + 3]};
+        *(f32x4*)(w + e) = (f32x4){bg * (f * kv[e]), bg * (f * kv[e + 1]), bg * (f * kv[e + 2]), bg * (f * kv[e + 3])};
+    }
+}
+
+// A target block (chunk c, v head h) and where its node's blocks are; the
+// wave's quadrant of a [32 target rows x 32 partner rows] matrix (rows
+// 16 qi + g4 + v, column 16 qj + c16 of lane l).
+struct BlockPair {
+    int b, nb, start, len, nstart, nlen, chunk0, h, hk;
+    int qi, qj, lane, c16, g4, qr, qc;
+    size_t chn;
+    __device__ __forceinline__ bool init(const GdnDev& p) {
+        int c, node;
+        chunk_head(p, c, h);
+        if (!chunk_block(p, c, node, b, nb) || !chunk_span(p, c, start, len)) return false;
+        hk = h / p.rep;
+        nstart = p.node_start[node];
+        nlen = p.node_len[node];
+        chunk0 = p.node_chunk0[node];
+        chn = (size_t)c * p.hv + h;
+        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        qi = wave >> 1;
+        qj = wave & 1;
+        lane = threadIdx.x & 63;
+        c16 = lane & 15;
+        g4 = 4 * (lane >> 4);
+        qr = 16 * qi + g4;
+        qc = 16 * qj + c16;
+        return true;
+    }
+    __device__ __forceinline__ size_t partner(const GdnDev& p, int bp, int& startp, int& lenp) const {
+        startp = nstart + GC * bp;
+        lenp = min(GC, nlen - GC * bp);
+        return (size_t)(chunk0 + bp) * p.hv + h;
+    }
+    // k rows 16 tile + c16 of the block at `st` (of `n` rows) as four operands, as they come
+    template <typename TIn>
+    __device__ __forceinline__ void k_rows(const GdnDev& p, int st, int n, int tile, Op<kInPlanes<TIn>> (&x)[4]) const {
+        const int r = 16 * tile + c16;
+        const TIn* row = (const TIn*)p.k + (int64_t)(st + r) * p.k_st + (int64_t)hk * p.k_sh;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) x[m] = op_global<TIn>(row, r < n, 32 * m, g4);
+    }
+    // beta of row r of the block at `st` (zero past its n rows)
+    __device__ __forceinline__ float beta(const GdnDev& p, int st, int n, int r) const {
+        return r < n ? p.beta[(int64_t)(st + r) * p.b_st + h] : 0.0f;
+    }
+};
+// k k^T of the quadrant (no norms).
+template <int NQ>
+__device__ __forceinline__ f32x4 kk_quadrant(const Op<NQ> (&a)[4], const Op<NQ> (&b)[4]) {
+    Sum2 x;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) x.add(a[m], b[m]);
+    return x.sum();
+}
+// Column operand of a [GC][ld] fp32 matrix in global memory: rows k (n of
+// them exist), column at `col`.
+__device__ __forceinline__ Op<3> op_gcols(const float* col, int ld, int g4) {
+    f32x4 a, b;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        a[v] = col[(g4 + v) * ld];
+        b[v] = col[(16 + g4 + v) * ld];
+    }
+    return op_acc(a, b);
+}
 
 // ----------------------------------------------------------------------------
 // out = R X over a node's blocks (lower: target block b, partners b' <= b) or
@@ -134,127 +176,117 @@ __global__ __launch_bounds__(64) void gdn_gnode_kernel(GdnDev p, const float* __
 // ----------------------------------------------------------------------------
 enum { TRI_Y1 = 0, TRI_UW = 1, TRI_DF1 = 2, TRI_DY0 = 3 };
 struct TriArgs {
-    const float* gn;      // [chunk, hv, 32] node-level decay
+    NodeRows rows;
     const float* xa;      // TRI_UW: y1; TRI_DF1: dV'; TRI_DY0: dF1
     const float* xb;      // TRI_DF1: dW
     const float* fa;      // TRI_DY0: dV' and dW (the target's dF)
     const float* fb;
     float* out;           // TRI_Y1: y1; TRI_DF1: dF1; TRI_DY0: dY0 ([chunk, hv, 32, 256])
-    float* prep;          // TRI_UW: U and W slots of the chunk terms
+    float* prep;          // chunk terms: U and W slots hold Y0, and U, W after TRI_UW
 };
 
-struct TriLds {
-    float Kt[GC * RS];
-    float Kp[GC * RS];
-    float X[GC * RX];
-    float KP[4 * GC * MS];
-    float R[GC * MS];
-    float Gt[GC], Gp[GC], Bt[GC], Bp[GC];
-};
-
-// MODE: TRI_Y1   y1 = R Y0 (Y0 from the inputs)
+// MODE: TRI_Y1   y1 = R Y0
 //       TRI_UW   [U | W] = Y0 + y1 + R y1, into the chunk terms
 //       TRI_DF1  dF1 = R^T [dV' | dW]
 //       TRI_DY0  dY0 = dF + dF1 + R^T dF1
-// Wave w owns output columns 64w .. 64w+63 (two accumulator tiles).
+// Wave w forms its quadrant of each R block from k rows read straight into MFMA
+// operands, shares it through LDS as planes (rows times alt; two buffers, one
+// barrier a block) and owns output columns 64w .. 64w+63, whose X it reads as
+// operands from global memory: 15 KB of LDS, so the chains of short blocks of
+// many workgroups overlap on a CU. 4,096-token tree, 16 v heads, bf16:
+// 281-403 -> 117-149 us a mode (fp32 MFMA before).
 template <int MODE, typename TIn>
 __global__ __launch_bounds__(GT) void gdn_tri_kernel(GdnDev p, TriArgs a) {
     constexpr bool UPPER = MODE >= TRI_DF1;
-    __shared__ __attribute__((aligned(16))) TriLds L;
-    const int c = blockIdx.x, h = blockIdx.y, t = threadIdx.x;
-    const int wave = t >> 6, lane = t & 63, col = lane & 31, half = lane >> 5;
-    int node, b, nb, start, len;
-    if (!chunk_block(p, c, node, b, nb) || !chunk_span(p, c, start, len)) return;
-    const int nstart = p.node_start[node], nlen = p.node_len[node], chunk0 = p.node_chunk0[node];
-    const size_t chn = (size_t)c * p.hv + h;
-
-    load_k_rows<TIn>(p, start, len, h, L.Kt, nullptr, nullptr);
-    load_gb(p, start, len, h, a.gn + chn * GC, L.Gt, L.Bt);
-    f32x16 acc0 = {}, acc1 = {};
-    const int bp0 = UPPER ? b : 0, bp1 = UPPER ? nb : b + 1;
+    constexpr int NQ = kInPlanes<TIn>;
+    __shared__ __attribute__((aligned(16))) __bf16 R[2][3 * GC * AR];
+    BlockPair q;
+    if (!q.init(p)) return;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool vcols = wave < 2;   // the wave's columns: of v (0 .. 127) or of k (128 .. 255)
+    const int cw = 64 * (wave & 1) + q.c16;
+    Op<NQ> kt[4];
+    q.k_rows<TIn>(p, q.start, q.len, q.qi, kt);
+    f32x4 gt, ft;   // decay and -(beta, lower) / |k| of the quadrant's rows, times alt
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int r = q.qr + v;
+        gt[v] = a.rows.gn[q.chn * GC + r];
+        ft[v] = -a.rows.fk[q.chn * GC + r] * alt(v) * (UPPER ? 1.0f : q.beta(p, q.start, q.len, r));
+    }
+    f32x4 acc[2][4] = {};
+    const int bp0 = UPPER ? q.b : 0, bp1 = UPPER ? q.nb : q.b + 1;
     for (int bp = bp0; bp < bp1; ++bp) {
-        const int cp = chunk0 + bp, startp = nstart + GC * bp, lenp = min(GC, nlen - GC * bp);
-        const size_t chp = (size_t)cp * p.hv + h;
-        __syncthreads();   // the previous partner's readers are done
-        if constexpr (MODE == TRI_Y1) {
-            load_k_rows<TIn>(p, startp, lenp, h, L.Kp, L.X, a.gn + chp * GC);
-        } else {
-            load_k_rows<TIn>(p, startp, lenp, h, L.Kp, nullptr, nullptr);
-            const int i = t >> 3, c0 = 32 * (t & 7);
-            const float* src;
-            if constexpr (MODE == TRI_DF1)
-                src = c0 < GD ? a.xa + (chp * GC + i) * GD + c0 : a.xb + (chp * GC + i) * GD + (c0 - GD);
-            else
-                src = a.xa + (chp * GC + i) * GW + c0;
+        int startp, lenp;
+        const size_t chp = q.partner(p, bp, startp, lenp);
+        __bf16* Rb = R[(bp - bp0) & 1];
+        {
+            f32x4 r = {};
+            if (bp != q.b || (UPPER ? q.qj >= q.qi : q.qi >= q.qj)) {
+                Op<NQ> kp[4];
+                q.k_rows<TIn>(p, startp, lenp, q.qj, kp);
+                const float gp = a.rows.gn[chp * GC + q.qc];
+                const float fp = a.rows.fk[chp * GC + q.qc] * (UPPER ? q.beta(p, startp, lenp, q.qc) : 1.0f);
+                r = kk_quadrant<NQ>(kt, kp);
 #pragma unroll
-            for (int e = 0; e < 32; e += 4) *(f32x4*)&L.X[i * RX + c0 + e] = *(const f32x4*)(src + e);
+                for (int v = 0; v < 4; ++v) {
+                    const int i = q.qr + v;
+                    const bool vis = i < q.len && q.qc < lenp && (bp != q.b || (UPPER ? q.qc > i : q.qc < i));
+                    r[v] = vis ? ft[v] * (r[v] * fp) * expf(UPPER ? gp - gt[v] : gt[v] - gp) : 0.0f;
+                }
+            }
+            put_quadrant<AR>(Rb, q.qr, q.qc, r);
         }
-        load_gb(p, startp, lenp, h, a.gn + chp * GC, L.Gp, L.Bp);
-        __syncthreads();
-        kk_partial(L.Kt, L.Kp, L.KP);
-        __syncthreads();
-        {   // R[target row][partner row] (R^T of the partner's rows for UPPER)
-            const int i = t >> 3;
+        // this wave's columns of the partner's X
+        Op<3> x[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int m = (t & 7) + 8 * e;
-                const float kk = sum4(L.KP, i * MS + m);
-                const bool vis = i < len && m < lenp && (UPPER ? (bp > b || m > i) : (bp < b || m < i));
-                float r = 0.0f;
-                if (vis) r = UPPER ? -L.Bp[m] * kk * expf(L.Gp[m] - L.Gt[i]) : -L.Bt[i] * kk * expf(L.Gt[i] - L.Gp[m]);
-                L.R[i * MS + m] = r;
+        for (int cb = 0; cb < 4; ++cb) {
+            const int col = cw + 16 * cb;
+            if constexpr (MODE == TRI_Y1) {
+                x[cb] = op_gcols(a.prep + chp * kWsChunk + (vcols ? kWsU : kWsW) + col, GD, q.g4);
+            } else if constexpr (MODE == TRI_DF1) {
+                x[cb] = op_gcols((vcols ? a.xa : a.xb) + chp * GC * GD + col, GD, q.g4);
+            } else {
+                x[cb] = op_gcols(a.xa + chp * GC * GW + (vcols ? 0 : GD) + col, GW, q.g4);
             }
         }
-        __syncthreads();
+        lds_barrier();   // the R block is complete
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const f32x4 rv = *(const f32x4*)&L.R[col * MS + 8 * q + 4 * half];
+        for (int tb = 0; tb < 2; ++tb) {
+            const Op<3> r = op_rows<3, AR>(Rb, 16 * tb + q.c16, 0, q.g4);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int k = 8 * q + 4 * half + e;
-                acc0 = mfma_f32(rv[e], L.X[k * RX + 64 * wave + col], acc0);
-                acc1 = mfma_f32(rv[e], L.X[k * RX + 64 * wave + 32 + col], acc1);
-            }
+            for (int cb = 0; cb < 4; ++cb) acc[tb][cb] += mul_planes(r, x[cb], (f32x4){});
         }
     }
 
-    // Accumulator element r: row acc_row(r, half), column 64 wave + 32 tile + col.
+    // Accumulator element v: row 16 tb + g4 + v (times alt), column 16 cb of the wave's.
 #pragma unroll
-    for (int tile = 0; tile < 2; ++tile) {
-        const f32x16& acc = tile ? acc1 : acc0;
-        const int j = 64 * wave + 32 * tile + col;
+    for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int i = acc_row(r, half);
-            float val = acc[r];
-            if constexpr (MODE == TRI_UW) {
-                float y0;
-                if (j < GD) {
-                    const float vj = i < len ? (float)((const TIn*)p.v)[(int64_t)(start + i) * p.v_st +
-                                                                         (int64_t)h * p.v_sh + j]
-                                             : 0.0f;
-                    y0 = L.Bt[i] * vj;
+        for (int v = 0; v < 4; ++v) {
+            const int i = 16 * tb + q.g4 + v;
+#pragma unroll
+            for (int cb = 0; cb < 4; ++cb) {
+                const int col = cw + 16 * cb, j = (vcols ? 0 : GD) + col;
+                float val = v & 1 ? -acc[tb][cb][v] : acc[tb][cb][v];
+                if constexpr (MODE == TRI_UW) {
+                    float* y0 = a.prep + q.chn * kWsChunk + (vcols ? kWsU : kWsW) + i * GD + col;
+                    *y0 = val + (*y0 + a.xa[(q.chn * GC + i) * GW + j]);
                 } else {
-                    y0 = L.Bt[i] * expf(L.Gt[i]) * L.Kt[i * RS + (j - GD)];
+                    if constexpr (MODE == TRI_DY0)
+                        val += (vcols ? a.fa : a.fb)[(q.chn * GC + i) * GD + col] + a.xa[(q.chn * GC + i) * GW + j];
+                    a.out[(q.chn * GC + i) * GW + j] = val;
                 }
-                val += y0 + a.xa[(chn * GC + i) * GW + j];
-                float* dst = a.prep + chn * kWsChunk + (j < GD ? kWsU + i * GD + j : kWsW + i * GD + (j - GD));
-                *dst = val;
-            } else {
-                if constexpr (MODE == TRI_DY0)
-                    val += (j < GD ? a.fa[(chn * GC + i) * GD + j] : a.fb[(chn * GC + i) * GD + (j - GD)]) +
-                           a.xa[(chn * GC + i) * GW + j];
-                a.out[(chn * GC + i) * GW + j] = val;
             }
         }
-    }
 }
 
 // ----------------------------------------------------------------------------
-// gradient of R, row side: per target block b over partners b' <= b
+// gradient of R: row side (per target block b over partners b' <= b) and
+// column side (partners b' >= b: rows of R in the partner, columns in the target)
 // ----------------------------------------------------------------------------
 struct EArgs {
-    const float* gn;
+    NodeRows rows;
     const float* y1;      // R Y0
     const float* dvp;     // dV' ([chunk, hv, 32, 128])
     const float* dw;      // dW
@@ -267,235 +299,210 @@ struct EArgs {
 };
 
 struct ELds {
-    float Kt[GC * RS];
-    float Kp[GC * RS];
-    float EP[4 * GC * MS];
-    float KP[4 * GC * MS];
-    float M[GC * MS];
-    float Gt[GC], Gp[GC], Bt[GC], Bp[GC];
+    union {
+        float E[4][GC * MS];    // the waves' slices of the 512-wide contraction
+        float J[GC * RS];       // at the end: dk^ rows
+    };
+    __bf16 M[3 * GC * AR];
+    float sum[2][GC];           // row sums over the column tiles
 };
 
-// Wave w's columns of the 512-wide contraction E = [dF | dF1] [Y0 + y1 | Y0]^T:
+// Wave w's 128 columns of the 512-wide contraction E = [dF | dF1] [Y0 + y1 | Y0]^T:
 //   w = 0: dV' . (beta v + y1_v)      w = 1: dW . (beta e^G k^ + y1_k)
 //   w = 2: dF1_v . beta v             w = 3: dF1_k . beta e^G k^
-// A row of [dF | dF1] (source `side` 0) or of [Y0 + y1 | Y0] (side 1) for the
-// lane's MFMA operand: 16 groups of 4 at columns 8 g + 4 half.
+// Row `row` of a block (chunk-head ch, tokens st .. st + n - 1) of [Y0 + y1 | Y0].
 template <typename TIn>
-__device__ __forceinline__ f32x4 e_operand_y(const GdnDev& p, const EArgs& a, int wave, int g, int half,
-                                             size_t ch, int row, int tok, bool in, int h, float bm, float bgm,
-                                             const float* K) {
-    const int d = 8 * g + 4 * half;
-    f32x4 y = {};
-    if (wave == 0 || wave == 2) {
-        if (in) y = load4((const TIn*)p.v + (int64_t)tok * p.v_st + (int64_t)h * p.v_sh + d) * bm;
-        if (wave == 0) y += *(const f32x4*)(a.y1 + (ch * GC + row) * GW + d);
-    } else {
-        y = *(const f32x4*)&K[row * RS + d] * bgm;
-        if (wave == 1) y += *(const f32x4*)(a.y1 + (ch * GC + row) * GW + GD + d);
+__device__ __forceinline__ Op<3> e_op_y(const GdnDev& p, const EArgs& a, const BlockPair& q, int wave, size_t ch,
+                                        int st, int n, int row, float f, int k0) {
+    const int64_t tok = st + row;
+    const TIn* x = (wave & 1) == 0 ? (const TIn*)p.v + tok * p.v_st + (int64_t)q.h * p.v_sh
+                                   : (const TIn*)p.k + tok * p.k_st + (int64_t)q.hk * p.k_sh;
+    f32x4 y[2] = {};
+#pragma unroll
+    for (int n2 = 0; n2 < 2; ++n2) {
+        const int d = k0 + 16 * n2 + q.g4;
+        if (row < n) y[n2] = load4(x + d) * f;
+        if (wave < 2) y[n2] += *(const f32x4*)(a.y1 + (ch * GC + row) * GW + (wave ? GD : 0) + d);
     }
-    return y;
+    return op_acc(y[0], y[1]);
 }
-__device__ __forceinline__ f32x4 e_operand_f(const EArgs& a, int wave, int g, int half, size_t ch, int row) {
-    const int d = 8 * g + 4 * half;
-    switch (wave) {
-        case 0: return *(const f32x4*)(a.dvp + (ch * GC + row) * GD + d);
-        case 1: return *(const f32x4*)(a.dw + (ch * GC + row) * GD + d);
-        case 2: return *(const f32x4*)(a.df1 + (ch * GC + row) * GW + d);
-        default: return *(const f32x4*)(a.df1 + (ch * GC + row) * GW + GD + d);
-    }
+// ... and of [dF | dF1].
+__device__ __forceinline__ Op<3> e_op_f(const EArgs& a, const BlockPair& q, int wave, size_t ch, int row, int k0) {
+    const float* x = wave == 0 ? a.dvp + (ch * GC + row) * GD
+                   : wave == 1 ? a.dw + (ch * GC + row) * GD
+                               : a.df1 + (ch * GC + row) * GW + (wave == 2 ? 0 : GD);
+    return op_acc(*(const f32x4*)(x + k0 + q.g4), *(const f32x4*)(x + k0 + 16 + q.g4));
 }
 
-template <typename TIn>
-__global__ __launch_bounds__(GT) void gdn_erow_kernel(GdnDev p, EArgs a) {
+// ROW: M = E * D over partners b' <= b: dk^ rows of the target
+// -= beta (M k^_p), dbeta, dG, and the Y0 terms (dv among them). Otherwise the
+// column side: M^T over partners b' >= b, dk^ += M^T (beta k^)_p (negated), dG.
+// The target's planes of F (ROW) or Y stay in registers (96); the partner's
+// rows come straight into operands. 4,096-token tree, 16 v heads, bf16:
+// rows 523 -> 405 us, columns 446 -> 283. Bound by the latency of those loads:
+// the registers leave two waves a SIMD.
+template <typename TIn, bool ROW>
+__global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn_e_kernel(GdnDev p, EArgs a) {
+    constexpr int NQ = kInPlanes<TIn>;
     __shared__ __attribute__((aligned(16))) ELds L;
-    const int c = blockIdx.x, h = blockIdx.y, t = threadIdx.x;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, col = lane & 31, half = lane >> 5;
-    int node, b, nb, start, len;
-    if (!chunk_block(p, c, node, b, nb) || !chunk_span(p, c, start, len)) return;
-    const int nstart = p.node_start[node], nlen = p.node_len[node], chunk0 = p.node_chunk0[node];
-    const size_t chn = (size_t)c * p.hv + h;
+    BlockPair q;
+    if (!q.init(p)) return;
+    const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int w0 = 32 * wave;   // this wave's columns of dk^
 
-    load_k_rows<TIn>(p, start, len, h, L.Kt, nullptr, nullptr);
-    load_gb(p, start, len, h, a.gn + chn * GC, L.Gt, L.Bt);
-    f32x4 ar[16];   // this lane's row of the target's [dF | dF1] slice
+    // y's factor of a row: beta (times e^G / |k| in the k slices)
+    auto y_factor = [&](size_t ch, int st, int n, int row) {
+        float f = q.beta(p, st, n, row);
+        if (wave & 1) f *= expf(a.rows.gn[ch * GC + row]) * a.rows.fk[ch * GC + row];
+        return f;
+    };
+    Op<3> at[2][4];
 #pragma unroll
-    for (int g = 0; g < 16; ++g) ar[g] = e_operand_f(a, wave, g, half, chn, col);
-    f32x16 dk = {};
-    float s_acc = 0.0f;   // row t/8: sum_m M (k^ . k^)
-    for (int bp = 0; bp <= b; ++bp) {
-        const int cp = chunk0 + bp, startp = nstart + GC * bp, lenp = min(GC, nlen - GC * bp);
-        const size_t chp = (size_t)cp * p.hv + h;
-        __syncthreads();
-        load_k_rows<TIn>(p, startp, lenp, h, L.Kp, nullptr, nullptr);
-        load_gb(p, startp, lenp, h, a.gn + chp * GC, L.Gp, L.Bp);
-        __syncthreads();
-        {
-            const bool in = col < lenp;
-            const float bm = L.Bp[col], bgm = bm * expf(L.Gp[col]);
-            f32x16 ep = {};
+    for (int tb = 0; tb < 2; ++tb) {
+        const int row = 16 * tb + q.c16;
+        const float f = ROW ? 0.0f : y_factor(q.chn, q.start, q.len, row);
 #pragma unroll
-            for (int g = 0; g < 16; ++g) {
-                const f32x4 y = e_operand_y<TIn>(p, a, wave, g, half, chp, col, startp + col, in, h, bm, bgm, L.Kp);
+        for (int m = 0; m < 4; ++m)
+            at[tb][m] = ROW ? e_op_f(a, q, wave, q.chn, row, 32 * m)
+                            : e_op_y<TIn>(p, a, q, wave, q.chn, q.start, q.len, row, f, 32 * m);
+    }
+    Op<NQ> kt[4];
+    q.k_rows<TIn>(p, q.start, q.len, q.qi, kt);
+    f32x4 gt, ft;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) ep = mfma_f32(ar[g][e], y[e], ep);
+    for (int v = 0; v < 4; ++v) {
+        gt[v] = a.rows.gn[q.chn * GC + q.qr + v];
+        ft[v] = a.rows.fk[q.chn * GC + q.qr + v];
+    }
+    f32x4 dk[2][2] = {};   // row tile, column tile w0 + 16 cb
+    f32x4 sums = {};       // sum over the partners of M (k^ . k^) (column side: times beta)
+    const int bp0 = ROW ? 0 : q.b, bp1 = ROW ? q.b + 1 : q.nb;
+    for (int bp = bp0; bp < bp1; ++bp) {
+        int startp, lenp;
+        const size_t chp = q.partner(p, bp, startp, lenp);
+#pragma unroll
+        for (int cb = 0; cb < 2; ++cb) {
+            const int row = 16 * cb + q.c16;
+            const float f = ROW ? y_factor(chp, startp, lenp, row) : 0.0f;
+            Sum2 e[2];
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                const Op<3> x = ROW ? e_op_y<TIn>(p, a, q, wave, chp, startp, lenp, row, f, 32 * m)
+                                    : e_op_f(a, q, wave, chp, row, 32 * m);
+                e[0].add(at[0][m], x);
+                e[1].add(at[1][m], x);
             }
 #pragma unroll
-            for (int r = 0; r < 16; ++r) L.EP[wave * GC * MS + acc_row(r, half) * MS + col] = ep[r];
-        }
-        kk_partial(L.Kt, L.Kp, L.KP);
-        __syncthreads();
-        {
-            const int i = t >> 3;
+            for (int tb = 0; tb < 2; ++tb) {
+                const f32x4 r = e[tb].sum();
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int m = (t & 7) + 8 * e;
-                const bool vis = i < len && m < lenp && (bp < b || m < i);
-                float mv = 0.0f;
-                if (vis) mv = sum4(L.EP, i * MS + m) * expf(L.Gt[i] - L.Gp[m]);
-                s_acc = fmaf(mv, sum4(L.KP, i * MS + m), s_acc);
-                L.M[i * MS + m] = mv;
+                for (int v = 0; v < 4; ++v) L.E[wave][(16 * tb + q.g4 + v) * MS + row] = r[v];
             }
         }
-        __syncthreads();
-        // dk^ (rows of the target) += M k^_p over head dims 32 wave + col
+        const float gp = a.rows.gn[chp * GC + q.qc], fp = a.rows.fk[chp * GC + q.qc];
+        const float bm = ROW ? 1.0f : q.beta(p, startp, lenp, q.qc);
+        f32x4 kk = {};
+        const bool any = bp != q.b || (ROW ? q.qi >= q.qj : q.qj >= q.qi);
+        if (any) {
+            Op<NQ> kp[4];
+            q.k_rows<TIn>(p, startp, lenp, q.qj, kp);
+            kk = kk_quadrant<NQ>(kt, kp);
+        }
+        lds_barrier();   // the four slices of E are complete
+        {
+            f32x4 mv = {};
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const f32x4 mv = *(const f32x4*)&L.M[col * MS + 8 * q + 4 * half];
+            for (int v = 0; v < 4; ++v) {
+                const int i = q.qr + v, idx = i * MS + q.qc;
+                const bool vis = i < q.len && q.qc < lenp && (bp != q.b || (ROW ? q.qc < i : q.qc > i));
+                if (vis)
+                    mv[v] = bm * (((L.E[0][idx] + L.E[1][idx]) + (L.E[2][idx] + L.E[3][idx])) *
+                                  expf(ROW ? gt[v] - gp : gp - gt[v]));
+                sums[v] = fmaf(mv[v], kk[v] * (ft[v] * fp), sums[v]);
+                mv[v] *= v & 1 ? -fp : fp;   // times alt; 1 / |k| of the partner's row
+            }
+            put_quadrant<AR>(L.M, q.qr, q.qc, mv);
+        }
+        lds_barrier();   // M is complete, E's readers are done
+        // dk^ rows += M k_p over head dims w0 + 16 cb + c16
+        const Op<3> m0 = op_rows<3, AR>(L.M, q.c16, 0, q.g4), m1 = op_rows<3, AR>(L.M, 16 + q.c16, 0, q.g4);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) dk = mfma_f32(mv[e], L.Kp[(8 * q + 4 * half + e) * RS + 32 * wave + col], dk);
+        for (int cb = 0; cb < 2; ++cb) {
+            const TIn* kc = (const TIn*)p.k + (int64_t)startp * p.k_st + (int64_t)q.hk * p.k_sh + w0 + 16 * cb + q.c16;
+            f32x4 x[2];
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int m = 16 * tb + q.g4 + v;
+                    x[tb][v] = m < lenp ? (float)kc[(int64_t)m * p.k_st] : 0.0f;
+                }
+            const Op<NQ> kx = op_in<TIn>(x[0], x[1]);
+            dk[0][cb] += mul_planes(m0, kx, (f32x4){});
+            dk[1][cb] += mul_planes(m1, kx, (f32x4){});
         }
     }
-    const float s_row = row8_sum(s_acc);
-    __syncthreads();   // Kp readers done: it takes -beta (M k^_p) in row order
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int i = acc_row(r, half);
-        L.Kp[i * RS + 32 * wave + col] = -L.Bt[i] * dk[r];
+    for (int v = 0; v < 4; ++v) {
+        const float r = sum16(sums[v]);
+        if (q.c16 == 0) L.sum[q.qj][q.qr + v] = r;
     }
-    __syncthreads();
-    // The Y0 terms, per row: thread t owns row t/8, dims 16 (t % 8) .. +15 of v and of k.
-    {
-        const int i = t >> 3, d0 = 16 * (t & 7);
-        const bool in = i < len;
-        const int64_t tok = start + i;
-        const float bt = L.Bt[i], eg = expf(L.Gt[i]);
-        const float* dyr = a.dy0 + (chn * GC + i) * GW;
-        float vv[16];
-        if (in) load16((const TIn*)p.v + tok * p.v_st + (int64_t)h * p.v_sh + d0, vv);
-        else
 #pragma unroll
-            for (int e = 0; e < 16; ++e) vv[e] = 0.0f;
+    for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+        for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)   // E's readers passed the last barrier
+                L.J[(16 * tb + q.g4 + v) * RS + w0 + 16 * cb + q.c16] = v & 1 ? dk[tb][cb][v] : -dk[tb][cb][v];
+    lds_barrier();
+    // Per row: thread t owns row t/8, dims 16 (t % 8) .. +15 of v and of k.
+    const int i = t >> 3, d0 = 16 * (t & 7);
+    const bool in = i < q.len;
+    const int64_t tok = q.start + i;
+    const float s_row = L.sum[0][i] + L.sum[1][i];
+    float* dst = a.dkr + (q.chn * GC + i) * GD + d0;
+    if constexpr (ROW) {
+        const float bt = q.beta(p, q.start, q.len, i), eg = expf(a.rows.gn[q.chn * GC + i]);
+        const float fk = a.rows.fk[q.chn * GC + i];
+        const float* dyr = a.dy0 + (q.chn * GC + i) * GW;
+        float vv[16], kv[16];
+        if (in) {
+            load16((const TIn*)p.v + tok * p.v_st + (int64_t)q.h * p.v_sh + d0, vv);
+            load16((const TIn*)p.k + tok * p.k_st + (int64_t)q.hk * p.k_sh + d0, kv);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) vv[e] = kv[e] = 0.0f;
+        }
         float vdot = 0.0f, kdot = 0.0f;
         f32x4 dvo[4];
 #pragma unroll
         for (int e4 = 0; e4 < 4; ++e4) {
             const f32x4 dyv = *(const f32x4*)(dyr + d0 + 4 * e4);
             const f32x4 dyk = *(const f32x4*)(dyr + GD + d0 + 4 * e4);
-            const f32x4 kh = *(const f32x4*)&L.Kt[i * RS + d0 + 4 * e4];
-            f32x4 kr = *(const f32x4*)&L.Kp[i * RS + d0 + 4 * e4];
+            f32x4 kr = *(const f32x4*)&L.J[i * RS + d0 + 4 * e4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 vdot = fmaf(dyv[e], vv[4 * e4 + e], vdot);
-                kdot = fmaf(dyk[e], kh[e], kdot);
-                kr[e] = fmaf(bt * eg, dyk[e], kr[e]);
+                kdot = fmaf(dyk[e], kv[4 * e4 + e] * fk, kdot);
+                kr[e] = fmaf(bt * eg, dyk[e], bt * kr[e]);
                 dvo[e4][e] = bt * dyv[e];
             }
-            *(f32x4*)(a.dkr + (chn * GC + i) * GD + d0 + 4 * e4) = kr;
+            *(f32x4*)(dst + 4 * e4) = kr;
         }
         if (in)
 #pragma unroll
-            for (int e4 = 0; e4 < 4; ++e4) store4((TIn*)a.dv + tok * p.dv_st + h * GD + d0 + 4 * e4, dvo[e4]);
+            for (int e4 = 0; e4 < 4; ++e4) store4((TIn*)a.dv + tok * p.dv_st + q.h * GD + d0 + 4 * e4, dvo[e4]);
         vdot = row8_sum(vdot);
         kdot = row8_sum(kdot);
         if ((t & 7) == 0) {
-            if (in) a.dbeta[tok * p.hv + h] = -s_row + vdot + eg * kdot;
-            a.dgn[chn * GC + i] = in ? bt * (eg * kdot - s_row) : 0.0f;
+            if (in) a.dbeta[tok * p.hv + q.h] = -s_row + vdot + eg * kdot;
+            a.dgn[q.chn * GC + i] = in ? bt * (eg * kdot - s_row) : 0.0f;
         }
-    }
-}
-
-// ----------------------------------------------------------------------------
-// gradient of R, column side: per target block b over partners b' >= b (rows
-// of R in the partner, columns in the target)
-// ----------------------------------------------------------------------------
-template <typename TIn>
-__global__ __launch_bounds__(GT) void gdn_ecol_kernel(GdnDev p, EArgs a) {
-    __shared__ __attribute__((aligned(16))) ELds L;
-    const int c = blockIdx.x, h = blockIdx.y, t = threadIdx.x;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, col = lane & 31, half = lane >> 5;
-    int node, b, nb, start, len;
-    if (!chunk_block(p, c, node, b, nb) || !chunk_span(p, c, start, len)) return;
-    const int nstart = p.node_start[node], nlen = p.node_len[node], chunk0 = p.node_chunk0[node];
-    const size_t chn = (size_t)c * p.hv + h;
-
-    load_k_rows<TIn>(p, start, len, h, L.Kt, nullptr, nullptr);
-    load_gb(p, start, len, h, a.gn + chn * GC, L.Gt, L.Bt);
-    __syncthreads();
-    f32x4 br[16];   // this lane's row of the target's [Y0 + y1 | Y0] slice
-    {
-        const bool in = col < len;
-        const float bm = L.Bt[col], bgm = bm * expf(L.Gt[col]);
-#pragma unroll
-        for (int g = 0; g < 16; ++g) br[g] = e_operand_y<TIn>(p, a, wave, g, half, chn, col, start + col, in, h, bm, bgm, L.Kt);
-    }
-    f32x16 dk = {};
-    float cs_acc = 0.0f;   // column t/8: sum_i beta_i M (k^ . k^)
-    for (int bq = b; bq < nb; ++bq) {
-        const int cp = chunk0 + bq, startp = nstart + GC * bq, lenp = min(GC, nlen - GC * bq);
-        const size_t chp = (size_t)cp * p.hv + h;
-        __syncthreads();
-        load_k_rows<TIn>(p, startp, lenp, h, L.Kp, nullptr, nullptr);
-        load_gb(p, startp, lenp, h, a.gn + chp * GC, L.Gp, L.Bp);
-        __syncthreads();
-        {   // E[partner row][target row]
-            f32x16 ep = {};
-#pragma unroll
-            for (int g = 0; g < 16; ++g) {
-                const f32x4 f = e_operand_f(a, wave, g, half, chp, col);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) ep = mfma_f32(f[e], br[g][e], ep);
-            }
-#pragma unroll
-            for (int r = 0; r < 16; ++r) L.EP[wave * GC * MS + acc_row(r, half) * MS + col] = ep[r];
-        }
-        kk_partial(L.Kp, L.Kt, L.KP);   // [partner row][target row]
-        __syncthreads();
-        {
-            const int m = t >> 3;   // target row
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int i = (t & 7) + 8 * e;   // partner row
-                const bool vis = i < lenp && m < len && (bq > b || i > m);
-                float mv = 0.0f;
-                if (vis) mv = sum4(L.EP, i * MS + m) * expf(L.Gp[i] - L.Gt[m]);
-                cs_acc = fmaf(L.Bp[i] * mv, sum4(L.KP, i * MS + m), cs_acc);
-                L.M[m * MS + i] = mv;   // transposed: rows = target
-            }
-        }
-        __syncthreads();
-        // dk^ (rows of the target) += M^T (beta k^)_p over head dims 32 wave + col
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const f32x4 mv = *(const f32x4*)&L.M[col * MS + 8 * q + 4 * half];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int k = 8 * q + 4 * half + e;
-                dk = mfma_f32(mv[e], L.Bp[k] * L.Kp[k * RS + 32 * wave + col], dk);
-            }
-        }
-    }
-    const float cs_row = row8_sum(cs_acc);
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < 16; ++r) L.Kp[acc_row(r, half) * RS + 32 * wave + col] = -dk[r];
-    __syncthreads();
-    {
-        const int i = t >> 3, d0 = 16 * (t & 7);
-        float* dst = a.dkr + (chn * GC + i) * GD + d0;
+    } else {
 #pragma unroll
         for (int e4 = 0; e4 < 4; ++e4)
-            *(f32x4*)(dst + 4 * e4) = *(const f32x4*)(dst + 4 * e4) + *(const f32x4*)&L.Kp[i * RS + d0 + 4 * e4];
-        if ((t & 7) == 0 && i < len) a.dgn[chn * GC + i] += cs_row;
+            *(f32x4*)(dst + 4 * e4) = *(const f32x4*)(dst + 4 * e4) + *(const f32x4*)&L.J[i * RS + d0 + 4 * e4];
+        if ((t & 7) == 0 && in) a.dgn[q.chn * GC + i] += s_row;
     }
 }
 
@@ -523,26 +530,34 @@ __global__ __launch_bounds__(64) void gdn_gsuffix_kernel(GdnDev p, float* __rest
     }
 }
 
+// The workspace's node rows: gn [chunk, Hv, 32], then fk.
+NodeRows node_rows(const GdnDev& d, const float* gn) { return {gn, gn + (size_t)d.n_chunks * d.hv * GC}; }
+
 template <typename TIn>
 int trunc_fwd(const GdnDev& d, float* prep, float* gn, float* y1, hipStream_t s) {
+    const NodeRows rows = node_rows(d, gn);
+    const dim3 grid((unsigned)((size_t)d.n_chunks * d.hv));
     hipLaunchKernelGGL(gdn_gnode_kernel, dim3(d.n_nodes, d.hv), dim3(64), 0, s, d, prep, gn);
-    TriArgs a{gn, nullptr, nullptr, nullptr, nullptr, y1, prep};
-    hipLaunchKernelGGL((gdn_tri_kernel<TRI_Y1, TIn>), dim3(d.n_chunks, d.hv), dim3(GT), 0, s, d, a);
+    hipLaunchKernelGGL((gdn_y0_kernel<TIn>), grid, dim3(GT), 0, s, d, prep, gn, const_cast<float*>(rows.fk));
+    TriArgs a{rows, nullptr, nullptr, nullptr, nullptr, y1, prep};
+    hipLaunchKernelGGL((gdn_tri_kernel<TRI_Y1, TIn>), grid, dim3(GT), 0, s, d, a);
     a.xa = y1;
     a.out = nullptr;
-    hipLaunchKernelGGL((gdn_tri_kernel<TRI_UW, TIn>), dim3(d.n_chunks, d.hv), dim3(GT), 0, s, d, a);
+    hipLaunchKernelGGL((gdn_tri_kernel<TRI_UW, TIn>), grid, dim3(GT), 0, s, d, a);
     return hipGetLastError() == hipSuccess ? TT_OK : TT_E_HIP;
 }
 
 template <typename TIn>
 int trunc_bwd(const GdnDev& d, const GdnTruncBwd& w, void* dv, float* dbeta, hipStream_t s) {
-    TriArgs t1{w.gn, w.dvp, w.dw, nullptr, nullptr, w.df1, nullptr};
-    hipLaunchKernelGGL((gdn_tri_kernel<TRI_DF1, TIn>), dim3(d.n_chunks, d.hv), dim3(GT), 0, s, d, t1);
-    TriArgs t2{w.gn, w.df1, nullptr, w.dvp, w.dw, w.dy0, nullptr};
-    hipLaunchKernelGGL((gdn_tri_kernel<TRI_DY0, TIn>), dim3(d.n_chunks, d.hv), dim3(GT), 0, s, d, t2);
-    EArgs e{w.gn, w.y1, w.dvp, w.dw, w.df1, w.dy0, w.dkr, w.dgn, dv, dbeta};
-    hipLaunchKernelGGL(gdn_erow_kernel<TIn>, dim3(d.n_chunks, d.hv), dim3(GT), 0, s, d, e);
-    hipLaunchKernelGGL(gdn_ecol_kernel<TIn>, dim3(d.n_chunks, d.hv), dim3(GT), 0, s, d, e);
+    const NodeRows rows = node_rows(d, w.gn);
+    const dim3 grid((unsigned)((size_t)d.n_chunks * d.hv));
+    TriArgs t1{rows, w.dvp, w.dw, nullptr, nullptr, w.df1, nullptr};
+    hipLaunchKernelGGL((gdn_tri_kernel<TRI_DF1, TIn>), grid, dim3(GT), 0, s, d, t1);
+    TriArgs t2{rows, w.df1, nullptr, w.dvp, w.dw, w.dy0, nullptr};
+    hipLaunchKernelGGL((gdn_tri_kernel<TRI_DY0, TIn>), grid, dim3(GT), 0, s, d, t2);
+    EArgs e{rows, w.y1, w.dvp, w.dw, w.df1, w.dy0, w.dkr, w.dgn, dv, dbeta};
+    hipLaunchKernelGGL((gdn_e_kernel<TIn, true>), grid, dim3(GT), 0, s, d, e);
+    hipLaunchKernelGGL((gdn_e_kernel<TIn, false>), grid, dim3(GT), 0, s, d, e);
     hipLaunchKernelGGL(gdn_gsuffix_kernel, dim3(d.n_nodes, d.hv), dim3(64), 0, s, d, w.dgn);
     return hipGetLastError() == hipSuccess ? TT_OK : TT_E_HIP;
 }
