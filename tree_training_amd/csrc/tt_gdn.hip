@@ -969,8 +969,8 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(sizeof(TIn) 
 }  // namespace
 
 // Float counts per (chunk, v head) of the truncated mode's node-level terms:
-// the node-level decay and 1 / |k| [32] each, and R (beta [v | e^G k]) rows [32 x 256].
-constexpr size_t kTrGn = 2 * GC, kTrY1 = (size_t)GC * 2 * GD;
+// the node-level decay [32] and R (beta [v | e^G k]) rows [32 x 256].
+constexpr size_t kTrGn = GC, kTrY1 = (size_t)GC * 2 * GD;
 
 size_t tt_gdn_ws_bytes_impl(int n_chunks, int n_heads_v, bool trunc) {
     return (size_t)n_chunks * (size_t)n_heads_v * (kWsChunk + (trunc ? kTrGn + kTrY1 : 0)) * sizeof(float);
@@ -1051,7 +1051,7 @@ int tt_gdn_fwd_launch(const GdnDev& d, const int32_t* level_offsets, int n_level
 
 // The backward's float buffers. "Saved" (what the forward can keep for it):
 // per (chunk, v head) the prep terms [kWsChunk], the chunk's initial state S
-// [128 x 128] and V' [32 x 128]; TRUNC: also the node-level decay and 1 / |k| [32] each and
+// [128 x 128] and V' [32 x 128]; TRUNC: also the node-level decay [32] and
 // R-rows y1 [32 x 256]. Scratch: per (chunk, v head) dS [128 x 128], dV', X,
 // dW, dK~ [32 x 128]; TRUNC: dF1, dY0 [32 x 256], the correction's dk^
 // [32 x 128] and dG [32]; per (node, v head) dS at entry [128 x 128]; when the
@@ -1159,7 +1159,7 @@ static int gdn_bwd_run(const GdnDev& d, const int32_t* level_offsets, int n_leve
     if (hipGetLastError() != hipSuccess) return TT_E_HIP;
     if constexpr (TRUNC) {
         hipLaunchKernelGGL(gdn_dw_s0_kernel, dim3(d.n_chunks, d.hv), dim3(GT), 0, s, d, w.sin, w.dvp, w.dw);
-        const GdnTruncBwd tb{w.gn, w.y1, w.dvp, w.dw, w.df1, w.dy0, w.dkr, w.dgn};
+        const GdnTruncBwd tb{w.prep, w.gn, w.y1, w.dvp, w.dw, w.df1, w.dy0, w.dkr, w.dgn};
         const int rc = tt_gdn_trunc_bwd_launch(d, tb, dv, dbeta, s);
         if (rc != TT_OK) return rc;
     }

@@ -38,11 +38,13 @@ __device__ __forceinline__ bool chunk_block(const GdnDev& p, int c, int& node, i
     return len >= 1 && b >= 0 && b < nb && c0 >= 0 && c0 <= p.n_chunks - nb;
 }
 
-// Values of the chunk rows held per (chunk, head) beside the chunk terms: the
-// node-level decay and 1 / |k| (1 without the l2 norm).
+// Values of the chunk rows per (chunk, head): the node-level decay, and 1 / |k|
+// (1 without the l2 norm) in the chunk terms' T slot, which this mode has no
+// inverse for.
 struct NodeRows {
-    const float* gn;   // [chunk, hv, 32]
-    const float* fk;   // [chunk, hv, 32]
+    const float* gn;     // [chunk, hv, 32]
+    const float* prep;   // the chunk terms
+    __device__ __forceinline__ float fk(size_t ch, int row) const { return prep[ch * kWsChunk + kWsT + row]; }
 };
 
 // Workgroup -> (chunk, v head), heads fastest: with Hv a multiple of 8 a head
@@ -71,11 +73,10 @@ __global__ __launch_bounds__(64) void gdn_gnode_kernel(GdnDev p, const float* __
         carry += last;
     }
 }
-// fk = 1 / |k| and Y0 = [beta v | beta e^G k^] of every row, Y0 into the
-// chunk terms' U and W slots.
+// 1 / |k| (NodeRows::fk) and Y0 = [beta v | beta e^G k^] of every row, Y0 into
+// the chunk terms' U and W slots.
 template <typename TIn>
-__global__ __launch_bounds__(GT) void gdn_y0_kernel(GdnDev p, float* __restrict__ prep, const float* __restrict__ gn,
-                                                    float* __restrict__ fk) {
+__global__ __launch_bounds__(GT) void gdn_y0_kernel(GdnDev p, float* __restrict__ prep, const float* __restrict__ gn) {
     int c, h, start, len;
     chunk_head(p, c, h);
     if (!chunk_span(p, c, start, len)) return;
@@ -96,7 +97,7 @@ __global__ __launch_bounds__(GT) void gdn_y0_kernel(GdnDev p, float* __restrict_
     for (int e = 0; e < 16; ++e) sk = fmaf(kv[e], kv[e], sk);
     sk = row8_sum(sk);
     const float f = p.l2 ? 1.0f / sqrtf(sk + 1e-6f) : 1.0f, bg = bt * expf(gn[chn * GC + i]);
-    if ((t & 7) == 0) fk[chn * GC + i] = f;
+    if ((t & 7) == 0) prep[chn * kWsChunk + kWsT + i] = f;
     float* u = prep + chn * kWsChunk + kWsU + i * GD + d0;
     float* w = prep + chn * kWsChunk + kWsW + i * GD + d0;
 #pragma unroll
@@ -212,7 +213,7 @@ __global__ __launch_bounds__(GT) void gdn_tri_kernel(GdnDev p, TriArgs a) {
     for (int v = 0; v < 4; ++v) {
         const int r = q.qr + v;
         gt[v] = a.rows.gn[q.chn * GC + r];
-        ft[v] = -a.rows.fk[q.chn * GC + r] * alt(v) * (UPPER ? 1.0f : q.beta(p, q.start, q.len, r));
+        ft[v] = -a.rows.fk(q.chn, r) * alt(v) * (UPPER ? 1.0f : q.beta(p, q.start, q.len, r));
     }
     f32x4 acc[2][4] = {};
     const int bp0 = UPPER ? q.b : 0, bp1 = UPPER ? q.nb : q.b + 1;
@@ -226,7 +227,7 @@ __global__ __launch_bounds__(GT) void gdn_tri_kernel(GdnDev p, TriArgs a) {
                 Op<NQ> kp[4];
                 q.k_rows<TIn>(p, startp, lenp, q.qj, kp);
                 const float gp = a.rows.gn[chp * GC + q.qc];
-                const float fp = a.rows.fk[chp * GC + q.qc] * (UPPER ? q.beta(p, startp, lenp, q.qc) : 1.0f);
+                const float fp = a.rows.fk(chp, q.qc) * (UPPER ? q.beta(p, startp, lenp, q.qc) : 1.0f);
                 r = kk_quadrant<NQ>(kt, kp);
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
@@ -353,7 +354,7 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     // y's factor of a row: beta (times e^G / |k| in the k slices)
     auto y_factor = [&](size_t ch, int st, int n, int row) {
         float f = q.beta(p, st, n, row);
-        if (wave & 1) f *= expf(a.rows.gn[ch * GC + row]) * a.rows.fk[ch * GC + row];
+        if (wave & 1) f *= expf(a.rows.gn[ch * GC + row]) * a.rows.fk(ch, row);
         return f;
     };
     Op<3> at[2][4];
@@ -372,7 +373,7 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
         gt[v] = a.rows.gn[q.chn * GC + q.qr + v];
-        ft[v] = a.rows.fk[q.chn * GC + q.qr + v];
+        ft[v] = a.rows.fk(q.chn, q.qr + v);
     }
     f32x4 dk[2][2] = {};   // row tile, column tile w0 + 16 cb
     f32x4 sums = {};       // sum over the partners of M (k^ . k^) (column side: times beta)
@@ -399,7 +400,7 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
                 for (int v = 0; v < 4; ++v) L.E[wave][(16 * tb + q.g4 + v) * MS + row] = r[v];
             }
         }
-        const float gp = a.rows.gn[chp * GC + q.qc], fp = a.rows.fk[chp * GC + q.qc];
+        const float gp = a.rows.gn[chp * GC + q.qc], fp = a.rows.fk(chp, q.qc);
         const float bm = ROW ? 1.0f : q.beta(p, startp, lenp, q.qc);
         f32x4 kk = {};
         const bool any = bp != q.b || (ROW ? q.qi >= q.qj : q.qj >= q.qi);
@@ -463,7 +464,7 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     float* dst = a.dkr + (q.chn * GC + i) * GD + d0;
     if constexpr (ROW) {
         const float bt = q.beta(p, q.start, q.len, i), eg = expf(a.rows.gn[q.chn * GC + i]);
-        const float fk = a.rows.fk[q.chn * GC + i];
+        const float fk = a.rows.fk(q.chn, i);
         const float* dyr = a.dy0 + (q.chn * GC + i) * GW;
         float vv[16], kv[16];
         if (in) {
@@ -530,15 +531,12 @@ __global__ __launch_bounds__(64) void gdn_gsuffix_kernel(GdnDev p, float* __rest
     }
 }
 
-// The workspace's node rows: gn [chunk, Hv, 32], then fk.
-NodeRows node_rows(const GdnDev& d, const float* gn) { return {gn, gn + (size_t)d.n_chunks * d.hv * GC}; }
-
 template <typename TIn>
 int trunc_fwd(const GdnDev& d, float* prep, float* gn, float* y1, hipStream_t s) {
-    const NodeRows rows = node_rows(d, gn);
+    const NodeRows rows{gn, prep};
     const dim3 grid((unsigned)((size_t)d.n_chunks * d.hv));
     hipLaunchKernelGGL(gdn_gnode_kernel, dim3(d.n_nodes, d.hv), dim3(64), 0, s, d, prep, gn);
-    hipLaunchKernelGGL((gdn_y0_kernel<TIn>), grid, dim3(GT), 0, s, d, prep, gn, const_cast<float*>(rows.fk));
+    hipLaunchKernelGGL((gdn_y0_kernel<TIn>), grid, dim3(GT), 0, s, d, prep, gn);
     TriArgs a{rows, nullptr, nullptr, nullptr, nullptr, y1, prep};
     hipLaunchKernelGGL((gdn_tri_kernel<TRI_Y1, TIn>), grid, dim3(GT), 0, s, d, a);
     a.xa = y1;
@@ -549,7 +547,7 @@ int trunc_fwd(const GdnDev& d, float* prep, float* gn, float* y1, hipStream_t s)
 
 template <typename TIn>
 int trunc_bwd(const GdnDev& d, const GdnTruncBwd& w, void* dv, float* dbeta, hipStream_t s) {
-    const NodeRows rows = node_rows(d, w.gn);
+    const NodeRows rows{w.gn, w.prep};
     const dim3 grid((unsigned)((size_t)d.n_chunks * d.hv));
     TriArgs t1{rows, w.dvp, w.dw, nullptr, nullptr, w.df1, nullptr};
     hipLaunchKernelGGL((gdn_tri_kernel<TRI_DF1, TIn>), grid, dim3(GT), 0, s, d, t1);

@@ -147,7 +147,8 @@ int tt_gdn_bwd_launch(const GdnDev& d, const int32_t* level_offsets, int n_level
 // backward part turns dF = [dV' | dW] into dv, dbeta (complete) and the
 // correction's dk^ and node-level dG suffix sums, which the chunk backward adds.
 struct GdnTruncBwd {
-    float* gn;            // [2][chunk, Hv, 32] node-level decay, 1 / |k| (from the forward)
+    const float* prep;    // the chunk terms (from the forward)
+    float* gn;            // [chunk, Hv, 32] node-level decay (from the forward)
     float* y1;            // [chunk, Hv, 32, 256] R Y0 (from the forward)
     float* dvp;           // [chunk, Hv, 32, 128] dV'
     float* dw;            // [chunk, Hv, 32, 128] dW
