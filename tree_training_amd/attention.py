@@ -37,16 +37,17 @@ def _layout(x: torch.Tensor, tok_dim: int, head_dim: int) -> Tuple[torch.Tensor,
     if x.dim() != 4 or x.shape[0] != 1:
         raise TreeAttnError(f"expected a 4-D tensor with batch 1, got shape {tuple(x.shape)}")
 
-    def stride(t, d):
-        return t.stride(d) if t.shape[d] > 1 else t.shape[3]
+    shape, D = x.shape, x.shape[3]
 
-    def ok(t):
-        return (t.stride(3) == 1 and t.data_ptr() % 16 == 0
-                and all(stride(t, d) % 8 == 0 and stride(t, d) >= t.shape[3] for d in (tok_dim, head_dim)))
+    def strides(t):
+        s = t.stride()
+        return s[3], s[tok_dim] if shape[tok_dim] > 1 else D, s[head_dim] if shape[head_dim] > 1 else D
 
-    if not ok(x):
+    one, tok, head = strides(x)
+    if one != 1 or x.data_ptr() % 16 or tok % 8 or head % 8 or tok < D or head < D:
         x = x.contiguous()
-    return x, stride(x, tok_dim), stride(x, head_dim)
+        _, tok, head = strides(x)
+    return x, tok, head
 
 
 def _hf_view(x: torch.Tensor) -> Tuple[torch.Tensor, int, int]:
