@@ -491,6 +491,25 @@ def test_attention_fp32_step_edges(lens, par, n_past):
             check_close(name, ref, got, TOL[torch.float32])
 
 
+@pytest.mark.parametrize("deterministic", [False, True], ids=["sums", "slots"])
+@pytest.mark.parametrize("heads,lens,par,n_past", [
+    ((3, 1), [300, 40], [-1, 0], 0),                    # 33 steps a group pair: one has a step less
+    ((6, 2), [340, 1, 90], [-1, 0, 0], 131),            # split items, gateway keys, a ragged last tile
+    ((8, 1), [90, 33], [-1, 0], 0), ((1, 1), [2050], [-1], 0)])
+def test_attention_dkdv_head_pairs(monkeypatch, heads, lens, par, n_past, deterministic):
+    """bf16 dK/dV of problems with few work items, whose steps two groups of
+    waves share: odd step counts, one and several q heads a kv head, split and
+    unsplit tiles, own and gateway keys, against the fp64 oracle at the bf16 bar."""
+    monkeypatch.setattr(sys.modules[__name__], "HQ", heads[0])
+    monkeypatch.setattr(sys.modules[__name__], "HKV", heads[1])
+    past_vis = [i % 7 != 3 for i in range(n_past)] if n_past else None
+    say(f"attention dkdv head pairs {heads} lens={lens} n_past={n_past} det={deterministic}")
+    res = _run(lens, par, torch.bfloat16, seed=sum(lens), past_vis=past_vis, deterministic=deterministic)
+    for name, (ref, got) in res.items():
+        if name != "lse":
+            check_close(name, ref, got, TOL[torch.bfloat16])
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
 @pytest.mark.parametrize("shape", ["short", "split"])
 def test_attention_gateway(dtype, shape):

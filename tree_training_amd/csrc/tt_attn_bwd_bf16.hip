@@ -3,6 +3,8 @@
 // described in tt_bf16_tiles.h.
 #include "tt_bf16_tiles.h"
 
+#include <algorithm>
+
 namespace {
 
 // ----------------------------------------------------------------------------
@@ -227,9 +229,9 @@ struct KvStage {
     float ndlt[TT_BQB];    // -delta: the dP accumulators start here
 };
 
-// Staging of a 32-query block of q head h: the Q and dO rows move straight
-// from global memory into the swizzled tiles (direct loads: waves 0-1 move Q,
-// waves 2-3 dO, five 1 KB pieces of the 10 KB tile each; the pieces' buffer
+// Staging of a 32-query block of q head h by four waves: the Q and dO rows move
+// straight from global memory into the swizzled tiles (direct loads: waves 0-1
+// move Q, waves 2-3 dO, five 1 KB pieces of the 10 KB tile each; the pieces' buffer
 // offsets per lane are fixed for the kernel, the padding bytes of each row
 // take row data that nothing reads); rows past the last query read as zeros.
 // The block's lse (wave 0) and delta (wave 1) come through registers.
@@ -238,7 +240,7 @@ struct QBlockStager {
     float sv;
     int q0;
     __device__ __forceinline__ void init(const AttnDev& a, const BwdDev& bw) {
-        const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+        const int wave = (threadIdx.x >> 6) & 3, lane = threadIdx.x & 63;
         const uint32_t stb = 2u * (uint32_t)(wave < 2 ? a.q_st : bw.do_st);
 #pragma unroll
         for (int i = 0; i < 5; ++i) {
@@ -251,7 +253,7 @@ struct QBlockStager {
     // Issues the direct loads of query block q0_, q head h into stage S.
     __device__ __forceinline__ void begin(const AttnDev& a, const BwdDev& bw, int q0_, int h, KvStage& S) {
         q0 = q0_;
-        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        const int wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
         const int rows = min(TT_BQB, a.n_q - q0);
         const bool isq = wave < 2;
         const uint32_t stb = 2u * (uint32_t)(isq ? a.q_st : bw.do_st);
@@ -269,7 +271,7 @@ struct QBlockStager {
     // Completes the stage (before the barrier that publishes it). Rows past
     // the last query get -inf for -lse / scale, so they contribute nothing.
     __device__ __forceinline__ void commit(const AttnDev& a, KvStage& S) {
-        const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+        const int wave = (threadIdx.x >> 6) & 3, lane = threadIdx.x & 63;
         if (wave < 2 && lane < TT_BQB) {
             const bool in = q0 + lane < a.n_q;
             if (wave == 0) S.nlse[lane] = in ? -sv / a.scale : -INFINITY;
@@ -279,14 +281,29 @@ struct QBlockStager {
     }
 };
 
-#ifndef TT_DKDV_WAVES_PER_EU
-#define TT_DKDV_WAVES_PER_EU 2
-#endif
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TT_DKDV_WAVES_PER_EU, TT_DKDV_WAVES_PER_EU))) void bwd_dkdv_bf16_kernel(AttnDev a, BwdDev bw) {
-    __shared__ __attribute__((aligned(16))) KvStage st[2];
-    __shared__ __attribute__((aligned(16))) bf16 Vs[TT_BKB * ROW_R];   // V rows of the item's keys (row reads only)
+// NG = 2 (512 threads): two groups of four waves share an item's keys and take
+// its (query block, q head) steps in turn, each through stages of its own; at
+// the end group 0 completes dK and group 1 dV from the other's sums. An item's
+// steps are a serial chain that one wave a SIMD leaves mostly waiting; the
+// launch takes this form when the items cannot fill the chip (dkdv_launch).
+template <int NG>
+struct DkdvLds {
+    union {
+        struct {
+            KvStage st[NG][2];
+            bf16 Vs[TT_BKB * ROW_R];   // V rows of the item's keys (row reads only)
+        };
+        f32x4 sum[NG == 1 ? 1 : 2][4 * 16 * 64];   // at the end: group 1's dK, group 0's dV
+    };
+};
+template <int NG>
+__global__ __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(2, 2))) void bwd_dkdv_bf16_kernel(AttnDev a, BwdDev bw) {
+    __shared__ __attribute__((aligned(16))) DkdvLds<NG> lds;
+    bf16* const Vs = lds.Vs;
 
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int grp = NG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    KvStage* const st = lds.st[grp];
+    const int wave = (threadIdx.x >> 6) & 3, lane = threadIdx.x & 63;
     const int col = lane & 31, half = lane >> 5;
     const float c = a.scale * TT_LOG2E;
     const int n_work = (*a.n_items) * a.hkv;
@@ -320,12 +337,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TT_DKDV_WAV
         // barrier)
         const int q_top = (q_stop > q_start) ? ((q_stop - 1) / TT_BQB) * TT_BQB : 0;
         const int n_steps = (q_stop > q_start) ? ((q_top - q_start) / TT_BQB + 1) * a.rep : 0;
-        if (n_steps > 0) stg.begin(a, bw, q_top, g * a.rep, st[0]);
+        // a group's steps: its first, then every NG-th; (q0, hh) is the query
+        // block and the q head g * rep + hh of its next one
+        int q0 = q_top, hh = grp;
+        const auto settle = [&]() {
+            while (hh >= a.rep) {
+                hh -= a.rep;
+                q0 -= TT_BQB;
+            }
+        };
+        settle();
+        if (grp < n_steps) stg.begin(a, bw, q0, g * a.rep + hh, st[0]);
 
         // V rows of the tile's 128 keys go to LDS (read as MFMA operands every
         // step); K of the lane's key stays in registers. Keys past the end alias
         // the last key and are never visible.
-        {
+        if (grp == 0) {
             const int k0 = kb * TT_BKB;
             RowRegs<TT_BKB> vr;
             if (k0 + TT_BKB <= a.n_past) {
@@ -364,20 +391,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TT_DKDV_WAV
 
         // Query blocks are walked from the top of the range down, so items whose
         // ranges end at the same subtree end read the same rows at the same time.
-        // step s covers query block q0 of q head g*rep + hh; (q0, hh) of the next
-        // step are kept incrementally
-        int q0 = q_top, hh = 0;
-        for (int s = 0; s < n_steps; ++s) {
-            KvStage& S = st[s & 1];
-            stg.commit(a, S);
+        for (int s = grp, n = 0; s < n_steps + grp; s += NG, ++n) {
+            KvStage& S = st[n & 1];
+            if (NG == 1 || s < n_steps) stg.commit(a, S);
             __syncthreads();
+            if (NG > 1 && s >= n_steps) break;   // the groups' step counts differ by one at most
             const int q0_cur = q0;
-            if (++hh == a.rep) {
-                hh = 0;
-                q0 -= TT_BQB;
-            }
-            // the other stage was last read in step s - 1, which every wave has left
-            if (s + 1 < n_steps) stg.begin(a, bw, q0, g * a.rep + hh, st[(s + 1) & 1]);
+            hh += NG;
+            settle();
+            // the other stage was last read in the step before, which every wave has left
+            if (s + NG < n_steps) stg.begin(a, bw, q0, g * a.rep + hh, st[(n + 1) & 1]);
             const int q1 = min(q0_cur + TT_BQB, a.n_q);
             if (!((q0_cur < w_hi) && (q1 > w_lo))) continue;   // no key of this wave is seen here
             const bool full = w_all_vis && (w_maxlo <= q0_cur) && (w_minhi >= q1);
@@ -465,6 +488,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TT_DKDV_WAV
             }
         }
 
+        if constexpr (NG == 2) {
+            __syncthreads();   // the stages and V are done with
+            const int at = wave * 16 * 64 + lane;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const f32x16& mine = grp ? dk[i >> 2] : dv[i >> 2];
+                const int r = 4 * (i & 3);
+                lds.sum[grp ^ 1][at + 64 * i] = (f32x4){mine[r], mine[r + 1], mine[r + 2], mine[r + 3]};
+            }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const f32x4 other = lds.sum[grp][at + 64 * i];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (grp == 0) dk[i >> 2][4 * (i & 3) + e] += other[e];
+                    else dv[i >> 2][4 * (i & 3) + e] += other[e];
+                }
+            }
+        }
+        const bool out_k = NG == 1 || grp == 0, out_v = NG == 1 || grp == 1;
+
         // Epilogue: rows of dk/dv = this wave's keys, columns = d. In the
         // deterministic mode a split tile's first item stores its partial sums
         // in the fp32 rows and each later item in its own slot (`slot` above);
@@ -490,28 +535,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TT_DKDV_WAV
                 const size_t widx = ((size_t)key * a.hkv + g) * D + d;
                 if (det_split) {
                     const size_t sidx = ((size_t)(srow + key) * a.hkv + g) * D + d;
-                    sk[sidx] = gk;
-                    sv[sidx] = gv;
+                    if (out_k) sk[sidx] = gk;
+                    if (out_v) sv[sidx] = gv;
                 } else if (key < a.n_past) {   // gateway key: fp32, added to the caller's accumulators
                     if (bw.dk_acc) {
                         if (split) {
-                            atomicAdd(bw.dk_acc + widx, gk);
-                            atomicAdd(bw.dv_acc + widx, gv);
+                            if (out_k) atomicAdd(bw.dk_acc + widx, gk);
+                            if (out_v) atomicAdd(bw.dv_acc + widx, gv);
                         } else {
-                            bw.dk_acc[widx] += gk;
-                            bw.dv_acc[widx] += gv;
+                            if (out_k) bw.dk_acc[widx] += gk;
+                            if (out_v) bw.dv_acc[widx] += gv;
                         }
                     }
                 } else if (split) {
                     if (sr.ok) {
                         const size_t cidx = ((size_t)(sr.row0 + key) * a.hkv + g) * D + d;
-                        atomicAdd(bw.dk_ws + cidx, gk);
-                        atomicAdd(bw.dv_ws + cidx, gv);
+                        if (out_k) atomicAdd(bw.dk_ws + cidx, gk);
+                        if (out_v) atomicAdd(bw.dv_ws + cidx, gv);
                     }
                 } else {
                     const size_t idx = ((size_t)(key - a.n_past) * a.hkv + g) * D + d;
-                    ((bf16*)bw.dk)[idx] = (bf16)gk;
-                    ((bf16*)bw.dv)[idx] = (bf16)gv;
+                    if (out_k) ((bf16*)bw.dk)[idx] = (bf16)gk;
+                    if (out_v) ((bf16*)bw.dv)[idx] = (bf16)gv;
                 }
             }
         }
@@ -542,15 +587,36 @@ int tt_selftest_mfma_launch(const void* a, const void* b, float* d, hipStream_t 
     return hipGetLastError() == hipSuccess ? TT_OK : TT_E_HIP;
 }
 
-// Persistent grid for the dK/dV pass: a multiple of Hkv so every workgroup
-// keeps one kv head (and, with Hkv = 8, one XCD). 2048 workgroups (four per
-// resident slot) leave at most one work item per workgroup on the 16K tree,
-// so the hardware's dispatch balances the uneven items (6 % faster than 1024,
-// which pairs items statically).
-static int dkdv_grid(const AttnDev& a) {
-    const int target = 2048;
-    const int gsz = (target / a.hkv) * a.hkv;
-    return gsz > 0 ? gsz : a.hkv;
+// Upper bound on the dK/dV work items, whose count is on the device: those of a
+// chain, where key j's queries are j .. n_q - 1 (gateway keys: all).
+static int64_t dkdv_items_max(const AttnDev& a) {
+    const int qch = tt_qch(a.n_q);
+    int64_t n = 0;
+    for (int kb = 0; kb < a.n_kb; ++kb) n += tt_kb_items(std::max(0, kb * TT_BKB - a.n_past), a.n_q, qch);
+    return n * a.hkv;
+}
+
+// The dK/dV launch. Two groups of waves an item (NG = 2) when the items, at
+// most one a CU, leave half the wave slots empty: 1,072-token tree, 32/8 heads,
+// 93 -> 77 us; 2,499-token chain, 16/4 heads (160 items), 167 -> 129; 4,998-token
+// chain, 16/2 heads, 595 -> 426. From 257 to 512 items the single group's two
+// workgroups a CU do better (2,046-token chain, 32/8 heads, 320 items: 111 us
+// against 142), and so they do for items of fewer than 32 steps (47 tokens:
+// 27 us against 29).
+// Otherwise a persistent grid: a multiple of Hkv so every workgroup keeps one
+// kv head (and, with Hkv = 8, one XCD). 2048 workgroups (four per resident
+// slot) leave at most one work item per workgroup on the 16K tree, so the
+// hardware's dispatch balances the uneven items (6 % faster than 1024, which
+// pairs items statically).
+static void dkdv_launch(const AttnDev& a, const BwdDev& b, hipStream_t s) {
+    const int steps = tt_cdiv(std::min(a.n_q, tt_qch(a.n_q)), TT_BQB) * a.rep;
+    const bool few = (int64_t)a.n_kb * a.hkv <= 256;
+    const int items = few ? (int)std::min<int64_t>(dkdv_items_max(a), 2048) : 2048;
+    const dim3 grid(std::max(items / a.hkv, 1) * a.hkv);
+    if (few && items <= 256 && steps >= 32)
+        hipLaunchKernelGGL(bwd_dkdv_bf16_kernel<2>, grid, dim3(512), 0, s, a, b);
+    else
+        hipLaunchKernelGGL(bwd_dkdv_bf16_kernel<1>, grid, dim3(256), 0, s, a, b);
 }
 
 int tt_bwd_bf16_launch(const AttnDev& a, const BwdDev& b, hipStream_t s) {
@@ -579,14 +645,14 @@ int tt_bwd_bf16_launch(const AttnDev& a, const BwdDev& b, hipStream_t s) {
     }
     if (b.parts & TT_BWD_DKDV) {
         if (b.det) {
-            hipLaunchKernelGGL(bwd_dkdv_bf16_kernel, dim3(dkdv_grid(a)), dim3(256), 0, s, a, b);
+            dkdv_launch(a, b, s);
             hipLaunchKernelGGL(bwd_split_finalize_det_kernel<bf16>, dim3(a.n_kb, a.hkv), dim3(256), 0, s, a, b);
         } else {
             // split sums start at zero: cleared by the dQ pass of this call,
             // else by a launch of their own
             if (!b.zero_in_dq)
                 hipLaunchKernelGGL(bwd_split_zero_kernel, dim3(a.n_kb, a.hkv), dim3(256), 0, s, a, b);
-            hipLaunchKernelGGL(bwd_dkdv_bf16_kernel, dim3(dkdv_grid(a)), dim3(256), 0, s, a, b);
+            dkdv_launch(a, b, s);
             hipLaunchKernelGGL(bwd_split_finalize_kernel<bf16>, dim3(a.n_kb, a.hkv, 4), dim3(256), 0, s, a, b);
         }
         if (hipGetLastError() != hipSuccess) return TT_E_HIP;
