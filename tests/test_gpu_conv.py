@@ -88,6 +88,20 @@ def test_conv_bf16_matches_oracle(case):
         assert _rel(a, r) < 2e-2, (case, name, _rel(a, r))
 
 
+@pytest.mark.parametrize("T", [1, 3, 4, 5, 15, 16, 17, 19, 64, 131])
+def test_conv_fp32_run_and_batch_edges(T):
+    """Token counts at the edges of the row batches (4) and of the shortest
+    runs (16); the second topology breaks a node on every kind of edge."""
+    cut = max(1, T // 3)
+    for lens, par in (([T], [-1]), ([cut] * 2 + [T], [-1, 0, 0])):
+        x, w, b, dy = _inputs(sum(lens), 8, 4, T, True)
+        print(f"tree conv fp32 edges: lens={lens}", flush=True)
+        got = _gpu(x, w, b, dy, lens, par, torch.float32)
+        ref = _oracle(x, w, b, dy, lens, par)
+        for name, a, r in zip(("y", "dx", "dw", "db"), got, ref):
+            assert _rel(a, r) < 1e-5, (T, name, _rel(a, r))
+
+
 def test_conv_autograd_and_dropin():
     """The autograd Function's gradients equal tree_conv_backward's, and the
     reference-signature drop-in (channel-major input, a module with conv1d)

@@ -13,7 +13,9 @@
 //   gp = dy * silu'(pre),  dw[c][i] = sum_t gp[t][c] x[prev^(K-1-i)(t)][c].
 // Layout: token-major rows of C channels; each thread owns 4 channels and
 // walks a run of tokens (the predecessor chain is uniform over the workgroup).
-// Memory-bound; fp32 arithmetic.
+// fp32 arithmetic. Bound by memory where the chip is full; a run is a serial
+// walk, so its rows are loaded CB at a time, a batch ahead of the tokens being
+// computed, and small trees take shorter runs (run_tokens).
 #include "tt_common.h"
 #include "tt_internal.h"
 
@@ -21,8 +23,34 @@ namespace {
 
 constexpr int CT = 256;              // threads per workgroup
 constexpr int CCH = 4 * CT;          // channels per workgroup
-constexpr int CTOK = 64;             // tokens per workgroup (forward, dx)
-constexpr int CTOK_W = 128;          // tokens per workgroup (gp + weight-gradient partials)
+constexpr int CB = 4;                // tokens per batch of row loads
+constexpr int CTOK = 64;             // tokens per workgroup at most (forward, dx)
+constexpr int CTOK_W = 128;          // tokens per workgroup at most (gp + weight-gradient partials)
+constexpr int CTOK_MIN = 16;         // and at least
+constexpr int CONV_WGS = 1024;       // workgroups that fill the chip (four a CU)
+
+// Tokens per workgroup: halved from `most` until the workgroups fill the chip
+// (CONV_WGS). 4,096 tokens, 4,096 channels, bf16, with the batched loads: gp
+// 102 -> 27 us, dx 38 -> 18, forward 36 -> 18. Short runs read the K - 1 rows
+// before them again and write more partial sums (a run of 16: 20 % more bytes),
+// so larger trees keep the long ones (16,318 tokens, 8,192 channels: gp 169 ->
+// 152 us at 5.3 TB/s, dx and forward at that rate before and after).
+int run_tokens(int n_tokens, int n_ch, int most) {
+    int r = most;
+    while (r > CTOK_MIN && tt_cdiv(n_tokens, r) * tt_cdiv(n_ch, CCH) < CONV_WGS) r >>= 1;
+    return r;
+}
+
+// Four channels of a row as they lie in memory.
+template <typename T>
+struct Raw4 {
+    typedef T V __attribute__((ext_vector_type(4)));
+    V v;
+    __device__ __forceinline__ void load(const T* p) { v = *(const V*)p; }
+    __device__ __forceinline__ f32x4 f() const {
+        return (f32x4){(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
+    }
+};
 
 template <typename T>
 __device__ __forceinline__ f32x4 ld4(const T* p) {
@@ -81,16 +109,16 @@ __device__ __forceinline__ void load_taps(const ConvDev& p, int c, float (&w)[4]
 // run (inside a node), t's window is the last one shifted by a row, so only
 // x[t] is new; otherwise (a node's first token, the run's first) the rows
 // before it are gathered along the predecessor chain. The test is uniform over
-// the workgroup (every thread walks the same tokens). x[t] itself is passed
-// in: the callers load it one token ahead, so that a wave keeps the next
-// token's rows in flight while it computes the current one.
+// the workgroup (every thread walks the same tokens). x[t] and prev(t) are
+// passed in: the callers load them a batch ahead, so that a wave keeps the next
+// tokens' rows in flight while it computes the current ones.
 template <int K, typename T>
 struct SlidingWindow {
     int idx[K];
     f32x4 xv[K];
     int last = -1;
-    __device__ __forceinline__ void advance(const ConvDev& p, int c, int t, const f32x4& xt) {
-        if (last >= 0 && prev_of(p, t) == last) {
+    __device__ __forceinline__ void advance(const ConvDev& p, int c, int t, int prev, const f32x4& xt) {
+        if (last >= 0 && prev == last) {
 #pragma unroll
             for (int i = 0; i < K - 1; ++i) {
                 idx[i] = idx[i + 1];
@@ -117,24 +145,42 @@ struct SlidingWindow {
 };
 
 template <int K, typename T>
-__global__ __launch_bounds__(CT) void conv_fwd_kernel(ConvDev p, T* __restrict__ y, int64_t y_st) {
+__global__ __launch_bounds__(CT) void conv_fwd_kernel(ConvDev p, T* __restrict__ y, int64_t y_st, int run) {
     const int c = 4 * (blockIdx.y * CT + threadIdx.x);
     if (c >= p.n_ch) return;
     float w[4][K], b[4];
     load_taps<K, T>(p, c, w, b);
-    const int t0 = blockIdx.x * CTOK, t1 = min(p.n_tokens, t0 + CTOK);
+    const int t0 = blockIdx.x * run, t1 = min(p.n_tokens, t0 + run);   // t0 < n_tokens: the grid covers the tokens
     const T* xc = (const T*)p.x + c;
     SlidingWindow<K, T> win;
-    f32x4 xn = ld4(xc + (int64_t)t0 * p.x_st);    // t0 < n_tokens: the grid covers the tokens
-    for (int t = t0; t < t1; ++t) {
-        const f32x4 xt = xn;
-        if (t + 1 < t1) xn = ld4(xc + (int64_t)(t + 1) * p.x_st);
-        win.advance(p, c, t, xt);
-        const f32x4 z = win.preact(w, b);
-        f32x4 o;
+    Raw4<T> xn[CB];
+    int pn[CB];
+    const auto fetch = [&](int t) {   // past the run's end: its last token again
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = z[e] * sigmoid_fast(z[e]);
-        st4(y + (int64_t)t * y_st + c, o);
+        for (int j = 0; j < CB; ++j) {
+            const int u = min(t + j, t1 - 1);
+            xn[j].load(xc + (int64_t)u * p.x_st);
+            pn[j] = p.prev[u];
+        }
+    };
+    fetch(t0);
+    for (int tb = t0; tb < t1; tb += CB) {
+        Raw4<T> xr[CB];
+        int pr[CB];
+#pragma unroll
+        for (int j = 0; j < CB; ++j) { xr[j] = xn[j]; pr[j] = pn[j]; }
+        if (tb + CB < t1) fetch(tb + CB);
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+            const int t = tb + j;
+            if (t >= t1) break;
+            win.advance(p, c, t, pr[j], xr[j].f());
+            const f32x4 z = win.preact(w, b);
+            f32x4 o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = z[e] * sigmoid_fast(z[e]);
+            st4(y + (int64_t)t * y_st + c, o);
+        }
     }
 }
 
@@ -143,7 +189,7 @@ __global__ __launch_bounds__(CT) void conv_fwd_kernel(ConvDev p, T* __restrict__
 // dw (taps 0..K-1) and db (slot K): part[blockIdx.x][slot][c].
 template <int K, typename T>
 __global__ __launch_bounds__(CT) void conv_bwd_gp_kernel(ConvDev p, const T* __restrict__ dy, int64_t dy_st,
-                                                         T* __restrict__ gp, float* __restrict__ part) {
+                                                         T* __restrict__ gp, float* __restrict__ part, int run) {
     const int c = 4 * (blockIdx.y * CT + threadIdx.x);
     if (c >= p.n_ch) return;
     float w[4][K], b[4];
@@ -151,30 +197,45 @@ __global__ __launch_bounds__(CT) void conv_bwd_gp_kernel(ConvDev p, const T* __r
     f32x4 aw[K], ab = {};
 #pragma unroll
     for (int i = 0; i < K; ++i) aw[i] = (f32x4){};
-    const int t0 = blockIdx.x * CTOK_W, t1 = min(p.n_tokens, t0 + CTOK_W);
+    const int t0 = blockIdx.x * run, t1 = min(p.n_tokens, t0 + run);   // t0 < n_tokens: the grid covers the tokens
     const T* xc = (const T*)p.x + c;
     SlidingWindow<K, T> win;
-    f32x4 xn = ld4(xc + (int64_t)t0 * p.x_st);    // t0 < n_tokens: the grid covers the tokens
-    f32x4 dn = ld4(dy + (int64_t)t0 * dy_st + c);
-    for (int t = t0; t < t1; ++t) {
-        const f32x4 xt = xn, d = dn;
-        if (t + 1 < t1) {
-            xn = ld4(xc + (int64_t)(t + 1) * p.x_st);
-            dn = ld4(dy + (int64_t)(t + 1) * dy_st + c);
-        }
-        win.advance(p, c, t, xt);
-        const f32x4 z = win.preact(w, b);
-        const f32x4* xv = win.xv;
-        f32x4 g;
+    Raw4<T> xn[CB], dn[CB];
+    int pn[CB];
+    const auto fetch = [&](int t) {   // past the run's end: its last token again
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float s = sigmoid_fast(z[e]);
-            g[e] = d[e] * s * fmaf(z[e], 1.0f - s, 1.0f);
+        for (int j = 0; j < CB; ++j) {
+            const int u = min(t + j, t1 - 1);
+            xn[j].load(xc + (int64_t)u * p.x_st);
+            dn[j].load(dy + (int64_t)u * dy_st + c);
+            pn[j] = p.prev[u];
         }
-        st4(gp + (int64_t)t * p.n_ch + c, g);
-        ab += g;
+    };
+    fetch(t0);
+    for (int tb = t0; tb < t1; tb += CB) {
+        Raw4<T> xr[CB], dr[CB];
+        int pr[CB];
 #pragma unroll
-        for (int i = 0; i < K; ++i) aw[i] += g * xv[i];
+        for (int j = 0; j < CB; ++j) { xr[j] = xn[j]; dr[j] = dn[j]; pr[j] = pn[j]; }
+        if (tb + CB < t1) fetch(tb + CB);
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+            const int t = tb + j;
+            if (t >= t1) break;
+            win.advance(p, c, t, pr[j], xr[j].f());
+            const f32x4 z = win.preact(w, b), d = dr[j].f();
+            const f32x4* xv = win.xv;
+            f32x4 g;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float s = sigmoid_fast(z[e]);
+                g[e] = d[e] * s * fmaf(z[e], 1.0f - s, 1.0f);
+            }
+            st4(gp + (int64_t)t * p.n_ch + c, g);
+            ab += g;
+#pragma unroll
+            for (int i = 0; i < K; ++i) aw[i] += g * xv[i];
+        }
     }
     float* pb = part + (size_t)blockIdx.x * (K + 1) * p.n_ch + c;
 #pragma unroll
@@ -186,18 +247,18 @@ __global__ __launch_bounds__(CT) void conv_bwd_gp_kernel(ConvDev p, const T* __r
 // after u). With D_m(u) that sum (D_0(u) = gp[u]), D_m(u) = D_{m-1}(u + 1) when
 // u's one successor is u + 1 (inside a node), so the workgroup walks its tokens
 // from the last down and, for such a token, shifts the sums of the token after
-// it: one new gp row per token, loaded one token ahead. Other tokens (a node's
+// it: one new gp row per token, loaded a batch ahead. Other tokens (a node's
 // last, the range's last) walk their successor lists. Either way every sum is
 // taken in the order of the successor lists, so the results do not depend on
 // the walk.
 template <int K, typename T>
 __global__ __launch_bounds__(CT) void conv_bwd_dx_kernel(ConvDev p, const T* __restrict__ gp,
-                                                         T* __restrict__ dx) {
+                                                         T* __restrict__ dx, int run) {
     const int c = 4 * (blockIdx.y * CT + threadIdx.x);
     if (c >= p.n_ch) return;
     float w[4][K], b[4];
     load_taps<K, T>(p, c, w, b);
-    const int u0 = blockIdx.x * CTOK, u1 = min(p.n_tokens, u0 + CTOK);
+    const int u0 = blockIdx.x * run, u1 = min(p.n_tokens, u0 + run);   // u0 < u1: the grid covers the tokens
     auto g_at = [&](int t) { return ld4(gp + (int64_t)t * p.n_ch + c); };
     auto succ = [&](int t, int& lo, int& hi) {
         lo = max(p.next_off[t], 0);
@@ -205,53 +266,80 @@ __global__ __launch_bounds__(CT) void conv_bwd_dx_kernel(ConvDev p, const T* __r
     };
     f32x4 s[K];                       // D_m of the token after u (once `have`)
     bool have = false;
-    f32x4 gn = g_at(u1 - 1);          // u0 < u1: the grid covers the tokens
-    for (int u = u1 - 1; u >= u0; --u) {
-        const f32x4 gu = gn;
-        if (u > u0) gn = g_at(u - 1);
-        int lo1, hi1;
-        succ(u, lo1, hi1);
-        if (have && hi1 - lo1 == 1 && p.next[lo1] == u + 1) {
+    // gp rows and successor lists of the batch's tokens, u, u - 1, ...: the
+    // list bounds with the rows, the first successors once the bounds are there
+    Raw4<T> gn[CB];
+    int lon[CB], hin[CB], sn[CB];
+    const auto fetch = [&](int u) {   // past the run's start: its first token again
 #pragma unroll
-            for (int m = K - 1; m >= 1; --m) s[m] = s[m - 1];
-            s[0] = gu;
-        } else {
+        for (int j = 0; j < CB; ++j) {
+            const int t = max(u - j, u0);
+            gn[j].load(gp + (int64_t)t * p.n_ch + c);
+            succ(t, lon[j], hin[j]);
+        }
+    };
+    const auto fetch_first = [&]() {
 #pragma unroll
-            for (int m = 0; m < K; ++m) s[m] = (f32x4){};
-            s[0] = gu;
-            if constexpr (K > 1) {
-                for (int a = lo1; a < hi1; ++a) {
-                    const int ta = p.next[a];
-                    if (ta < 0 || ta >= p.n_tokens) continue;
-                    s[1] += g_at(ta);
-                    if constexpr (K > 2) {
-                        int lo2, hi2;
-                        succ(ta, lo2, hi2);
-                        for (int bb = lo2; bb < hi2; ++bb) {
-                            const int tb = p.next[bb];
-                            if (tb < 0 || tb >= p.n_tokens) continue;
-                            s[2] += g_at(tb);
-                            if constexpr (K > 3) {
-                                int lo3, hi3;
-                                succ(tb, lo3, hi3);
-                                for (int cc = lo3; cc < hi3; ++cc) {
-                                    const int tc = p.next[cc];
-                                    if (tc < 0 || tc >= p.n_tokens) continue;
-                                    s[3] += g_at(tc);
+        for (int j = 0; j < CB; ++j) sn[j] = hin[j] > lon[j] ? p.next[lon[j]] : -1;
+    };
+    fetch(u1 - 1);
+    fetch_first();
+    for (int ub = u1 - 1; ub >= u0; ub -= CB) {
+        Raw4<T> gr[CB];
+        int lor[CB], hir[CB], sr[CB];
+#pragma unroll
+        for (int j = 0; j < CB; ++j) { gr[j] = gn[j]; lor[j] = lon[j]; hir[j] = hin[j]; sr[j] = sn[j]; }
+        const bool more = ub - CB >= u0;
+        if (more) fetch(ub - CB);
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+            const int u = ub - j;
+            if (u < u0) break;
+            const f32x4 gu = gr[j].f();
+            const int lo1 = lor[j], hi1 = hir[j];
+            if (have && hi1 - lo1 == 1 && sr[j] == u + 1) {
+#pragma unroll
+                for (int m = K - 1; m >= 1; --m) s[m] = s[m - 1];
+                s[0] = gu;
+            } else {
+#pragma unroll
+                for (int m = 0; m < K; ++m) s[m] = (f32x4){};
+                s[0] = gu;
+                if constexpr (K > 1) {
+                    for (int a = lo1; a < hi1; ++a) {
+                        const int ta = p.next[a];
+                        if (ta < 0 || ta >= p.n_tokens) continue;
+                        s[1] += g_at(ta);
+                        if constexpr (K > 2) {
+                            int lo2, hi2;
+                            succ(ta, lo2, hi2);
+                            for (int bb = lo2; bb < hi2; ++bb) {
+                                const int tb = p.next[bb];
+                                if (tb < 0 || tb >= p.n_tokens) continue;
+                                s[2] += g_at(tb);
+                                if constexpr (K > 3) {
+                                    int lo3, hi3;
+                                    succ(tb, lo3, hi3);
+                                    for (int cc = lo3; cc < hi3; ++cc) {
+                                        const int tc = p.next[cc];
+                                        if (tc < 0 || tc >= p.n_tokens) continue;
+                                        s[3] += g_at(tc);
+                                    }
                                 }
                             }
                         }
                     }
                 }
             }
+            have = true;
+            f32x4 o = {};
+#pragma unroll
+            for (int m = 0; m < K; ++m)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = fmaf(w[e][K - 1 - m], s[m][e], o[e]);
+            st4(dx + (int64_t)u * p.n_ch + c, o);
         }
-        have = true;
-        f32x4 o = {};
-#pragma unroll
-        for (int m = 0; m < K; ++m)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = fmaf(w[e][K - 1 - m], s[m][e], o[e]);
-        st4(dx + (int64_t)u * p.n_ch + c, o);
+        if (more) fetch_first();
     }
 }
 
@@ -282,22 +370,24 @@ __global__ __launch_bounds__(CT) void conv_bwd_reduce_kernel(const float* __rest
 
 template <int K, typename T>
 int conv_fwd_run(const ConvDev& d, void* y, int64_t y_st, hipStream_t s) {
-    const dim3 grid(tt_cdiv(d.n_tokens, CTOK), tt_cdiv(d.n_ch, CCH));
-    hipLaunchKernelGGL((conv_fwd_kernel<K, T>), grid, dim3(CT), 0, s, d, (T*)y, y_st);
+    const int run = run_tokens(d.n_tokens, d.n_ch, CTOK);
+    const dim3 grid(tt_cdiv(d.n_tokens, run), tt_cdiv(d.n_ch, CCH));
+    hipLaunchKernelGGL((conv_fwd_kernel<K, T>), grid, dim3(CT), 0, s, d, (T*)y, y_st, run);
     return hipGetLastError() == hipSuccess ? TT_OK : TT_E_HIP;
 }
 
 template <int K, typename T>
 int conv_bwd_run(const ConvDev& d, const void* dy, int64_t dy_st, void* dx, float* dw, float* db, float* ws,
                  hipStream_t s) {
-    const int n_parts = tt_cdiv(d.n_tokens, CTOK_W);
+    const int run_w = run_tokens(d.n_tokens, d.n_ch, CTOK_W), run = run_tokens(d.n_tokens, d.n_ch, CTOK);
+    const int n_parts = tt_cdiv(d.n_tokens, run_w);
     T* gp = reinterpret_cast<T*>(ws);
     float* part = ws + (size_t)d.n_tokens * d.n_ch;
     hipLaunchKernelGGL((conv_bwd_gp_kernel<K, T>), dim3(n_parts, tt_cdiv(d.n_ch, CCH)), dim3(CT), 0, s, d,
-                       (const T*)dy, dy_st, gp, part);
+                       (const T*)dy, dy_st, gp, part, run_w);
     if (hipGetLastError() != hipSuccess) return TT_E_HIP;
-    hipLaunchKernelGGL((conv_bwd_dx_kernel<K, T>), dim3(tt_cdiv(d.n_tokens, CTOK), tt_cdiv(d.n_ch, CCH)), dim3(CT),
-                       0, s, d, (const T*)gp, (T*)dx);
+    hipLaunchKernelGGL((conv_bwd_dx_kernel<K, T>), dim3(tt_cdiv(d.n_tokens, run), tt_cdiv(d.n_ch, CCH)), dim3(CT),
+                       0, s, d, (const T*)gp, (T*)dx, run);
     if (hipGetLastError() != hipSuccess) return TT_E_HIP;
     hipLaunchKernelGGL(conv_bwd_reduce_kernel, dim3(tt_cdiv((K + 1) * d.n_ch, RJ)), dim3(CT), 0, s,
                        (const float*)part, n_parts, d.n_ch, K, dw, db);
@@ -330,7 +420,7 @@ int conv_bwd_k(const ConvDev& d, const void* dy, int64_t dy_st, void* dx, float*
 }  // namespace
 
 size_t tt_conv_bwd_ws_bytes_impl(int n_tokens, int n_ch, int k) {
-    const size_t parts = (size_t)tt_cdiv(n_tokens, CTOK_W);
+    const size_t parts = (size_t)tt_cdiv(n_tokens, run_tokens(n_tokens, n_ch, CTOK_W));
     return ((size_t)n_tokens * n_ch + parts * (k + 1) * n_ch) * sizeof(float);
 }
 
