@@ -46,6 +46,36 @@ def test_ce_rows_matches_torch(dtype, tol, N, V, ld):
     assert not xd[1, :V].any()                              # the ignored row's gradient is zero
 
 
+@pytest.mark.parametrize("dtype,tol,V", [
+    (torch.bfloat16, 2e-2, 32768), (torch.bfloat16, 2e-2, 32776), (torch.bfloat16, 2e-2, 65535),
+    (torch.bfloat16, 2e-2, 65544), (torch.bfloat16, 2e-2, 98311), (torch.bfloat16, 2e-2, 131080),
+    (torch.bfloat16, 2e-2, 163840), (torch.bfloat16, 2e-2, 163847), (torch.bfloat16, 2e-2, 163848),
+    (torch.float32, 1e-5, 12288), (torch.float32, 1e-5, 12292), (torch.float32, 1e-5, 16387),
+    (torch.float32, 1e-5, 81923), (torch.float32, 1e-5, 81924)])
+def test_ce_rows_register_range_edges(dtype, tol, V):
+    """Vocabularies at the edges of the rows held in registers (vectors a
+    thread, elements past the last whole vector), labels in the first and last
+    element, and a row whose first quarter is -inf (whole threads see nothing)."""
+    g = torch.Generator().manual_seed(V)
+    ld = -(-V // 8) * 8
+    x = torch.randn(4, ld, generator=g) * 3.0
+    held = V // (8 if dtype == torch.bfloat16 else 4) <= 20 * 1024 and V > 40000
+    if held:
+        x[2, :V // 4] = -float("inf")
+    labels = torch.tensor([0, V - 1, V // 2, -100])
+    scale = torch.rand(4, generator=g) + 0.5
+    xd = x.to(DEV, dtype)
+    print(f"ce_rows {dtype} V={V} ld={ld}", flush=True)
+    loss = ce_rows(xd[:, :V], labels.to(DEV), scale.to(DEV))
+    torch.cuda.synchronize()
+    ref_x = x.to(dtype)[:, :V].double().requires_grad_(True)
+    per = F.cross_entropy(ref_x, labels, ignore_index=-100, reduction="none") * scale.double()
+    (gx,) = torch.autograd.grad(per.sum(), ref_x)
+    assert _rel(loss.cpu(), per.detach()) < tol
+    assert _rel(xd[:, :V].cpu(), gx) < tol
+    assert torch.equal(xd[:, V:].cpu(), x.to(dtype)[:, V:])    # nothing past the row is written
+
+
 def test_ce_rows_bad_label_gives_nan_not_a_fault():
     x = torch.randn(2, 1000, device=DEV)
     loss = ce_rows(x, torch.tensor([5, 1000], device=DEV), torch.ones(2, device=DEV))
