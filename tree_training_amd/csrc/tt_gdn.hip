@@ -24,8 +24,8 @@
 //    independent per value column) and walks the node's chunks. Levels of
 //    one or two nodes use gdn_scan_rows_kernel instead (eight workgroups per
 //    pair, each wave a 32 x 16 slice), which gives the same bits.
-// fp32 accuracy end to end: the prep on fp32 MFMA (v_mfma_f32_32x32x2_f32) and
-// the vector ALUs, the scans (tt_gdn_scan.h) on bf16 planes of fp32 operands.
+// fp32 accuracy end to end: products on bf16 planes of fp32 operands
+// (tt_gdn_planes.h), the inverse and element-wise work on the vector ALUs.
 #include "tt_gdn_common.h"
 #include "tt_gdn_scan.h"
 
@@ -35,34 +35,105 @@ namespace {
 // ----------------------------------------------------------------------------
 // prep: per (chunk, v head) A, T, U, W, G
 // ----------------------------------------------------------------------------
-struct PrepLds {
-    float Q[GC * RS];     // q^ * scale; v once A is done
-    float K[GC * RS];
-    float R[8 * 16 * 17]; // q^ k^T at 0 and k^ k^T at GC * RR (rows of RR); then T's 16 x 16 blocks
-    float N[GC * MS];     // N = -strictly_lower(beta k^ k^T * D)
-    float Tm[GC * MS];    // I + N, then T = (I - N)^-1
-    float G[GC];
-    float Glo[GC];
-    float beta[GC];
-    float bg[GC];         // beta e^G
-};
-static_assert(2 * GC * RR <= 8 * 16 * 17, "the two 32 x 32 partial products fit the inverse's scratch");
+// bf16 problems move q and v through LDS too (coalesced rows, and 37 KB still let
+// four workgroups share a CU: 268 us against 358 for operands straight from
+// memory); in fp32 their planes would leave two (32 us against 23).
+template <typename TIn>
+constexpr bool kPrepTiles = sizeof(TIn) == 2;
 
-// q^ k^T and k^ k^T on fp32 MFMA (waves 0-1 and 2-3, each half of the
-// 128-deep contraction), the inverse T on the vector ALUs, then U and W on
-// fp32 MFMA, split by columns over the waves.
+template <typename TIn>
+struct PrepLds {
+    __bf16 K[kInPlanes<TIn> * GC * PC];           // k as it comes
+    __bf16 Q[kPrepTiles<TIn> ? GC * PC : 8];      // q as it comes; v once the products with q are done
+    float R[8 * 16 * 17];     // the 16 x 16 blocks of the inverse
+    float N[GC * MS];         // N = -strictly_lower(beta k^ k^T * D)
+    float Tm[GC * MS];        // T = (I - N)^-1
+    float G[GC], Glo[GC], beta[GC];
+    float bg[GC];             // beta e^G / |k|
+    float fq[GC], fk[GC];     // scale / |q|, 1 / |k|
+};
+
+// q k^T and k k^T (a 16 x 16 quadrant a wave, the upper one not read), U and W
+// (32 columns a wave) on planes, the norms and decays as factors of rows and
+// columns; the inverse T on the vector ALUs. A chain of a dozen barriers, so
+// latency bounds the kernel. 16K agent tree, 32 v heads, bf16: 384 us on fp32
+// MFMAs (three workgroups a CU) -> 268; fp32, 2,111 tokens, 8 v heads: 23 us both.
 // TRUNC (the reference's per-node correction): only A and G here; U and W
 // come from the node-level kernels of tt_gdn_trunc.hip.
 template <typename TIn, bool TRUNC>
 __global__ __launch_bounds__(GT) void gdn_prep_kernel(GdnDev p, float* __restrict__ ws) {
-    __shared__ __attribute__((aligned(16))) PrepLds L;
+    constexpr int NQ = kInPlanes<TIn>;
+    __shared__ __attribute__((aligned(16))) PrepLds<TIn> L;
     const int c = blockIdx.x, h = blockIdx.y;
-    const int t = threadIdx.x, wave = t >> 6, lane = t & 63, col = lane & 31, half = lane >> 5;
+    const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
+    const int c16 = lane & 15, g4 = 4 * (lane >> 4);
     int start, len;
     if (!chunk_span(p, c, start, len)) return;
     float* out = ws + ((size_t)c * p.hv + h) * kWsChunk;
 
-    load_chunk_rows<TIn>(p, start, len, h, L.Q, L.K, nullptr);
+    const int qi = wave >> 1, qj = wave & 1;            // this wave's quadrant
+    const int qr = 16 * qi + g4, qc = 16 * qj + c16;    // this lane's first row and its column there
+    const int w0 = 32 * wave;                           // this wave's columns of U and W
+    constexpr bool TILES = kPrepTiles<TIn>;
+    using Vec = typename std::conditional<sizeof(TIn) == 2, bf16x8, f32x4>::type;
+    constexpr int NV = (int)sizeof(TIn);
+    const int i8 = t >> 3, d8 = 16 * (t & 7);           // this thread's row and its first dim there
+    Vec vv[NV];        // TILES: that part of v
+    Op<NQ> qop[4];     // else: q rows of the quadrant's row tile
+    f32x4 vx[2][2];    // and v columns w0 + 16 cb + c16, rows 16 tb + g4 .. +3
+    {
+        const int hk = h / p.rep;
+        const auto row16 = [&](const void* x, int64_t st, int64_t off, Vec (&r)[NV]) {
+            const TIn* xp = (const TIn*)x + (int64_t)(start + i8) * st + off + d8;
+#pragma unroll
+            for (int n = 0; n < NV; ++n) {
+                if (i8 < len) {
+                    r[n] = *(const Vec*)(xp + 16 / NV * n);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 16 / NV; ++e) r[n][e] = (TIn)0.0f;
+                }
+            }
+        };
+        Vec kv[NV], qv[NV];
+        row16(p.k, p.k_st, hk * p.k_sh, kv);
+        if constexpr (TILES) {
+            row16(p.q, p.q_st, hk * p.q_sh, qv);
+            if constexpr (!TRUNC) row16(p.v, p.v_st, h * p.v_sh, vv);
+            put16<PC>(L.Q, i8, d8, qv);
+            const float nq = row_norm(p, qv);
+            if ((t & 7) == 0) L.fq[i8] = nq * p.scale;
+        } else if (qi >= qj) {
+            const int row = 16 * qi + c16;
+            const TIn* qp = (const TIn*)p.q + (int64_t)(start + row) * p.q_st + (int64_t)hk * p.q_sh + g4;
+            float ss = 0.0f;
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                const f32x4 x0 = row < len ? load4(qp + 32 * m) : (f32x4){};
+                const f32x4 x1 = row < len ? load4(qp + 32 * m + 16) : (f32x4){};
+                ss += dot4(x0, x0) + dot4(x1, x1);
+                qop[m] = op_in<TIn>(x0, x1);
+            }
+            ss += __shfl_xor(ss, 16);
+            ss += __shfl_xor(ss, 32);
+            if (qj == 0 && lane < 16) L.fq[row] = (p.l2 ? 1.0f / sqrtf(ss + 1e-6f) : 1.0f) * p.scale;
+        }
+        if constexpr (!TRUNC && !TILES) {
+            const TIn* vp = (const TIn*)p.v + (int64_t)start * p.v_st + (int64_t)h * p.v_sh + w0 + c16;
+#pragma unroll
+            for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+                for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const int m = 16 * tb + g4 + v;
+                        vx[cb][tb][v] = m < len ? (float)vp[(int64_t)m * p.v_st + 16 * cb] : 0.0f;
+                    }
+        }
+        put16<PC>(L.K, i8, d8, kv);
+        const float nk = row_norm(p, kv);
+        if ((t & 7) == 0) L.fk[i8] = nk;
+    }
     if (wave == 0) {
         // cumulative decay over the chunk (lanes 0..31; padded rows add 0),
         // each step's rounding error (two-sum) carried in lo
@@ -83,44 +154,52 @@ __global__ __launch_bounds__(GT) void gdn_prep_kernel(GdnDev p, float* __restric
             L.G[lane] = gv;
             L.Glo[lane] = lo;
             L.beta[lane] = bv;
-            L.bg[lane] = bv * expf(gv + lo);
             out[kWsG + lane] = gv;
             out[kWsGlo + lane] = lo;
         }
     }
-    __syncthreads();
-    {   // the odd wave of each pair stores its half of the contraction, the
-        // even one adds its own in place (two 32 x 32 buffers, not four)
-        const float* X = wave < 2 ? L.Q : L.K;
-        const int q0 = 2 * (wave & 1);
-        f32x16 acc = quarter_nt(X, L.K, 1.0f, col, half, q0, (f32x16){});
-        acc = quarter_nt(X, L.K, 1.0f, col, half, q0 + 1, acc);
-        float* Rw = L.R + (wave >> 1) * GC * RR;
-        if (wave & 1) put_partial(Rw, acc, col, half);
-        __syncthreads();
-        if constexpr (!TRUNC)   // Q's readers are done
-            tile_in((const TIn*)p.v + (int64_t)start * p.v_st + (int64_t)h * p.v_sh, p.v_st, len, L.Q);
-        if (!(wave & 1)) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) Rw[acc_row(r, half) * RR + col] += acc[r];
-        }
-    }
-    __syncthreads();
+    lds_barrier();
 
-    // A = lower_incl(q^ k^T * D), N = -strictly_lower(beta k^ k^T * D).
+    // A = lower_incl(q^ k^T * D), N = -strictly_lower(beta k^ k^T * D); the
+    // diagonal quadrants of N also start the inverse (below).
+    constexpr int BS = 17;                                   // row stride of the 16 x 16 blocks
+    constexpr int B16 = 16 * BS;
+    float* sc = L.R;
+    {
+        f32x4 qk = {}, kk = {};
+        if (qi >= qj) {
+            Sum2 x, y;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int pi = t + GT * u, i = pi >> 5, j = pi & 31;
-        const float dqk = L.R[i * RR + j];
-        const float dkk = L.R[GC * RR + i * RR + j];
-        const float dec = j <= i ? expf(gdiff(L.G[i], L.Glo[i], L.G[j], L.Glo[j])) : 0.0f;
-        const float nij = j < i ? -L.beta[i] * dkk * dec : 0.0f;
-        out[kWsA + i * GC + j] = dqk * dec;
-        L.N[i * MS + j] = nij;
-        L.Tm[i * MS + j] = nij + (i == j ? 1.0f : 0.0f);
+            for (int m = 0; m < 4; ++m) {
+                const Op<NQ> kj = op_rows<NQ, PC>(L.K, 16 * qj + c16, 32 * m, g4);
+                if constexpr (TILES) x.add(op_rows<NQ, PC>(L.Q, 16 * qi + c16, 32 * m, g4), kj);
+                else x.add(qop[m], kj);
+                if constexpr (!TRUNC) y.add(op_rows<NQ, PC>(L.K, 16 * qi + c16, 32 * m, g4), kj);
+            }
+            qk = x.sum();
+            kk = y.sum();
+        }
+        const float gj = L.G[qc], glj = L.Glo[qc], fkj = L.fk[qc];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int i = qr + v;
+            const float dec = qc <= i ? expf(gdiff(L.G[i], L.Glo[i], gj, glj)) : 0.0f;
+            out[kWsA + i * GC + qc] = qc <= i ? qk[v] * (L.fq[i] * fkj) * dec : 0.0f;
+            if constexpr (!TRUNC) {
+                const float n = qc < i ? -L.beta[i] * (kk[v] * (L.fk[i] * fkj)) * dec : 0.0f;
+                L.N[i * MS + qc] = n;
+                if (qi == qj) {
+                    float* b = sc + qi * 4 * B16 + (g4 + v) * BS + c16;
+                    b[0] = n;
+                    b[2 * B16] = n + (qc == i ? 1.0f : 0.0f);
+                }
+            }
+        }
+        if (!TRUNC && t < GC) L.bg[t] = L.beta[t] * expf(L.G[t] + L.Glo[t]) * L.fk[t];
     }
     if constexpr (TRUNC) return;
-    __syncthreads();
+    lds_barrier();   // N complete, q's readers are done
+    if constexpr (TILES) put16<PC>(L.Q, i8, d8, vv);
 
     // T = (I - N)^-1 by 16 x 16 blocks. With N = [[N11, 0], [N21, N22]],
     // T = [[T11, 0], [T22 N21 T11, T22]] and, each Nbb strictly lower
@@ -131,20 +210,9 @@ __global__ __launch_bounds__(GT) void gdn_prep_kernel(GdnDev p, float* __restric
     // buffer R (free again); then X = N21 T11 and T21 = T22 X, a thread an
     // entry. A quarter of the work of squaring the whole 32 x 32 matrix.
     {
-        constexpr int BS = 17;                                   // row stride of the 16 x 16 blocks
-        constexpr int B16 = 16 * BS;
-        float* sc = L.R;
         const int blk = t >> 7, u = t & 127, bi = u >> 3, bj = 2 * (u & 7), o = 16 * blk;
         // block blk: P buffers at pb, pb + B16; T buffers at pb + 2 B16, pb + 3 B16
         const int pb = blk * 4 * B16, tb = pb + 2 * B16;
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const int j = bj + e;
-            const float n = L.N[(o + bi) * MS + o + j];
-            sc[pb + bi * BS + j] = n;
-            sc[tb + bi * BS + j] = n + (bi == j ? 1.0f : 0.0f);
-        }
-        __syncthreads();
 #pragma unroll
         for (int r = 0; r < 3; ++r) {
             const int pc = pb + (r & 1) * B16, pn = pb + ((r + 1) & 1) * B16;
@@ -193,24 +261,35 @@ __global__ __launch_bounds__(GT) void gdn_prep_kernel(GdnDev p, float* __restric
         *(f32x4*)(out + kWsT + ti * GC + tc) = *(const f32x4*)&L.Tm[ti * MS + tc];
     }
 
-    // U = T (beta v), W = T (beta e^G k^): wave w produces columns 32w .. 32w+31.
+    // U = T (beta v), W = T (beta e^G k^): wave w produces columns 32w .. 32w+31,
+    // the odd rows formed negated (alt).
     {
-        const int cw0 = 32 * wave;
-        f32x16 u = {}, w = {};
+        Op<3> tu[2], tw[2];   // rows of T, its columns times beta and beta e^G / |k|
+        const f32x4 b0 = *(const f32x4*)&L.beta[g4], b1 = *(const f32x4*)&L.beta[16 + g4];
+        const f32x4 e0 = *(const f32x4*)&L.bg[g4], e1 = *(const f32x4*)&L.bg[16 + g4];
 #pragma unroll
-        for (int m = 0; m < 4; ++m) {
-            const f32x4 a = op_row4(L.Tm, MS, col, half, 0, m);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int r = 4 * m + e, k = acc_row(r, half);
-                u = mfma_f32(a[e], L.beta[k] * L.Q[k * RS + cw0 + col], u);
-                w = mfma_f32(a[e], L.bg[k] * L.K[k * RS + cw0 + col], w);
-            }
+        for (int tb = 0; tb < 2; ++tb) {
+            const float* row = &L.Tm[(16 * tb + c16) * MS + g4];
+            const f32x4 x0 = alt(c16) * *(const f32x4*)row, x1 = alt(c16) * *(const f32x4*)(row + 16);
+            tu[tb] = op_acc(x0 * b0, x1 * b1);
+            tw[tb] = op_acc(x0 * e0, x1 * e1);
         }
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            out[kWsU + acc_row(r, half) * GD + cw0 + col] = u[r];
-            out[kWsW + acc_row(r, half) * GD + cw0 + col] = w[r];
+        for (int cb = 0; cb < 2; ++cb) {
+            const Op<NQ> kc = op_cols<NQ, PC>(L.K, w0 + 16 * cb, lane);
+            Op<NQ> vc;
+            if constexpr (TILES) vc = op_cols<NQ, PC>(L.Q, w0 + 16 * cb, lane);
+            else vc = op_in<TIn>(vx[cb][0], vx[cb][1]);
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb) {
+                const f32x4 u = mul_planes(tu[tb], vc, (f32x4){}), w = mul_planes(tw[tb], kc, (f32x4){});
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int o = (16 * tb + g4 + v) * GD + w0 + 16 * cb + c16;
+                    out[kWsU + o] = v & 1 ? -u[v] : u[v];
+                    out[kWsW + o] = v & 1 ? -w[v] : w[v];
+                }
+            }
         }
     }
 }

@@ -13,7 +13,6 @@ constexpr int GC = TT_GDN_CHUNK;  // chunk length (32)
 constexpr int GT = 256;           // threads per workgroup
 constexpr int RS = GD + 4;        // row stride of [GC x GD] tiles (floats): rows 4 banks apart
 constexpr int MS = GC + 4;        // row stride of [GC x GC] matrices
-constexpr int RR = GC + 1;        // row stride of per-wave 32 x 32 partial products
 
 // Workspace per (chunk, v head), floats: W [GC][GD], U [GC][GD], A [GC][GC],
 // T [GC][GC] (the inverse, for the backward), G [GC] and its low part Glo [GC].
@@ -82,41 +81,6 @@ __device__ __forceinline__ bool chunk_span(const GdnDev& p, int c, int& start, i
     return true;
 }
 
-// Rows of one chunk (zeros past its length): l2-normalised q (times scale),
-// k, and, when V is given, v; thread t handles row t/8, 16 dims.
-template <typename TIn>
-__device__ __forceinline__ void load_chunk_rows(const GdnDev& p, int start, int len, int h, float* Q, float* K,
-                                                float* V) {
-    const int t = threadIdx.x, i = t >> 3, d0 = 16 * (t & 7), hk = h / p.rep;
-    const bool valid = i < len;
-    const int64_t tok = start + i;
-    float qv[16], kv[16], vv[16];
-    if (valid) {
-        load16((const TIn*)p.q + tok * p.q_st + hk * p.q_sh + d0, qv);
-        load16((const TIn*)p.k + tok * p.k_st + hk * p.k_sh + d0, kv);
-        if (V) load16((const TIn*)p.v + tok * p.v_st + h * p.v_sh + d0, vv);
-    } else {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) qv[e] = kv[e] = vv[e] = 0.0f;
-    }
-    float sq = 0.0f, sk = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-        sq = fmaf(qv[e], qv[e], sq);
-        sk = fmaf(kv[e], kv[e], sk);
-    }
-    sq = row8_sum(sq);
-    sk = row8_sum(sk);
-    const float fq = (p.l2 ? 1.0f / sqrtf(sq + 1e-6f) : 1.0f) * p.scale;
-    const float fk = p.l2 ? 1.0f / sqrtf(sk + 1e-6f) : 1.0f;
-#pragma unroll
-    for (int e = 0; e < 16; e += 4) {
-        *(f32x4*)&Q[i * RS + d0 + e] = (f32x4){qv[e] * fq, qv[e + 1] * fq, qv[e + 2] * fq, qv[e + 3] * fq};
-        *(f32x4*)&K[i * RS + d0 + e] = (f32x4){kv[e] * fk, kv[e + 1] * fk, kv[e + 2] * fk, kv[e + 3] * fk};
-        if (V) *(f32x4*)&V[i * RS + d0 + e] = (f32x4){vv[e], vv[e + 1], vv[e + 2], vv[e + 3]};
-    }
-}
-
 // v_mfma_f32_32x32x2_f32: D[32x32] += A[32x2] B[2x32]; lane l supplies
 // A[l & 31][l >> 5] and B[l >> 5][l & 31], and accumulator element r of lane l
 // is D[acc_row(r, l >> 5)][l & 31]. The contraction order is free, so step r
@@ -175,46 +139,6 @@ __device__ __forceinline__ f32x4 load4(const T* p) {
 
 __device__ __forceinline__ float dot4(const f32x4& a, const f32x4& b) {
     return fmaf(a[0], b[0], fmaf(a[1], b[1], fmaf(a[2], b[2], a[3] * b[3])));
-}
-
-// Rows of a [GC x GD] tile into LDS (stride RS): thread t copies row t/8,
-// dims 16*(t%8)..+15; rows at or past `len` are zero.
-template <typename T>
-__device__ __forceinline__ void tile_in(const T* base, int64_t row_stride, int len, float* dst) {
-    const int i = threadIdx.x >> 3, d0 = 16 * (threadIdx.x & 7);
-    float x[16];
-    if (i < len) {
-        load16(base + i * row_stride + d0, x);
-    } else {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) x[e] = 0.0f;
-    }
-#pragma unroll
-    for (int e = 0; e < 16; e += 4) *(f32x4*)&dst[i * RS + d0 + e] = (f32x4){x[e], x[e + 1], x[e + 2], x[e + 3]};
-}
-
-// fp32 MFMA operands from LDS, in the k order of mfma_f32 (step r pairs
-// k = acc_row(r, 0) on lanes 0-31 with k = acc_row(r, 1) on lanes 32-63).
-// Row operand X[col][kb + k]: four steps per 16-byte read.
-__device__ __forceinline__ f32x4 op_row4(const float* X, int stride, int col, int half, int kb, int m) {
-    return *(const f32x4*)&X[col * stride + kb + 8 * m + 4 * half];
-}
-// 32 x 32 partial product over this wave's quarter of a 128-deep contraction:
-// D[i][j] = sum_k A[i][k] B[j][k] (both read as rows), B scaled by bs (a
-// per-column factor), added to acc.
-__device__ __forceinline__ f32x16 quarter_nt(const float* A, const float* B, float bs, int col, int half, int wave,
-                                             f32x16 acc) {
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        const f32x4 a = op_row4(A, RS, col, half, 32 * wave, m), b = op_row4(B, RS, col, half, 32 * wave, m);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc = mfma_f32(a[e], b[e] * bs, acc);
-    }
-    return acc;
-}
-__device__ __forceinline__ void put_partial(float* R, const f32x16& acc, int col, int half) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) R[acc_row(r, half) * RR + col] = acc[r];
 }
 
 }  // namespace
