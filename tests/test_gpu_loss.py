@@ -105,6 +105,27 @@ def test_fused_linear_ce_matches_torch(dtype, tol):
     assert _rel(wd.grad.cpu(), wr.grad) < tol
 
 
+def test_fused_linear_ce_autocast_adds_apart():
+    """float32 tensors under bf16 autocast, three chunks: the weight gradient's
+    GEMM result and the sum differ in type, so they are added separately. Bar:
+    the bf16 one of the test above (logits and GEMM operands are rounded to it)."""
+    g = torch.Generator().manual_seed(1)
+    N, H, V = 300, 256, 1000
+    h, w = torch.randn(N, H, generator=g), torch.randn(V, H, generator=g) * 0.05
+    labels = torch.randint(0, V, (N,), generator=g)
+    scale = torch.full((N,), 1.0 / 7.0)
+    hd, wd = h.to(DEV).requires_grad_(True), w.to(DEV).requires_grad_(True)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        loss = fused_linear_ce(hd, wd, labels.to(DEV), scale.to(DEV), chunk=128)
+    loss.backward()
+    hr, wr = h.double().requires_grad_(True), w.double().requires_grad_(True)
+    ref = (F.cross_entropy(hr @ wr.t(), labels, reduction="none") * scale.double()).sum()
+    ref.backward()
+    assert _rel(loss.detach().cpu(), ref.detach()) < 2e-2
+    assert _rel(hd.grad.cpu(), hr.grad) < 2e-2
+    assert _rel(wd.grad.cpu(), wr.grad) < 2e-2
+
+
 @pytest.mark.parametrize("driver", ["sequential", "hybrid"])
 def test_drivers_fused_leaf_ce_fp32(driver):
     """make_tree_loss_fn losses take the hidden-state path (no [T, V] logits)
