@@ -54,14 +54,13 @@ def test_ce_rows_matches_torch(dtype, tol, N, V, ld):
     (torch.float32, 1e-5, 81923), (torch.float32, 1e-5, 81924)])
 def test_ce_rows_register_range_edges(dtype, tol, V):
     """Vocabularies at the edges of the rows held in registers (vectors a
-    thread, elements past the last whole vector), labels in the first and last
-    element, and a row whose first quarter is -inf (whole threads see nothing)."""
+    thread, elements past the last whole vector) and one step outside them,
+    labels in the first and last element, and a row whose first quarter is -inf
+    (whole threads see nothing)."""
     g = torch.Generator().manual_seed(V)
     ld = -(-V // 8) * 8
     x = torch.randn(4, ld, generator=g) * 3.0
-    held = V // (8 if dtype == torch.bfloat16 else 4) <= 20 * 1024 and V > 40000
-    if held:
-        x[2, :V // 4] = -float("inf")
+    x[2, :V // 4] = -float("inf")
     labels = torch.tensor([0, V - 1, V // 2, -100])
     scale = torch.rand(4, generator=g) + 0.5
     xd = x.to(DEV, dtype)
@@ -74,6 +73,40 @@ def test_ce_rows_register_range_edges(dtype, tol, V):
     assert _rel(loss.cpu(), per.detach()) < tol
     assert _rel(xd[:, :V].cpu(), gx) < tol
     assert torch.equal(xd[:, V:].cpu(), x.to(dtype)[:, V:])    # nothing past the row is written
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-5), (torch.bfloat16, 2e-2)])
+@pytest.mark.parametrize("V", [40, 1001, 20000, 65544, 163848])
+def test_ce_rows_masked_logits(dtype, tol, V):
+    """Vocabulary masks of -inf (a masked tail, a masked head, every second
+    group of 8, all but the label) give torch's loss and gradient on both routes
+    (rows in registers, two passes); a NaN among masked logits, or a row with
+    nothing but -inf, gives a NaN loss, and its neighbours keep theirs."""
+    inf = float("inf")
+    g = torch.Generator().manual_seed(V)
+    ld = -(-V // 8) * 8
+    x = torch.randn(8, ld, generator=g) * 3.0
+    x[0, V - V // 4:V] = -inf
+    x[1, :V // 2] = -inf
+    x[2, :V] = torch.where(torch.arange(V) // 8 % 2 == 1, -inf, x[2, :V])
+    x[3, :V] = -inf
+    labels = torch.tensor([3, V - 1, 0, V // 2, 5, 1, 2, 4])
+    x[3, labels[3]] = 1.5
+    x[4, :V] = -inf                          # nothing to choose from
+    x[5, :V] = -inf
+    x[5, 17], x[5, V - 1] = float("nan"), 0.5
+    x[6, V - 3], x[6, :8] = float("nan"), -inf
+    scale = torch.rand(8, generator=g) + 0.5
+    xd = x.to(DEV, dtype)
+    print(f"ce_rows masked {dtype} V={V}", flush=True)
+    loss = ce_rows(xd[:, :V], labels.to(DEV), scale.to(DEV)).cpu()
+    ref_x = x.to(dtype)[:, :V].double().requires_grad_(True)
+    per = F.cross_entropy(ref_x, labels, reduction="none") * scale.double()
+    (gx,) = torch.autograd.grad(per.sum(), ref_x)
+    assert torch.equal(torch.isnan(loss), torch.isnan(per)), (loss, per)
+    for r in (0, 1, 2, 3, 7):
+        assert abs(loss[r].double() - per[r]).item() <= tol * max(1.0, per[r].item()), (r, loss[r], per[r])
+        assert _rel(xd[r, :V].cpu(), gx[r]) < tol or not gx[r].any() and not xd[r, :V].any(), r
 
 
 def test_ce_rows_bad_label_gives_nan_not_a_fault():

@@ -45,10 +45,14 @@ __device__ __forceinline__ void ce_st8(T* p, const float (&x)[8]) {
     }
 }
 
-// (m, s) <- merge of two online-softmax partials (s relative to m).
+// (m, s) <- merge of two online-softmax partials (s relative to m). Without a
+// logit above -inf on either side the sums are zero, or a NaN that must stay.
 __device__ __forceinline__ void merge_ms(float& m, float& s, float m2, float s2) {
     const float mn = fmaxf(m, m2);
-    if (mn == -INFINITY) return;
+    if (mn == -INFINITY) {
+        s += s2;
+        return;
+    }
     s = s * exp2f((m - mn) * TT_LOG2E) + s2 * exp2f((m2 - mn) * TT_LOG2E);
     m = mn;
 }
@@ -76,12 +80,17 @@ __global__ __launch_bounds__(CE_T) void ce_rows_kernel(const T* logits, int64_t 
         float m8 = v[0];
 #pragma unroll
         for (int e = 1; e < 8; ++e) m8 = fmaxf(m8, v[e]);
+        // a group of nothing but -inf (a masked vocabulary) adds exp(-inf) = 0, not exp(-inf + inf)
+        const float ms = m8 == -INFINITY ? 0.0f : m8;
         float s8 = 0.0f;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) s8 += exp2f((v[e] - m8) * TT_LOG2E);
+        for (int e = 0; e < 8; ++e) s8 += exp2f((v[e] - ms) * TT_LOG2E);
         merge_ms(m, s, m8, s8);
     }
-    for (int j = v8 + tid; j < V; j += CE_T) merge_ms(m, s, (float)x[j], 1.0f);
+    for (int j = v8 + tid; j < V; j += CE_T) {
+        const float vj = (float)x[j], mj = vj == -INFINITY ? 0.0f : vj;
+        merge_ms(m, s, vj, exp2f((vj - mj) * TT_LOG2E));   // as a group of one
+    }
     // wave, then workgroup
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
