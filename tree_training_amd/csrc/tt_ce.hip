@@ -6,9 +6,9 @@
 //   loss[r] = c (lse - x_y),   grad[r][j] = c (exp(x_j - lse) - [j == y]);
 // a row whose label is ignore_index gets loss 0 and a zero gradient. grad may
 // alias the logits (each element is read before the same thread writes it).
-// One workgroup per row. Rows of 64 to 320 KB are held in registers (2 x row
-// bytes of HBM traffic); others take an online max/sum pass, then the gradient
-// pass (3 x row bytes). fp32 arithmetic.
+// One workgroup per row. Rows of 64 (fp32: 48) to 320 KB are held in registers
+// (2 x row bytes of HBM traffic); others take an online max/sum pass, then the
+// gradient pass (3 x row bytes). fp32 arithmetic.
 #include "tt_common.h"
 #include "tt_internal.h"
 
@@ -222,9 +222,12 @@ __global__ __launch_bounds__(CE_TR) void ce_rows_reg_kernel(const T* logits, int
 
 // The register kernel where it is the faster one: from more than 4 vectors a
 // thread in bf16, 4 in fp32, to the 20 that leave its 16 waves a CU. 4,096 rows,
-// two-pass against registers (us): bf16 vocab 32,000 122 / 135, 50,304 228 / 179,
-// 65,536 304 / 213, 128,256 648 / 438, 151,936 759 / 539 (4.6 TB/s); fp32 8,192
-// 59 / 78, 16,384 119 / 90, 32,000 288 / 204, 65,536 630 / 414.
+// two-pass against registers (us): bf16 vocab 32,000 122 / 135, 32,776 130 / 125,
+// 40,960 161 / 142, 50,304 230 / 173, 65,536 304 / 213, 128,256 648 / 438,
+// 151,936 759 / 539 (4.6 TB/s); fp32 8,192 59 / 78, 12,292 91 / 82, 16,384
+// 119 / 90, 32,000 288 / 204, 65,536 630 / 414. Five vectors have an instance of
+// their own: in that of eight their three empty ones cost more than the second
+// read (vocab 32,776: 145 us).
 template <typename T>
 void ce_launch(const void* logits, int64_t ld, int n_rows, int vocab, const int32_t* labels, const float* row_scale,
                int ignore_index, float* loss, void* grad, int64_t ldg, hipStream_t s) {
@@ -238,7 +241,8 @@ void ce_launch(const void* logits, int64_t ld, int n_rows, int vocab, const int3
     else if (nv > 16) CE_REG(20);
     else if (nv > 12) CE_REG(16);
     else if (nv > 8) CE_REG(12);
-    else if (nv > 4) CE_REG(8);
+    else if (nv > 5) CE_REG(8);
+    else if (nv > 4) CE_REG(5);
     else if (nv > 3 && sizeof(T) == 4) CE_REG(4);
     else
         hipLaunchKernelGGL(ce_rows_kernel<T>, dim3(n_rows), dim3(CE_T), 0, s, (const T*)logits, ld, vocab, labels,
