@@ -46,6 +46,26 @@ def test_mfma_layout_selftest():
 
 
 # --------------------------------------------------------------------------- metadata
+def test_trees_under_a_default_device():
+    """A program that sets the GPU as torch's default device builds the same
+    trees and plans: topologies are staged in (pinned) host memory all the same."""
+    from tree_training_amd.gdn import GdnTree
+    from tree_training_amd.meta import KeyPlan, build_trees
+    lens, par = [33, 4, 150, 7], [-1, 0, 0, 2]
+    m = _meta(lens, par)
+    kp = KeyPlan(m.horizon)
+    say("trees under a default device")
+    with torch.device(DEV):
+        got = [(_meta(lens, par), None), *build_trees([(lens, par, 0, None)], DEV)]
+        got[0] = (got[0][0], KeyPlan(got[0][0].horizon))
+        links = GdnTree(lens, par, torch.device(DEV)).token_links()
+    for a, plan in got:
+        assert torch.equal(a.pos, m.pos) and torch.equal(a.horizon, m.horizon)
+        assert torch.equal(plan.key_lo, kp.key_lo) and torch.equal(plan.key_hi, kp.key_hi)
+    for a, b in zip(links, GdnTree(lens, par, torch.device(DEV)).token_links()):
+        assert torch.equal(a, b)
+
+
 def test_meta_c1_fixture():
     spec = load_golden("c1_tree.json")
     lens = [n["len"] for n in spec["nodes"]]

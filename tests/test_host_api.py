@@ -297,3 +297,27 @@ def test_packed_partitions_see_exactly_the_whole_tree(c1_spec):
                 if child.parent is p:
                     gw_tokens[id(child)] = gtok + own[:end[id(child.parent_cut_node)]]
     assert merged_any
+
+
+def test_upload_under_a_default_device(monkeypatch):
+    """Topologies are staged in host memory whatever device a program sets as
+    the default: pinned memory only exists on the host. (Without a GPU nothing
+    can be pinned, so the flag is dropped here; the meta device stands for
+    the GPU.)"""
+    from tree_training_amd import meta
+    seen = []
+
+    class Torch:
+        def __getattr__(self, name):
+            return getattr(torch, name)
+
+        def empty(self, *a, pin_memory=False, **kw):
+            t = torch.empty(*a, **kw)
+            seen.append((pin_memory, t.device.type))
+            return t
+
+    monkeypatch.setattr(meta, "torch", Torch())
+    with torch.device("meta"):
+        got = meta.upload_i32([[3, 4, 5], [-1, 0, 1]], torch.device("cpu"))
+    assert seen == [(True, "cpu")]
+    assert got.device.type == "cpu" and got.dtype == torch.int32 and got.tolist() == [[3, 4, 5], [-1, 0, 1]]

@@ -45,7 +45,7 @@ def upload_i32(rows, device) -> torch.Tensor:
     straight into pinned memory, the copy is queued like a kernel; torch's
     caching host allocator keeps the pinned block until the copy has run."""
     a = np.asarray(rows, dtype=np.int32)
-    h = torch.empty(a.shape, dtype=torch.int32, pin_memory=True)
+    h = torch.empty(a.shape, dtype=torch.int32, device="cpu", pin_memory=True)   # whatever the default device
     h.numpy()[...] = a
     return h.to(device, non_blocking=True)
 
