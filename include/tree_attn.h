@@ -454,7 +454,12 @@ int tt_tree_conv_fwd(const tt_conv_problem* p, void* y, int64_t y_stride_tok, vo
 /* Gradients for dy [T, C] (rows dy + t*dy_stride_tok): dx [T, C] contiguous
  * (problem dtype), dweight [C, K] and dbias [C] float32 (dbias may be NULL).
  * Deterministic: the weight gradient is summed in a fixed order, dx gathers
- * over the successor lists. Workspace: tt_tree_conv_bwd_workspace_bytes. */
+ * over the successor lists. Workspace: tt_tree_conv_bwd_workspace_bytes, the
+ * size at which it runs fastest; small trees ask for more partial sums per token
+ * than large ones, so a tree can ask for more than a larger one does. Any size from
+ *   4 C (T + ceil(T / 128) (K + 1))
+ * bytes on is taken (smaller ones sum the weight gradient in longer runs, in the
+ * order that the size fixes), so a buffer made for the largest tree serves all. */
 size_t tt_tree_conv_bwd_workspace_bytes(const tt_conv_problem* p);
 int tt_tree_conv_bwd(const tt_conv_problem* p, const void* dy, int64_t dy_stride_tok, void* dx, float* dweight,
                      float* dbias, void* ws, size_t ws_bytes, void* stream);

@@ -102,6 +102,49 @@ def test_conv_fp32_run_and_batch_edges(T):
             assert _rel(a, r) < 1e-5, (T, name, _rel(a, r))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("T,larger", [(2010, 2020), (4020, 4040), (100, 130)])
+def test_conv_bwd_takes_a_larger_trees_workspace(T, larger, dtype):
+    """A tree takes the workspace that a larger tree asks for, where that is
+    less than its own (shorter runs), and the smallest one that the header
+    states: dx bitwise the same, the weight gradients equal up to their order of
+    summation, and nothing written past the end."""
+    import ctypes
+    from tree_training_amd import _lib
+    from tree_training_amd.conv import _problem
+    from tree_training_amd.meta import _ptr, _stream
+    C, K = 16384, 4                                        # 16 workgroups a run
+    lib = _lib.lib()
+    gen = torch.Generator(device=DEV).manual_seed(T)
+    x, dy = (torch.randn(T, C, generator=gen, device=DEV).to(dtype) for _ in range(2))
+    w, b = (torch.randn(C, n, generator=gen, device=DEV).to(dtype) for n in (K, 1))
+    tree = GdnTree([T // 2, T - T // 2], [-1, 0], DEV)
+    p, *keep = _problem(x, w, b.flatten(), tree)
+    want = lib.tt_tree_conv_bwd_workspace_bytes(ctypes.byref(p))
+    p.n_tokens = larger
+    other = lib.tt_tree_conv_bwd_workspace_bytes(ctypes.byref(p))
+    p.n_tokens = T
+    least = 4 * C * (T + -(-T // 128) * (K + 1))
+    assert least <= other
+    res = []
+    for ws_bytes in (want, max(other, least), least):
+        print(f"conv bwd T={T} {dtype} workspace {ws_bytes} of {want}", flush=True)
+        ws = torch.full((ws_bytes // 4 + 64,), 7.0, device=DEV)
+        dx, dw, db = torch.empty_like(x), torch.empty(C, K, device=DEV), torch.empty(C, device=DEV)
+        _lib.check(lib.tt_tree_conv_bwd(ctypes.byref(p), _ptr(dy), C, _ptr(dx), _ptr(dw), _ptr(db), _ptr(ws),
+                                        ws_bytes, _stream(DEV)), "tt_tree_conv_bwd")
+        torch.cuda.synchronize()
+        assert (ws[ws_bytes // 4:] == 7.0).all()
+        res.append((dx, dw, db))
+    assert lib.tt_tree_conv_bwd(ctypes.byref(p), _ptr(dy), C, _ptr(dx), _ptr(dw), _ptr(db), _ptr(ws), least - 4,
+                                _stream(DEV)) == _lib.TT_E_WORKSPACE
+    for dx, dw, db in res[1:]:
+        assert torch.equal(dx, res[0][0])
+        # sums of T fp32 products in two orders: below T roundings of 2^-24 of the largest
+        assert _rel(dw.cpu().numpy(), res[0][1].cpu().numpy()) < 1e-5
+        assert _rel(db.cpu().numpy(), res[0][2].cpu().numpy()) < 1e-5
+
+
 def test_conv_autograd_and_dropin():
     """The autograd Function's gradients equal tree_conv_backward's, and the
     reference-signature drop-in (channel-major input, a module with conv1d)

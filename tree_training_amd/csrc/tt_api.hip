@@ -577,8 +577,8 @@ int tt_tree_conv_bwd(const tt_conv_problem* p, const void* dy, int64_t dy_stride
     if (dy_stride_tok < p->n_channels || (dy_stride_tok % 4) || !aligned(dy, ea) || !aligned(dx, ea) ||
         !aligned(ws, 16) || !aligned(dweight, 4) || (dbias && !aligned(dbias, 4)))
         return TT_E_ARG;
-    if (ws_bytes < tt_conv_bwd_ws_bytes_impl(p->n_tokens, p->n_channels, p->kernel_size)) return TT_E_WORKSPACE;
-    return tt_conv_bwd_launch(d, dy, dy_stride_tok, dx, dweight, dbias, (float*)ws, (hipStream_t)stream);
+    if (ws_bytes < tt_conv_bwd_ws_min_bytes_impl(p->n_tokens, p->n_channels, p->kernel_size)) return TT_E_WORKSPACE;
+    return tt_conv_bwd_launch(d, dy, dy_stride_tok, dx, dweight, dbias, (float*)ws, ws_bytes, (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -376,10 +376,24 @@ int conv_fwd_run(const ConvDev& d, void* y, int64_t y_st, hipStream_t s) {
     return hipGetLastError() == hipSuccess ? TT_OK : TT_E_HIP;
 }
 
+// Floats of a backward workspace with n_parts partial sums.
+size_t bwd_ws_floats(int n_tokens, int n_ch, int k, int n_parts) {
+    return (size_t)n_tokens * n_ch + (size_t)n_parts * (k + 1) * n_ch;
+}
+// The run of the gradient pass: run_tokens', or a longer one where its partial
+// sums do not fit the workspace (those of the longest run always do).
+int run_tokens_w(const ConvDev& d, size_t ws_bytes) {
+    int r = run_tokens(d.n_tokens, d.n_ch, CTOK_W);
+    while (r < CTOK_W &&
+           bwd_ws_floats(d.n_tokens, d.n_ch, d.k, tt_cdiv(d.n_tokens, r)) > ws_bytes / sizeof(float))
+        r <<= 1;
+    return r;
+}
+
 template <int K, typename T>
 int conv_bwd_run(const ConvDev& d, const void* dy, int64_t dy_st, void* dx, float* dw, float* db, float* ws,
-                 hipStream_t s) {
-    const int run_w = run_tokens(d.n_tokens, d.n_ch, CTOK_W), run = run_tokens(d.n_tokens, d.n_ch, CTOK);
+                 size_t ws_bytes, hipStream_t s) {
+    const int run_w = run_tokens_w(d, ws_bytes), run = run_tokens(d.n_tokens, d.n_ch, CTOK);
     const int n_parts = tt_cdiv(d.n_tokens, run_w);
     T* gp = reinterpret_cast<T*>(ws);
     float* part = ws + (size_t)d.n_tokens * d.n_ch;
@@ -407,12 +421,12 @@ int conv_fwd_k(const ConvDev& d, void* y, int64_t y_st, hipStream_t s) {
 
 template <typename T>
 int conv_bwd_k(const ConvDev& d, const void* dy, int64_t dy_st, void* dx, float* dw, float* db, float* ws,
-               hipStream_t s) {
+               size_t ws_bytes, hipStream_t s) {
     switch (d.k) {
-        case 1: return conv_bwd_run<1, T>(d, dy, dy_st, dx, dw, db, ws, s);
-        case 2: return conv_bwd_run<2, T>(d, dy, dy_st, dx, dw, db, ws, s);
-        case 3: return conv_bwd_run<3, T>(d, dy, dy_st, dx, dw, db, ws, s);
-        case 4: return conv_bwd_run<4, T>(d, dy, dy_st, dx, dw, db, ws, s);
+        case 1: return conv_bwd_run<1, T>(d, dy, dy_st, dx, dw, db, ws, ws_bytes, s);
+        case 2: return conv_bwd_run<2, T>(d, dy, dy_st, dx, dw, db, ws, ws_bytes, s);
+        case 3: return conv_bwd_run<3, T>(d, dy, dy_st, dx, dw, db, ws, ws_bytes, s);
+        case 4: return conv_bwd_run<4, T>(d, dy, dy_st, dx, dw, db, ws, ws_bytes, s);
     }
     return TT_E_UNSUPPORTED;
 }
@@ -420,8 +434,10 @@ int conv_bwd_k(const ConvDev& d, const void* dy, int64_t dy_st, void* dx, float*
 }  // namespace
 
 size_t tt_conv_bwd_ws_bytes_impl(int n_tokens, int n_ch, int k) {
-    const size_t parts = (size_t)tt_cdiv(n_tokens, run_tokens(n_tokens, n_ch, CTOK_W));
-    return ((size_t)n_tokens * n_ch + parts * (k + 1) * n_ch) * sizeof(float);
+    return bwd_ws_floats(n_tokens, n_ch, k, tt_cdiv(n_tokens, run_tokens(n_tokens, n_ch, CTOK_W))) * sizeof(float);
+}
+size_t tt_conv_bwd_ws_min_bytes_impl(int n_tokens, int n_ch, int k) {
+    return bwd_ws_floats(n_tokens, n_ch, k, tt_cdiv(n_tokens, CTOK_W)) * sizeof(float);
 }
 
 int tt_conv_fwd_launch(const ConvDev& d, void* y, int64_t y_st, hipStream_t s) {
@@ -429,7 +445,7 @@ int tt_conv_fwd_launch(const ConvDev& d, void* y, int64_t y_st, hipStream_t s) {
 }
 
 int tt_conv_bwd_launch(const ConvDev& d, const void* dy, int64_t dy_st, void* dx, float* dw, float* db, float* ws,
-                       hipStream_t s) {
-    return d.dtype == TT_DTYPE_BF16 ? conv_bwd_k<__bf16>(d, dy, dy_st, dx, dw, db, ws, s)
-                                    : conv_bwd_k<float>(d, dy, dy_st, dx, dw, db, ws, s);
+                       size_t ws_bytes, hipStream_t s) {
+    return d.dtype == TT_DTYPE_BF16 ? conv_bwd_k<__bf16>(d, dy, dy_st, dx, dw, db, ws, ws_bytes, s)
+                                    : conv_bwd_k<float>(d, dy, dy_st, dx, dw, db, ws, ws_bytes, s);
 }

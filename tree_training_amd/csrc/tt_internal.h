@@ -107,9 +107,10 @@ struct ConvDev {
 };
 
 size_t tt_conv_bwd_ws_bytes_impl(int n_tokens, int n_ch, int k);
+size_t tt_conv_bwd_ws_min_bytes_impl(int n_tokens, int n_ch, int k);   // the least the backward takes
 int tt_conv_fwd_launch(const ConvDev& d, void* y, int64_t y_st, hipStream_t s);
 int tt_conv_bwd_launch(const ConvDev& d, const void* dy, int64_t dy_st, void* dx, float* dw, float* db, float* ws,
-                       hipStream_t s);
+                       size_t ws_bytes, hipStream_t s);
 
 // Device-side view of a tt_prologue_problem.
 struct PrologueDev {
