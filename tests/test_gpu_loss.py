@@ -139,6 +139,18 @@ def test_fused_linear_ce_matches_torch(dtype, tol):
     assert _rel(wd.grad.cpu(), wr.grad) < tol
 
 
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-5), (torch.bfloat16, 2e-2)])
+def test_fused_linear_ce_gemms_add_themselves(monkeypatch, dtype, tol):
+    """Outside autocast no chunk's weight gradient is formed apart and added."""
+    from tree_training_amd import loss as loss_module
+
+    def apart(a, b):
+        raise AssertionError("a separate product")
+
+    monkeypatch.setattr(loss_module, "_mm_f32", apart)
+    test_fused_linear_ce_matches_torch(dtype, tol)
+
+
 def test_fused_linear_ce_autocast_adds_apart():
     """float32 tensors under bf16 autocast, three chunks: the weight gradient's
     GEMM result and the sum differ in type, so they are added separately. Bar:

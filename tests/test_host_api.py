@@ -321,3 +321,27 @@ def test_upload_under_a_default_device(monkeypatch):
         got = meta.upload_i32([[3, 4, 5], [-1, 0, 1]], torch.device("cpu"))
     assert seen == [(True, "cpu")]
     assert got.device.type == "cpu" and got.dtype == torch.int32 and got.tolist() == [[3, 4, 5], [-1, 0, 1]]
+
+
+@pytest.mark.parametrize("first", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_weight_gradient_gemm_errors_propagate(monkeypatch, dtype, first):
+    """The leaf loss's accumulating GEMM: only a torch or device without a
+    float32-out overload (as the CPU in bfloat16) takes the separate addition; out of
+    memory and device errors reach the caller."""
+    from tree_training_amd import loss
+    a, b = torch.randn(6, 5).to(dtype), torch.randn(5, 4).to(dtype)
+    acc = torch.full((6, 4), 3.0)
+    loss._acc_mm(acc, a, b, first)
+    want = a.float() @ b.float() + (0.0 if first else 3.0)
+    assert torch.allclose(acc, want, rtol=1e-2 if dtype == torch.bfloat16 else 1e-5, atol=2e-2)
+    for err in (torch.OutOfMemoryError("out of memory"), RuntimeError("HIP error: launch failure")):
+        def fail(*a, **kw):
+            raise err
+        monkeypatch.setattr(torch, "mm", fail)
+        monkeypatch.setattr(torch, "addmm", fail)
+        with pytest.raises(type(err)):
+            loss._acc_mm(acc, a, b, first)
+        if dtype == torch.bfloat16:
+            with pytest.raises(type(err)):
+                loss._mm_f32(a, b)

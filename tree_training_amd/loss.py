@@ -49,12 +49,15 @@ def ce_rows(logits: torch.Tensor, labels: torch.Tensor, row_scale: torch.Tensor,
 
 def _mm_f32(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     """a @ b with a float32 result straight from the GEMM (no rounding to the
-    inputs' dtype in between)."""
+    inputs' dtype in between; inputs of two dtypes, as autocast leaves them, go
+    through its own product)."""
     if a.dtype == torch.float32:
         return a @ b
+    if a.dtype != b.dtype:
+        return (a @ b).float()
     try:
         return torch.mm(a, b, out_dtype=torch.float32)
-    except (RuntimeError, NotImplementedError, TypeError):
+    except (NotImplementedError, TypeError):     # no such overload; other errors are the caller's
         return (a @ b).float()
 
 
@@ -71,7 +74,7 @@ def _acc_mm(acc: torch.Tensor, a: torch.Tensor, b: torch.Tensor, first: bool) ->
             else:
                 torch.addmm(acc, a, b, out=acc, **kw)
             return
-        except (RuntimeError, NotImplementedError, TypeError):
+        except (NotImplementedError, TypeError):     # no such overload; other errors are the caller's
             pass
     if first:
         acc.copy_(_mm_f32(a, b))
