@@ -35,6 +35,12 @@ enum {
     TT_E_WORKSPACE = -4     /* workspace or plan buffer too small */
 };
 
+/* float32 attention, and the gated delta rule's float32 operands in either
+ * dtype, run on the bf16 matrix cores, every operand as the sum of three bf16
+ * planes, to float32 accuracy. The planes hold all 24 bits of magnitudes from
+ * 2^-110 to 3.389e38 (below, up to 2^-134 is lost). Results that a NaN, an
+ * infinity or a larger magnitude reaches are not finite; an infinity may come out
+ * as NaN. */
 enum { TT_DTYPE_F32 = 0, TT_DTYPE_BF16 = 1 };
 
 /* Parts of the backward (tt_attn_problem.bwd_parts); they must run in this

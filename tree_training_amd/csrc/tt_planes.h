@@ -2,13 +2,15 @@
 // three bf16 planes, x = h + m + l (h = bf16(x), m = bf16(x - h), l = the rest,
 // exact: 3 x 8 significant bits), and a product x y is the six plane products
 // h h + (h m + m h) + (m m + h l + l h), each exact, summed in the MFMA's fp32
-// accumulators. The dropped m l, l m, l l lie below 2^-26 of the product, a
-// quarter of one fp32 rounding. gfx950 runs 16 bf16 MFMAs in the time of one
-// fp32 MFMA of the same size, so six of them take 2.7 times less matrix time;
-// an operand that is bf16 to begin with is its own h plane, and its products
-// with a split one take three. A non-finite operand gives non-finite results,
-// but an infinity may come out as NaN (inf - inf in the split), and so may a
-// magnitude above 3.389e38, which bf16 rounds to infinity.
+// accumulators. The dropped m l, l m, l l reach 2^-24 of the product at the
+// worst (x = y = 1 + 2^-8 - 2^-17), one rounding of fp32, and 2^-27.5 in the root
+// mean square. gfx950 runs 16 bf16 MFMAs in the time of one fp32 MFMA of the
+// same size, so six of them take 2.7 times less matrix time; an operand that is
+// bf16 to begin with is its own h plane, and its products with a split one take
+// three. Below 2^-110 the planes end at bf16's smallest step and miss up to
+// 2^-134 of x. A non-finite operand gives non-finite results, but an infinity
+// may come out as NaN (inf - inf in the split), and so may a magnitude above
+// 3.389e38, which bf16 rounds to infinity.
 #pragma once
 
 #include "tt_common.h"
