@@ -102,6 +102,31 @@ def test_conv_fp32_run_and_batch_edges(T):
             assert _rel(a, r) < 1e-5, (T, name, _rel(a, r))
 
 
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-5), (torch.bfloat16, 2e-2)], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("T", [67, 2101, 4135, 8263])
+def test_conv_run_lengths(T, dtype, tol):
+    """16,384 channels (16 workgroups a run), where runs of 16, 32, 64 and (the
+    gradient pass) 128 tokens are taken: eight channels repeated give the
+    oracle's results in the first and the last repetition and the same bits in
+    all of them. Nodes break inside runs and batches."""
+    cut = T // 3 + 2
+    lens, par = [cut, 1, cut - 9, T - 2 * cut + 8], [-1, 0, 0, 2]
+    x, w, b, dy = _inputs(T, 8, 4, T, True)
+    if dtype == torch.bfloat16:
+        x, w, b, dy = (torch.from_numpy(a).bfloat16().float().numpy() for a in (x, w, b, dy))
+    R = 2048
+    print(f"tree conv run lengths T={T} {dtype}", flush=True)
+    tree = GdnTree(lens, par, DEV)
+    t = lambda a, *reps: torch.from_numpy(a).to(DEV, dtype).repeat(*reps)
+    y = tree_conv_forward(t(x, 1, R), t(w, R, 1), t(b, R), tree)
+    dx, dw, db = tree_conv_backward(t(x, 1, R), t(w, R, 1), t(b, R), t(dy, 1, R), tree)
+    torch.cuda.synchronize()
+    got = [y.view(T, R, 8).transpose(0, 1), dx.view(T, R, 8).transpose(0, 1), dw.view(R, 8, 4), db.view(R, 8)]
+    for name, a, r in zip(("y", "dx", "dw", "db"), got, _oracle(x, w, b, dy, lens, par)):
+        assert torch.equal(a, a[:1].expand_as(a)), name
+        assert _rel(a[0].float().cpu().numpy(), r) < tol, (T, name, _rel(a[0].float().cpu().numpy(), r))
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("T,larger", [(2010, 2020), (4020, 4040), (100, 130)])
 def test_conv_bwd_takes_a_larger_trees_workspace(T, larger, dtype):

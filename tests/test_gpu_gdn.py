@@ -194,23 +194,61 @@ def test_gdn_bwd_fp32_matches_autograd_oracle(case):
         assert _rel(a, b) < 1e-5, (case, name, _rel(a, b))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("Hk,Hv", [(1, 2), (16, 32)], ids=["row_layout", "column_layout"])
-def test_gdn_scan_chunk_edges(Hk, Hv):
+def test_gdn_scan_chunk_edges(Hk, Hv, dtype):
     """Nodes of 1, 31, 32, 33, 64 and 65 tokens on one level (and a root of 33),
     in the row layout of the level scans (12 pairs) and the column layout (192
-    pairs): fp32 outputs, states and gradients against the float64 oracle, at
-    the fp32 bar."""
+    pairs), with operands of three planes (fp32) and as they come (bf16): outputs,
+    states and gradients against the float64 oracle, at each dtype's bar (the
+    states are fp32 from exact inputs in both)."""
     lens, par = [33, 1, 31, 32, 33, 64, 65], [-1] + [0] * 6
     T = sum(lens)
     q, k, v, g, beta = _inputs(T, Hk, Hv, 41 + Hv, realistic_gates=True)
     d_o = np.random.default_rng(12).standard_normal((T, Hv, D)).astype(np.float32)
-    print(f"gdn scan chunk edges: T={T} heads {Hk}/{Hv}", flush=True)
-    o, st = _run(q, k, v, g, beta, lens, par, torch.float32)
+    tol = 1e-5
+    if dtype == torch.bfloat16:
+        tol = 2e-2
+        q, k, v, d_o = (torch.from_numpy(x).bfloat16().float().numpy() for x in (q, k, v, d_o))
+    print(f"gdn scan chunk edges: T={T} heads {Hk}/{Hv} {dtype}", flush=True)
+    o, st = _run(q, k, v, g, beta, lens, par, dtype)
     o_ref, st_ref = ogdn.gdn_tree(q, k, v, g, beta, lens, par, mode="exact")
-    assert _rel(o, o_ref) < 1e-5 and _rel(st, st_ref) < 1e-5
-    got = _run_bwd(q, k, v, g, beta, d_o, lens, par, torch.float32)
+    assert _rel(o, o_ref) < tol and _rel(st, st_ref) < 1e-5
+    got = _run_bwd(q, k, v, g, beta, d_o, lens, par, dtype)
     for name, a, b in zip(BWD_NAMES, got, _oracle_grads(q, k, v, g, beta, d_o, lens, par)):
-        assert _rel(a, b) < 1e-5, (name, _rel(a, b))
+        assert _rel(a, b) < (1e-5 if name in ("dg", "dbeta") else tol), (name, _rel(a, b))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("truncated", [False, True], ids=["exact", "truncated"])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")], ids=str)
+def test_gdn_non_finite_inputs(value, truncated, dtype):
+    """A non-finite value of one v head in one root of a forest: that head's
+    later rows of the root and of its child come out non-finite, the forest's
+    other tree and the other v heads' outputs keep their bits."""
+    lens, par = [70, 40, 90, 33], [-1, 0, -1, 2]
+    T, n0 = sum(lens), 110
+    dev = torch.device("cuda", 0)
+    ins = [torch.from_numpy(x).to(dev) for x in _inputs(T, 2, 4, 5, realistic_gates=True)]
+    ins[:3] = [x.to(dtype) for x in ins[:3]]
+    d_o = torch.from_numpy(np.random.default_rng(3).standard_normal((T, 4, D)).astype(np.float32)).to(dev, dtype)
+    tree = GdnTree(lens, par, dev)
+    res = []
+    for bad in (False, True):
+        x = [t.clone() for t in ins]
+        if bad:
+            x[2][37, 1, 3] = value
+        print(f"gdn non-finite {value} truncated={truncated} {dtype} in={bad}", flush=True)
+        o, st = gdn_tree_forward(*x, tree, reference_truncated=truncated)
+        res.append((o, st, *gdn_tree_backward(*x, d_o, tree, reference_truncated=truncated)))
+        torch.cuda.synchronize()
+    (o0, st0, *g0), (o1, st1, *g1) = res
+    assert all(torch.isfinite(t.float()).all() for t in res[0])
+    assert torch.equal(o0[n0:], o1[n0:]) and torch.equal(st0[2:], st1[2:])
+    assert torch.equal(o0[:, [0, 2, 3]], o1[:, [0, 2, 3]])
+    assert not torch.isfinite(o1[37:n0, 1, 3].float()).any() and not torch.isfinite(st1[:2, 1, :, 3]).any()
+    for name, a, b in zip(BWD_NAMES, g0, g1):
+        assert torch.equal(a[n0:], b[n0:]), name
 
 
 @pytest.mark.parametrize("case", ["forest_multi_chunk", "c1_heads"])

@@ -165,23 +165,30 @@ def test_reference_mode_saved_forward_equals_recompute(dtype):
         assert torch.equal(a, b), name
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("Hk,Hv", [(1, 2), (16, 32)])
-def test_reference_mode_block_edges(Hk, Hv):
+def test_reference_mode_block_edges(Hk, Hv, dtype):
     """Nodes of 1, 31, 32, 33, 64, 65 and 97 tokens on one level (and a root of
     33): whole, ragged and single-token correction blocks, in the row layout of
-    the level scans (14 pairs) and the column layout (224 pairs): fp32 outputs,
-    states and gradients against the float64 oracle, at the fp32 bar."""
+    the level scans (14 pairs) and the column layout (224 pairs), with operands
+    of three planes (fp32) and as they come (bf16): outputs, states and gradients
+    against the float64 oracle, at each dtype's bar (the states are fp32 from
+    exact inputs in both)."""
     lens, par = [33, 1, 31, 32, 33, 64, 65, 97], [-1] + [0] * 7
     T = sum(lens)
     q, k, v, g, beta = _inputs(T, Hk, Hv, 43 + Hv, realistic_gates=True)
     d_o = np.random.default_rng(14).standard_normal((T, Hv, D)).astype(np.float32)
-    print(f"gdn reference block edges: T={T} heads {Hk}/{Hv}", flush=True)
-    o, st = _run(q, k, v, g, beta, lens, par, torch.float32)
+    tol = 1e-5
+    if dtype == torch.bfloat16:
+        tol = 2e-2
+        q, k, v, d_o = (torch.from_numpy(x).bfloat16().float().numpy() for x in (q, k, v, d_o))
+    print(f"gdn reference block edges: T={T} heads {Hk}/{Hv} {dtype}", flush=True)
+    o, st = _run(q, k, v, g, beta, lens, par, dtype)
     o_ref, st_ref = ogdn.gdn_tree(q, k, v, g, beta, lens, par, mode="reference")
-    assert _rel(o, o_ref) < 1e-5 and _rel(st, st_ref) < 1e-5
-    got = _run_bwd(q, k, v, g, beta, d_o, lens, par, torch.float32)
+    assert _rel(o, o_ref) < tol and _rel(st, st_ref) < 1e-5
+    got = _run_bwd(q, k, v, g, beta, d_o, lens, par, dtype)
     for name, a, b in zip(BWD_NAMES, got, _oracle_grads(q, k, v, g, beta, d_o, lens, par)):
-        assert _rel(a, b) < 1e-5, (name, _rel(a, b))
+        assert _rel(a, b) < (1e-5 if name in ("dg", "dbeta") else tol), (name, _rel(a, b))
 
 
 def test_reference_mode_agent16k_two_heads_matches_oracle():

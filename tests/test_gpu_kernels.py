@@ -511,15 +511,31 @@ def test_attention_fp32_step_edges(lens, par, n_past):
             check_close(name, ref, got, TOL[torch.float32])
 
 
+def _takes_two_groups(heads, n_q, n_past):
+    """Whether the bf16 dK/dV launch gives an item two groups of waves: at most
+    256 work items (a chain's, an upper bound) of at least 32 steps each."""
+    rep = heads[0] // heads[1]
+    qch = min(max(256, (1 << (n_q.bit_length() - 1)) // 2), 4096)
+    n_kb = -(-(n_q + n_past) // 128)
+    items = 0
+    for kb in range(n_kb):
+        qlo = max(0, kb * 128 - n_past)
+        items += 1 if n_q - qlo <= qch else (n_q - 1) // qch - qlo // qch + 1
+    return items * heads[1] <= 256 and -(-min(n_q, qch) // 32) * rep >= 32
+
+
 @pytest.mark.parametrize("deterministic", [False, True], ids=["sums", "slots"])
 @pytest.mark.parametrize("heads,lens,par,n_past", [
-    ((3, 1), [300, 40], [-1, 0], 0),                    # 33 steps a group pair: one has a step less
-    ((6, 2), [340, 1, 90], [-1, 0, 0], 131),            # split items, gateway keys, a ragged last tile
+    ((3, 1), [1060, 40], [-1, 0], 0),                   # odd step counts: one group has a step less
+    ((6, 2), [800, 1, 299], [-1, 0, 0], 131),           # split items, gateway keys, a ragged last tile
+    ((4, 2), [1500, 700], [-1, 0], 300),                # gateway keys seen by several items
+    ((8, 2), [200, 33], [-1, 0], 131),                  # gateway keys of one item each
     ((8, 1), [90, 33], [-1, 0], 0), ((1, 1), [2050], [-1], 0)])
 def test_attention_dkdv_head_pairs(monkeypatch, heads, lens, par, n_past, deterministic):
     """bf16 dK/dV of problems with few work items, whose steps two groups of
     waves share: odd step counts, one and several q heads a kv head, split and
     unsplit tiles, own and gateway keys, against the fp64 oracle at the bf16 bar."""
+    assert _takes_two_groups(heads, sum(lens), n_past)
     monkeypatch.setattr(sys.modules[__name__], "HQ", heads[0])
     monkeypatch.setattr(sys.modules[__name__], "HKV", heads[1])
     past_vis = [i % 7 != 3 for i in range(n_past)] if n_past else None
@@ -528,6 +544,64 @@ def test_attention_dkdv_head_pairs(monkeypatch, heads, lens, par, n_past, determ
     for name, (ref, got) in res.items():
         if name != "lse":
             check_close(name, ref, got, TOL[torch.bfloat16])
+
+
+@pytest.mark.parametrize("exps", [(-100, 100, 0, 0), (0, 0, -100, 0), (0, 0, 0, -100), (0, 0, 100, -60)],
+                         ids=["q,k", "small v", "small dO", "large v"])
+def test_attention_fp32_scaled_operands(monkeypatch, exps):
+    """The bf16 planes of fp32 operands hold all 24 bits down to 2^-110: inputs
+    scaled by powers of two as far as 2^-100 and 2^100 keep the fp32 bar."""
+    plain = _qkv
+
+    def scaled(T, Lp, dtype, seed):
+        q, k, v, do, kp, vp = plain(T, Lp, dtype, seed)
+        e = [2.0 ** x for x in exps]
+        return q * e[0], k * e[1], v * e[2], do * e[3], kp, vp
+
+    monkeypatch.setattr(sys.modules[__name__], "_qkv", scaled)
+    say(f"attention fp32 scaled operands 2^{exps}")
+    for name, (ref, got) in _run([150, 40, 60], [-1, 0, 0], torch.float32, seed=7).items():
+        if name != "lse":
+            rel = np.abs(ref - got).max() / np.abs(ref).max()
+            assert rel < TOL[torch.float32], (name, rel)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 3.4e38], ids=str)
+def test_attention_non_finite_inputs(dtype, value):
+    """One non-finite value, or one that bf16 rounds to infinity, in a tree's V
+    and dO: that tree's results that depend on it come out non-finite (infinite
+    or NaN), and the other tree of the forest (its own key tiles and query
+    blocks) keeps its bits."""
+    if dtype == torch.bfloat16 and value == 3.4e38:
+        value = float("inf")                            # what bf16 inputs hold of it
+    from tree_training_amd.attention import attn_backward, attn_forward
+    from tree_training_amd.meta import KeyPlan
+    lens, par, n0 = [256, 150, 60], [-1, -1, 1], 256
+    T, scale = sum(lens), D ** -0.5
+    q, k, v, do, _, _ = _qkv(T, 0, dtype, 3)
+    m = _meta(lens, par)
+    plan = KeyPlan(m.horizon)
+    tr = lambda x: x.to(DEV).transpose(1, 2)
+    out = []
+    for bad in (False, True):
+        v1, do1 = v.clone(), do.clone()
+        if bad:
+            v1[0, 20, 0, 5] = value
+            do1[0, 40, 1, 9] = value
+        say(f"attention non-finite {value} dtype={dtype} in={bad}")
+        o, lse = attn_forward(tr(q), tr(k), tr(v1), plan, scale)
+        out.append([o, *attn_backward(tr(q), tr(k), tr(v1), plan, scale, o, lse, do1.to(DEV), deterministic=True)])
+        torch.cuda.synchronize()
+    for name, a, b in zip(("o", "dq", "dk", "dv"), *out):
+        assert torch.isfinite(a.float()).all()
+        assert torch.equal(a[n0:], b[n0:]), name
+    bad = [x.float() for x in out[1]]
+    if value == 3.4e38:       # a finite input: every result it reaches is huge at least
+        assert (~(bad[0][20:n0, :4, 5].abs() < 1e30)).all()
+    else:
+        assert not torch.isfinite(bad[0][20:n0, :4, 5]).any()
+        assert not torch.isfinite(bad[1][40, 1]).any() and not torch.isfinite(bad[3][:41, 0, 9]).any()
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
