@@ -235,12 +235,15 @@ struct KvStage {
 // offsets per lane are fixed for the kernel, the padding bytes of each row
 // take row data that nothing reads); rows past the last query read as zeros.
 // The block's lse (wave 0) and delta (wave 1) come through registers.
+// NG: the groups of four waves in the workgroup, each staging blocks of its own.
+template <int NG>
 struct QBlockStager {
+    static __device__ __forceinline__ int group_wave() { return NG == 1 ? threadIdx.x >> 6 : (threadIdx.x >> 6) & 3; }
     uint32_t vo[5];   // this lane's buffer offset in each of its wave's pieces
     float sv;
     int q0;
     __device__ __forceinline__ void init(const AttnDev& a, const BwdDev& bw) {
-        const int wave = (threadIdx.x >> 6) & 3, lane = threadIdx.x & 63;
+        const int wave = group_wave(), lane = threadIdx.x & 63;
         const uint32_t stb = 2u * (uint32_t)(wave < 2 ? a.q_st : bw.do_st);
 #pragma unroll
         for (int i = 0; i < 5; ++i) {
@@ -253,7 +256,7 @@ struct QBlockStager {
     // Issues the direct loads of query block q0_, q head h into stage S.
     __device__ __forceinline__ void begin(const AttnDev& a, const BwdDev& bw, int q0_, int h, KvStage& S) {
         q0 = q0_;
-        const int wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
+        const int wave = __builtin_amdgcn_readfirstlane(group_wave());
         const int rows = min(TT_BQB, a.n_q - q0);
         const bool isq = wave < 2;
         const uint32_t stb = 2u * (uint32_t)(isq ? a.q_st : bw.do_st);
@@ -271,7 +274,7 @@ struct QBlockStager {
     // Completes the stage (before the barrier that publishes it). Rows past
     // the last query get -inf for -lse / scale, so they contribute nothing.
     __device__ __forceinline__ void commit(const AttnDev& a, KvStage& S) {
-        const int wave = (threadIdx.x >> 6) & 3, lane = threadIdx.x & 63;
+        const int wave = group_wave(), lane = threadIdx.x & 63;
         if (wave < 2 && lane < TT_BQB) {
             const bool in = q0 + lane < a.n_q;
             if (wave == 0) S.nlse[lane] = in ? -sv / a.scale : -INFINITY;
@@ -303,13 +306,13 @@ __global__ __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(2, 2))
 
     const int grp = NG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
     KvStage* const st = lds.st[grp];
-    const int wave = (threadIdx.x >> 6) & 3, lane = threadIdx.x & 63;
+    const int wave = QBlockStager<NG>::group_wave(), lane = threadIdx.x & 63;
     const int col = lane & 31, half = lane >> 5;
     const float c = a.scale * TT_LOG2E;
     const int n_work = (*a.n_items) * a.hkv;
     const RowOffsX qro = row_offsx(col, half);   // this lane's query row in the Q / dO blocks
     const TrOffsX tro = tr_offsx(lane);
-    QBlockStager stg;
+    QBlockStager<NG> stg;
     stg.init(a, bw);
 
     for (int w_id = blockIdx.x; w_id < n_work; w_id += gridDim.x) {
@@ -338,7 +341,9 @@ __global__ __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(2, 2))
         const int q_top = (q_stop > q_start) ? ((q_stop - 1) / TT_BQB) * TT_BQB : 0;
         const int n_steps = (q_stop > q_start) ? ((q_top - q_start) / TT_BQB + 1) * a.rep : 0;
         // a group's steps: its first, then every NG-th; (q0, hh) is the query
-        // block and the q head g * rep + hh of its next one
+        // block and the q head g * rep + hh of its next one. The one-group form
+        // steps by a compare: the general form's scalar work shows there (9,001
+        // tokens, 32/8 heads: 689 us against 679).
         int q0 = q_top, hh = grp;
         const auto settle = [&]() {
             while (hh >= a.rep) {
@@ -346,7 +351,7 @@ __global__ __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(2, 2))
                 q0 -= TT_BQB;
             }
         };
-        settle();
+        if constexpr (NG > 1) settle();
         if (grp < n_steps) stg.begin(a, bw, q0, g * a.rep + hh, st[0]);
 
         // V rows of the tile's 128 keys go to LDS (read as MFMA operands every
@@ -391,14 +396,22 @@ __global__ __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(2, 2))
 
         // Query blocks are walked from the top of the range down, so items whose
         // ranges end at the same subtree end read the same rows at the same time.
-        for (int s = grp, n = 0; s < n_steps + grp; s += NG, ++n) {
+        for (int n = 0; NG * n < n_steps; ++n) {
+            const int s = NG * n + grp;
             KvStage& S = st[n & 1];
             if (NG == 1 || s < n_steps) stg.commit(a, S);
             __syncthreads();
             if (NG > 1 && s >= n_steps) break;   // the groups' step counts differ by one at most
             const int q0_cur = q0;
-            hh += NG;
-            settle();
+            if constexpr (NG == 1) {
+                if (++hh == a.rep) {
+                    hh = 0;
+                    q0 -= TT_BQB;
+                }
+            } else {
+                hh += NG;
+                settle();
+            }
             // the other stage was last read in the step before, which every wave has left
             if (s + NG < n_steps) stg.begin(a, bw, q0, g * a.rep + hh, st[(n + 1) & 1]);
             const int q1 = min(q0_cur + TT_BQB, a.n_q);
