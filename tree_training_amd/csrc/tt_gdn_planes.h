@@ -14,6 +14,18 @@ namespace {
 // both reach every bank once a pass.
 constexpr int PR = GD + 8, PC = GD + 16;   // [token][state row] tiles
 constexpr int AR = GC + 8, AC = GC + 16;   // [token][token]
+// The same without padding: the 16-byte pieces of a row exchanged by its number
+// (rows that one read covers, and the writes, still reach every bank once a
+// pass). PRS for tiles read by rows, PCS by columns.
+constexpr int PRS = GD, PCS = -GD;
+constexpr int row_elems(int P) { return P < 0 ? -P : P; }
+constexpr bool swapped(int P) { return P == PRS || P == PCS; }
+// Element (row, d) of such a tile.
+template <int P>
+__device__ __forceinline__ int tile_at(int row, int d) {
+    const int x = P == PRS ? row & 15 : (2 * (row & 7)) ^ (row & 1);
+    return row * GD + (((d >> 3) ^ x) << 3) + (d & 7);
+}
 template <typename TIn>
 constexpr int kInPlanes = sizeof(TIn) == 2 ? 1 : 3;
 
@@ -80,8 +92,13 @@ __device__ __forceinline__ Op<N> op_rows(const __bf16* X, int row, int k0, int g
     Op<N> o;
 #pragma unroll
     for (int n = 0; n < N; ++n) {
-        const __bf16* x = X + n * GC * P + row * P + k0 + g4;
-        o.p[n] = cat44(*(const bf16x4*)x, *(const bf16x4*)(x + 16));
+        if constexpr (swapped(P)) {
+            const __bf16* x = X + n * GC * GD;
+            o.p[n] = cat44(*(const bf16x4*)(x + tile_at<P>(row, k0 + g4)), *(const bf16x4*)(x + tile_at<P>(row, k0 + 16 + g4)));
+        } else {
+            const __bf16* x = X + n * GC * P + row * P + k0 + g4;
+            o.p[n] = cat44(*(const bf16x4*)x, *(const bf16x4*)(x + 16));
+        }
     }
     return o;
 }
@@ -92,8 +109,13 @@ __device__ __forceinline__ Op<N> op_cols(const __bf16* X, int c0, int lane) {
     Op<N> o;
 #pragma unroll
     for (int n = 0; n < N; ++n) {
-        const __bf16* x = X + n * GC * P + (4 * (lane >> 4) + (j >> 2)) * P + c0 + 4 * (j & 3);
-        o.p[n] = cat44(ds_read_tr(x), ds_read_tr(x + 16 * P));
+        if constexpr (swapped(P)) {
+            const __bf16* x = X + n * GC * GD + tile_at<P>(4 * (lane >> 4) + (j >> 2), c0 + 4 * (j & 3));
+            o.p[n] = cat44(ds_read_tr(x), ds_read_tr(x + 16 * GD));
+        } else {
+            const __bf16* x = X + n * GC * P + (4 * (lane >> 4) + (j >> 2)) * P + c0 + 4 * (j & 3);
+            o.p[n] = cat44(ds_read_tr(x), ds_read_tr(x + 16 * P));
+        }
     }
     return o;
 }
@@ -111,10 +133,12 @@ __device__ __forceinline__ void put16(__bf16* X, int i, int d0, const f32x4 (&x)
         Split8 w = split_begin(x[2 * n], x[2 * n + 1]);
         w.all();
         const Planes q = w.planes();
-        __bf16* d = X + i * P + d0 + 8 * n;
+        __bf16* d;
+        if constexpr (swapped(P)) d = X + tile_at<P>(i, d0 + 8 * n);
+        else d = X + i * P + d0 + 8 * n;
         *(bf16x8*)d = q.h;
-        *(bf16x8*)(d + GC * P) = q.m;
-        *(bf16x8*)(d + 2 * GC * P) = q.l;
+        *(bf16x8*)(d + GC * row_elems(P)) = q.m;
+        *(bf16x8*)(d + 2 * GC * row_elems(P)) = q.l;
     }
 }
 // 1 / sqrt(|row|^2 + eps) (1 without the l2 norm) of the row whose 128

@@ -10,9 +10,17 @@
 // 108 MFMAs of 16 cycles forward and 102 reverse (bf16 problems) where
 // v_mfma_f32_16x16x4_f32 took 208 and 200 of 32. On the 16K agent tree (32 v
 // heads, bf16) the column-layout levels went 867 -> 600 us forward and 1098 ->
-// 830 reverse, the row-layout ones 164 -> 140 and 256 -> 228. What bounds them
-// now is what they move: the states and their gradients (2.2 GB written), W,
-// U, V' and dV'.
+// 830 reverse, the row-layout ones 164 -> 140 and 256 -> 228. Neither the pipes
+// nor memory are full now (column levels: MFMA 12 and 8 % busy, 4.0 and 2.6 TB/s
+// of a copy's 6.2): a level is a chain of chunks, two barriers each, at two waves a
+// SIMD.
+//
+// fp32 problems hold q and k as three planes too. The forward's tiles are packed
+// for two workgroups a CU (kScanPacked), the reverse ones and the truncated
+// rule's (88 to 104 KB) leave one. 16,318 tokens, 32 v heads, exact rule: forward
+// 1,311 us on fp32 MFMAs, 1,419 on padded tiles, 1,247 packed; forward and
+// backward 5.59 -> 5.25 ms. Trees of one or two chunks a node pay the splits once a
+// launch (47 tokens: 22.2 -> 22.8 us forward, 89 -> 86 both).
 #pragma once
 
 #include "tt_gdn_planes.h"
@@ -87,9 +95,9 @@ __device__ __forceinline__ void alt_row(f32x4 (&x)[4], int i) {
 template <typename TIn, int PQ, int PK, int PW, int PA, bool ALT>
 struct ScanTiles {
     static constexpr int NQ = kInPlanes<TIn>;
-    __bf16 Q[NQ * GC * PQ];
-    __bf16 K[NQ * GC * PK];
-    __bf16 W[3 * GC * PW];
+    __bf16 Q[NQ * GC * row_elems(PQ)];
+    __bf16 K[NQ * GC * row_elems(PK)];
+    __bf16 W[3 * GC * row_elems(PW)];
     __bf16 A[3 * GC * PA];
     float fq[GC], fk[GC];
     float el;   // e^{G_L}
@@ -125,8 +133,12 @@ struct ScanTiles {
         }
     }
 };
-template <typename TIn>
-using FwdTiles = ScanTiles<TIn, PR, PC, PR, AR, false>;   // q, W and A by rows, k by columns
+// fp32, exact rule: the forward's tiles without padding, 82 KB a workgroup instead
+// of 88 (rows: 104), so that two share a CU.
+template <typename TIn, bool TRUNC>
+constexpr bool kScanPacked = kInPlanes<TIn> == 3 && !TRUNC;
+template <typename TIn, int P = PR, int C = PC>
+using FwdTiles = ScanTiles<TIn, P, C, P, AR, false>;   // q, W and A by rows, k by columns
 template <typename TIn>
 using RevTiles = ScanTiles<TIn, PC, PR, PC, AC, true>;   // k by rows, q, W and A by columns
 
@@ -156,7 +168,7 @@ __device__ __forceinline__ f32x4 out_tok(const f32x4& qs, const float* fq, int t
 
 // Column layout of the level scans. The value columns of the delta rule are
 // independent (column j of V', O and S depends only on column j of U, S and
-// V'); each wave owns 16 of them (16 x 16 fp32 MFMA tiles), and a (node,
+// V'); each wave owns 16 of them (16 x 16 accumulator tiles), and a (node,
 // v head) takes two workgroups of four waves (64 columns each) on different
 // CUs. A level with few nodes is a serial chain of chunks per node while most
 // CUs idle, and each chunk then runs on twice the MFMA pipes of one
@@ -218,7 +230,9 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
                                                       TIn* __restrict__ out, float* __restrict__ states,
                                                       float* __restrict__ chunk_sin, float* __restrict__ chunk_vp) {
     constexpr int NQ = kInPlanes<TIn>;
-    __shared__ __attribute__((aligned(16))) FwdTiles<TIn> L;
+    constexpr bool packed = kScanPacked<TIn, TRUNC>;
+    constexpr int P = packed ? PRS : PR, C = packed ? PCS : PC;
+    __shared__ __attribute__((aligned(16))) FwdTiles<TIn, P, C> L;
     ScanNode nd;
     if (!nd.init(p, lvl_begin)) return;
     int h, cb;
@@ -265,16 +279,23 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
         if (ci + 1 < n_ch) fetch(ci + 1);
         lds_barrier();
 
+        // packed: the operands' LDS offsets are formed once a chunk, and their
+        // reads stay with their products (held across, they spill)
+        int lo = lane;
+        if constexpr (packed) asm volatile("" : "+v"(lo));
+        const int lane = lo, c16 = lane & 15, g4 = 4 * (lane >> 4);
+
         // V' = U - W S and q S over the 128 state rows as four partial sums
         // added in order: the partition of the row layout's waves
         // (gdn_scan_rows_kernel), so both layouts give the same bits.
 #pragma unroll
         for (int w4 = 0; w4 < 4; ++w4) {
+            if constexpr (packed) __builtin_amdgcn_sched_barrier(0);
             const Op<3> sp = op_acc(S[2 * w4], S[2 * w4 + 1]);
 #pragma unroll
             for (int tb = 0; tb < 2; ++tb) {
-                vp[tb] -= mul_planes(op_rows<3, PR>(L.W, 16 * tb + c16, 32 * w4, g4), TRUNC ? s0p[w4] : sp, (f32x4){});
-                qs[tb] += mul_planes(op_rows<NQ, PR>(L.Q, 16 * tb + c16, 32 * w4, g4), sp, (f32x4){});
+                vp[tb] -= mul_planes(op_rows<3, P>(L.W, 16 * tb + c16, 32 * w4, g4), TRUNC ? s0p[w4] : sp, (f32x4){});
+                qs[tb] += mul_planes(op_rows<NQ, P>(L.Q, 16 * tb + c16, 32 * w4, g4), sp, (f32x4){});
             }
         }
         if (chunk_vp) {
@@ -300,8 +321,10 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
             const Op<3> vs = op_acc(scale_tok(vp[0], L.fk, g4), scale_tok(vp[1], L.fk, 16 + g4));
             const float el = L.el;
 #pragma unroll
-            for (int rb = 0; rb < 8; ++rb)
-                S[rb] = fma_tile(S[rb], el, mul_planes(op_cols<NQ, PC>(L.K, 16 * rb, lane), vs, (f32x4){}));
+            for (int rb = 0; rb < 8; ++rb) {
+                if (packed && rb % 2 == 0) __builtin_amdgcn_sched_barrier(0);
+                S[rb] = fma_tile(S[rb], el, mul_planes(op_cols<NQ, C>(L.K, 16 * rb, lane), vs, (f32x4){}));
+            }
         }
     }
 
@@ -333,10 +356,23 @@ __device__ __forceinline__ void rows_block(const GdnDev& p, int& h, int& c0) {
     c0 = ROWS_COLS * cs;
 }
 
-template <typename TIn>
+// A wave's partial products (W S and q S, both token tiles) lie lane-major in a
+// buffer or, packed, over the wave's own columns of W's first two planes, which
+// no other wave reads.
+template <typename TIn, bool PACKED>
 struct ScanRowsLds {
     FwdTiles<TIn> T;
-    f32x4 P[4][2][2][64];   // per wave: its partial W S and q S, both token tiles, lane-major
+    f32x4 P[4][4][64];
+    __device__ __forceinline__ f32x4& part(int w, int n, int lane) { return P[w][n][lane]; }
+};
+typedef f32x4 __attribute__((may_alias)) f32x4_alias;
+template <typename TIn>
+struct ScanRowsLds<TIn, true> {
+    FwdTiles<TIn, PRS, PCS> T;
+    __device__ __forceinline__ f32x4_alias& part(int w, int n, int lane) {
+        const int row = 16 * (n & 1) + (lane & 15);
+        return *(f32x4_alias*)(T.W + (n >> 1) * GC * GD + tile_at<PRS>(row, 32 * w + 8 * (lane >> 4)));
+    }
 };
 
 // As gdn_scan_cols_kernel, in the row layout: wave w holds the 32 x 16 slice
@@ -346,7 +382,9 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
                                                       TIn* __restrict__ out, float* __restrict__ states,
                                                       float* __restrict__ chunk_sin, float* __restrict__ chunk_vp) {
     constexpr int NQ = kInPlanes<TIn>;
-    __shared__ __attribute__((aligned(16))) ScanRowsLds<TIn> L;
+    constexpr bool packed = kScanPacked<TIn, TRUNC>;
+    constexpr int P = packed ? PRS : PR, C = packed ? PCS : PC;
+    __shared__ __attribute__((aligned(16))) ScanRowsLds<TIn, packed> L;
     ScanNode nd;
     if (!nd.init(p, lvl_begin)) return;
     int h, cb;
@@ -384,22 +422,23 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
         const Op<3> sp = op_acc(S[0], S[1]);
         lds_barrier();
 
-        // this wave's rows of W S and q S
+        // this wave's rows of W S and q S (all of W's reads before the partials)
+        f32x4 part[4];
 #pragma unroll
         for (int tb = 0; tb < 2; ++tb) {
-            L.P[wave][0][tb][lane] =
-                mul_planes(op_rows<3, PR>(L.T.W, 16 * tb + c16, 32 * wave, g4), TRUNC ? s0p : sp, (f32x4){});
-            L.P[wave][1][tb][lane] =
-                mul_planes(op_rows<NQ, PR>(L.T.Q, 16 * tb + c16, 32 * wave, g4), sp, (f32x4){});
+            part[tb] = mul_planes(op_rows<3, P>(L.T.W, 16 * tb + c16, 32 * wave, g4), TRUNC ? s0p : sp, (f32x4){});
+            part[2 + tb] = mul_planes(op_rows<NQ, P>(L.T.Q, 16 * tb + c16, 32 * wave, g4), sp, (f32x4){});
         }
+#pragma unroll
+        for (int n = 0; n < 4; ++n) L.part(wave, n, lane) = part[n];
         lds_barrier();
         // V' = U - W S and q S, the partials summed in wave order
 #pragma unroll
         for (int tb = 0; tb < 2; ++tb) {
 #pragma unroll
             for (int w = 0; w < 4; ++w) {
-                vp[tb] -= L.P[w][0][tb][lane];
-                qs[tb] += L.P[w][1][tb][lane];
+                vp[tb] -= L.part(w, tb, lane);
+                qs[tb] += L.part(w, 2 + tb, lane);
             }
         }
         if (chunk_vp && wave == 0) {
@@ -411,7 +450,7 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
         const float el = L.T.el;
 #pragma unroll
         for (int r = 0; r < 2; ++r)
-            S[r] = fma_tile(S[r], el, mul_planes(op_cols<NQ, PC>(L.T.K, 16 * (rb0 + r), lane), vs, (f32x4){}));
+            S[r] = fma_tile(S[r], el, mul_planes(op_cols<NQ, C>(L.T.K, 16 * (rb0 + r), lane), vs, (f32x4){}));
         // O = fq (q S) + A V': waves 0 and 1 take one token tile each
         if (out && wave < 2) {
             const int tb = wave;
