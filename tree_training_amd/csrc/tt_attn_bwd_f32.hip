@@ -496,7 +496,7 @@ int tt_bwd_f32_launch(const AttnDev& a, const BwdDev& b, hipStream_t s) {
         if (hipGetLastError() != hipSuccess) return TT_E_HIP;
     }
     if (b.parts & TT_BWD_DKDV) {
-        // one workgroup per CU (the kernel holds a SIMD's whole register file and 100 KB of LDS)
+        // one workgroup per CU (the kernel holds a SIMD's whole register file and 130 KB of LDS)
         const int grid = (1024 / a.hkv) * a.hkv > 0 ? (1024 / a.hkv) * a.hkv : a.hkv;
         if (b.det) {
             hipLaunchKernelGGL(bwd_dkdv_f32_kernel, dim3(grid), dim3(256), 0, s, a, b);

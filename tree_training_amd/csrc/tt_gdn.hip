@@ -300,7 +300,7 @@ __global__ __launch_bounds__(GT) void gdn_prep_kernel(GdnDev p, float* __restric
 // The backward recomputes the forward (prep + level scans, keeping each
 // chunk's initial state S and V'), then:
 //  * gdn_rscan_cols_kernel — reverse level scan (deepest level first) of dS, the
-//    gradient of the state after a chunk, per (node, v head), on fp32 MFMA:
+//    gradient of the state after a chunk, per (node, v head):
 //      dV' = A^T dO + (e^{G_L - G} k^) dS,
 //      dS <- e^{G_L} dS + (e^G q^)^T dO - W^T dV'.
 //    A node's last chunk starts from the incoming gradient of its final
@@ -341,9 +341,7 @@ __global__ __launch_bounds__(GT) void gdn_init_grad_kernel(GdnDev p, const float
 constexpr int SCS = 34;
 struct StateGradLds {     // gdn_dw_s0_kernel: one chunk of S0 and of dV'
     float S[GD * SCS];
-    float A1[GC * SCS];
     float A2[GC * SCS];
-    float red[GT / 64];
 };
 
 // One 32-column slice of the value dimension of both S and dS (all 128 rows)

@@ -20,7 +20,7 @@
 // rule's (88 to 104 KB) leave one. 16,318 tokens, 32 v heads, exact rule: forward
 // 1,311 us on fp32 MFMAs, 1,419 on padded tiles, 1,247 packed; forward and
 // backward 5.59 -> 5.25 ms. Trees of one or two chunks a node pay the splits once a
-// launch (47 tokens: 22.2 -> 22.8 us forward, 89 -> 86 both).
+// launch (47 tokens: 22.2 -> 22.8 us forward, 66.6 -> 64.0 backward).
 #pragma once
 
 #include "tt_gdn_planes.h"

@@ -341,7 +341,9 @@ __device__ __forceinline__ Op<3> e_op_f(const EArgs& a, const BlockPair& q, int 
 // The target's planes of F (ROW) or Y stay in registers (96); the partner's
 // rows come straight into operands. 4,096-token tree, 16 v heads, bf16:
 // rows 523 -> 405 us, columns 446 -> 283. Bound by the latency of those loads:
-// the registers leave two waves a SIMD.
+// the registers leave two waves a SIMD. fp32 problems, with three planes of k as
+// well, spill 35 and 41 registers there (the same tree, the whole fp32 step: 3.94 ->
+// 2.58 ms; 16,318 tokens, 32 v heads: 23.5 -> 16.9).
 template <typename TIn, bool ROW>
 __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn_e_kernel(GdnDev p, EArgs a) {
     constexpr int NQ = kInPlanes<TIn>;
