@@ -195,11 +195,11 @@ def test_gdn_bwd_fp32_matches_autograd_oracle(case):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
-@pytest.mark.parametrize("Hk,Hv", [(1, 2), (16, 32)], ids=["row_layout", "column_layout"])
+@pytest.mark.parametrize("Hk,Hv", [(1, 2), (8, 16), (16, 32)], ids=["row_layout", "column_layout", "column_layout_packed"])
 def test_gdn_scan_chunk_edges(Hk, Hv, dtype):
     """Nodes of 1, 31, 32, 33, 64 and 65 tokens on one level (and a root of 33),
-    in the row layout of the level scans (12 pairs) and the column layout (192
-    pairs), with operands of three planes (fp32) and as they come (bf16): outputs,
+    in the row layout of the level scans (12 pairs) and the column layout (96
+    and, with fp32's packed tiles, 192 pairs), with operands of three planes (fp32) and as they come (bf16): outputs,
     states and gradients against the float64 oracle, at each dtype's bar (the
     states are fp32 from exact inputs in both)."""
     lens, par = [33, 1, 31, 32, 33, 64, 65], [-1] + [0] * 6

@@ -134,7 +134,8 @@ struct ScanTiles {
     }
 };
 // fp32, exact rule: the forward's tiles without padding, 82 KB a workgroup instead
-// of 88 (rows: 104), so that two share a CU.
+// of 88 (rows: 104), so that two share a CU. The column layout takes them for
+// levels of more than a workgroup a CU (launch_scan).
 template <typename TIn, bool TRUNC>
 constexpr bool kScanPacked = kInPlanes<TIn> == 3 && !TRUNC;
 template <typename TIn, int P = PR, int C = PC>
@@ -225,12 +226,11 @@ struct ScanNode {
 // and [n_chunks, Hv, 32, 128] floats).
 // TRUNC (the reference's per-node correction): V' = U - W S0 with S0 the
 // node's initial state, whose planes stay in registers, for every chunk.
-template <typename TIn, bool TRUNC>
+template <typename TIn, bool TRUNC, bool packed>
 __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn_scan_cols_kernel(GdnDev p, int lvl_begin, float* __restrict__ ws,
                                                       TIn* __restrict__ out, float* __restrict__ states,
                                                       float* __restrict__ chunk_sin, float* __restrict__ chunk_vp) {
     constexpr int NQ = kInPlanes<TIn>;
-    constexpr bool packed = kScanPacked<TIn, TRUNC>;
     constexpr int P = packed ? PRS : PR, C = packed ? PCS : PC;
     __shared__ __attribute__((aligned(16))) FwdTiles<TIn, P, C> L;
     ScanNode nd;
