@@ -221,6 +221,30 @@ def test_gdn_scan_chunk_edges(Hk, Hv, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("truncated", [False, True], ids=["exact", "truncated"])
+def test_gdn_scan_layouts_same_bits(truncated, dtype):
+    """A tree alone (row layout: 16 and 48 pairs), twice in a forest (column
+    layout of 192 workgroups: padded tiles) and four times (384: packed ones in
+    fp32): outputs, states and gradients of every copy have the same bits."""
+    lens, par, Hk, Hv = [33, 64, 1, 70], [-1, 0, 0, 0], 8, 16
+    T, dev = sum(lens), torch.device("cuda", 0)
+    ins = [torch.from_numpy(x).to(dev) for x in _inputs(T, Hk, Hv, 6, realistic_gates=True)]
+    ins[:3] = [x.to(dtype) for x in ins[:3]]
+    d_o = torch.from_numpy(np.random.default_rng(4).standard_normal((T, Hv, D)).astype(np.float32)).to(dev, dtype)
+    ref = None
+    for copies in (1, 2, 4):
+        tree = GdnTree(lens * copies, [p if p < 0 else p + 4 * c for c in range(copies) for p in par], dev)
+        print(f"gdn scan layouts truncated={truncated} {dtype} copies={copies}", flush=True)
+        x = [t.repeat(copies, *[1] * (t.dim() - 1)) for t in ins]
+        res = [*gdn_tree_forward(*x, tree, reference_truncated=truncated),
+               *gdn_tree_backward(*x, d_o.repeat(copies, 1, 1), tree, reference_truncated=truncated)]
+        torch.cuda.synchronize()
+        ref = ref or res
+        for name, a, b in zip(("o", "states", *BWD_NAMES), ref, res):
+            assert torch.equal(a.repeat(copies, *[1] * (a.dim() - 1)), b), (name, copies)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("truncated", [False, True], ids=["exact", "truncated"])
 @pytest.mark.parametrize("value", [float("inf"), float("nan")], ids=str)
 def test_gdn_non_finite_inputs(value, truncated, dtype):
     """A non-finite value of one v head in one root of a forest: that head's
